@@ -134,25 +134,21 @@ hipError_t launch_reduce_segments(const float2* psi, int64_t plane, const int32_
                                   const int32_t* tile_off, const int32_t* seg_kind, int n_tiles,
                                   int batch, double* seg_out, hipStream_t s);
 // (small: the groups of at most 64 segments, one lane each; large: the rest,
-// one wavefront each; combine_split forms both lists from seg_of_group)
+// one wavefront each; combine_split forms both lists from seg_of_group);
+// adf (may be null) gets group 0 of every position
 hipError_t launch_combine_segments(const double* seg_in, int n_seg_stride,
                                    const int32_t* seg_of_group, const int32_t* small, int n_small,
                                    const int32_t* large, int n_large, int groups, int batch,
-                                   double* out, hipStream_t s);
+                                   double* out, double* adf, hipStream_t s);
 void combine_split(const std::vector<int32_t>& seg_of_group, std::vector<int32_t>& small,
                    std::vector<int32_t>& large);
-// ADF column of the partial sums -> adf[pos0 + b]
-hipError_t launch_collect_adf(const double* partial, int groups, int batch, double* adf,
-                              hipStream_t s);
-// FEM Welford update over the batch in raster order; state[3*nbins] = (n, mean, M2)
-hipError_t launch_fem_welford(const double* partial, int groups, int batch, int nbins,
-                              const int32_t* counts, const uint8_t* zeroed, double* state,
-                              hipStream_t s);
-hipError_t launch_fem_finalize(const double* state, int nbins, double* v, hipStream_t s);
-// Vbar_r accumulation over a batch (per-position ring ratios, raster order)
-hipError_t launch_fem_vbar(const double* partial, int groups, int batch, int nbins, int off_abs,
-                           int off_sqr, const int32_t* counts, const uint8_t* zeroed,
-                           double* vsum, hipStream_t s);
+// FEM statistics of a batch in raster order, from the ring sums at off_abs
+// (|psi|) and off_sqr (|psi|^2): d1, the Welford state[3*nbins] = (n, mean,
+// M2) and V_omega of the positions so far in v; d2, the Vbar_r sums in vsum
+hipError_t launch_fem_stats(const double* partial, int groups, int batch, int nbins, bool d1,
+                            bool d2, int off_abs, int off_sqr, const int32_t* counts,
+                            const uint8_t* zeroed, double* state, double* v, double* vsum,
+                            hipStream_t s);
 // FP64 sums over pixel groups of count full-grid FP64 waves: out[count][groups]
 hipError_t launch_group_sums_f64(const double2* psi, int64_t plane, const int32_t* offsets,
                                  const int32_t* pixels, const int32_t* kind, int groups,

@@ -447,39 +447,56 @@ hipError_t launch_reduce_segments(const float2* psi, int64_t plane, const int32_
 // adds them in segment order.  Larger groups (the ADF annulus at 1024^2:
 // ~5,500 segments): one wavefront, lane l adding segments l, l + 64, ... in
 // order, the lanes' sums meeting in a fixed butterfly.
+// One launch forms both kinds (blocks below small_blocks: the small groups,
+// the rest: one wavefront per large group) and writes group 0, the ADF ring,
+// to adf as well, where there were three launches of ~4.5 us each.
 constexpr int kWaveGroup = 64;
 
-__global__ void combine_small_kernel(const double* seg_in, int n_seg_stride,
-                                     const int32_t* seg_of_group, const int32_t* ids, int n_ids,
-                                     int groups, int batch, double* out)
-{
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (int64_t)n_ids * batch) return;
-    const int g = ids[(int)(idx % n_ids)];
-    const int b = (int)(idx / n_ids);
-    const double* in = seg_in + (int64_t)b * n_seg_stride;
-    double acc = 0.0;
-    for (int k = seg_of_group[g]; k < seg_of_group[g + 1]; ++k) acc += in[k];
-    out[(int64_t)b * groups + g] = acc;
-}
+constexpr int kCombinePos = 4; // positions per lane of a small group: its index loads serve them all
 
-__global__ void __launch_bounds__(256) combine_large_kernel(const double* seg_in, int n_seg_stride,
-                                                            const int32_t* seg_of_group,
-                                                            const int32_t* ids, int n_ids,
-                                                            int groups, int batch, double* out)
+__global__ void __launch_bounds__(256) combine_segments_kernel(
+    const double* seg_in, int n_seg_stride, const int32_t* seg_of_group, const int32_t* small,
+    int n_small, int small_blocks, const int32_t* large, int n_large, int groups, int batch,
+    double* out, double* adf)
 {
-    const int64_t pair = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (pair >= (int64_t)n_ids * batch) return; // whole wavefronts
-    const int lane = threadIdx.x & 63;
-    const int g = ids[(int)(pair % n_ids)];
-    const int b = (int)(pair / n_ids);
-    const double* in = seg_in + (int64_t)b * n_seg_stride;
-    const int s1 = seg_of_group[g + 1];
-    double acc = 0.0;
-    for (int k = seg_of_group[g] + lane; k < s1; k += 64) acc += in[k];
+    if ((int)blockIdx.x < small_blocks) {
+        const int id = (int)blockIdx.x * 256 + (int)threadIdx.x;
+        if (id >= n_small) return;
+        const int g = small[id];
+        const int s0 = seg_of_group[g], s1 = seg_of_group[g + 1];
+        const int b0 = (int)blockIdx.y * kCombinePos;
+        const double* in[kCombinePos]; // positions past the batch repeat its last and store nothing
+        double acc[kCombinePos] = {};
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off);
-    if (lane == 0) out[(int64_t)b * groups + g] = acc;
+        for (int j = 0; j < kCombinePos; ++j)
+            in[j] = seg_in + (int64_t)min(b0 + j, batch - 1) * n_seg_stride;
+        for (int k = s0; k < s1; ++k)
+#pragma unroll
+            for (int j = 0; j < kCombinePos; ++j) acc[j] += in[j][k];
+#pragma unroll
+        for (int j = 0; j < kCombinePos; ++j)
+            if (b0 + j < batch) {
+                out[(int64_t)(b0 + j) * groups + g] = acc[j];
+                if (adf && g == 0) adf[b0 + j] = acc[j];
+            }
+        return;
+    }
+    const int id = ((int)blockIdx.x - small_blocks) * 4 + (int)(threadIdx.x >> 6);
+    if (id >= n_large) return; // whole wavefronts
+    const int lane = threadIdx.x & 63;
+    const int g = large[id];
+    const int s1 = seg_of_group[g + 1];
+    for (int b = (int)blockIdx.y * kCombinePos; b < min(batch, ((int)blockIdx.y + 1) * kCombinePos); ++b) {
+        const double* in = seg_in + (int64_t)b * n_seg_stride;
+        double acc = 0.0;
+        for (int k = seg_of_group[g] + lane; k < s1; k += 64) acc += in[k];
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off);
+        if (lane == 0) {
+            out[(int64_t)b * groups + g] = acc;
+            if (adf && g == 0) adf[b] = acc;
+        }
+    }
 }
 
 void combine_split(const std::vector<int32_t>& seg_of_group, std::vector<int32_t>& small,
@@ -494,114 +511,119 @@ void combine_split(const std::vector<int32_t>& seg_of_group, std::vector<int32_t
 hipError_t launch_combine_segments(const double* seg_in, int n_seg_stride,
                                    const int32_t* seg_of_group, const int32_t* small, int n_small,
                                    const int32_t* large, int n_large, int groups, int batch,
-                                   double* out, hipStream_t s)
+                                   double* out, double* adf, hipStream_t s)
 {
-    if (batch <= 0) return hipSuccess;
-    const int64_t ns = (int64_t)n_small * batch, nl = (int64_t)n_large * batch;
-    if (ns > 0)
-        hipLaunchKernelGGL(combine_small_kernel, dim3((unsigned)((ns + 255) / 256)), dim3(256), 0,
-                           s, seg_in, n_seg_stride, seg_of_group, small, n_small, groups, batch,
-                           out);
-    if (nl > 0)
-        hipLaunchKernelGGL(combine_large_kernel, dim3((unsigned)((nl + 3) / 4)), dim3(256), 0, s,
-                           seg_in, n_seg_stride, seg_of_group, large, n_large, groups, batch, out);
+    if (batch <= 0 || n_small + n_large <= 0) return hipSuccess;
+    const int sb = (n_small + 255) / 256, lb = (n_large + 3) / 4;
+    hipLaunchKernelGGL(combine_segments_kernel, dim3((unsigned)(sb + lb), (unsigned)((batch + kCombinePos - 1) / kCombinePos)),
+                       dim3(256), 0, s, seg_in, n_seg_stride, seg_of_group, small, n_small, sb,
+                       large, n_large, groups, batch, out, adf);
     return hipGetLastError();
 }
 
-__global__ void collect_adf_kernel(const double* partial, int groups, int batch, double* adf)
-{
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < batch) adf[b] = partial[(int64_t)b * groups];
-}
+// Per-bin FEM statistics over a batch in raster order.
+//   which 0 (d1): r = radial sum / count (adfstem.cpp:2591-2599), direct-beam
+//     bins zeroed first (:2518-2522), Welford (n, mean, M2) in state, and
+//     V = Npos sum r^2 / (sum r)^2 - 1 = M2 / (n mean^2), 0 when sum r == 0
+//     (:2837-2856), of the positions so far in v;
+//   which 1 (d2, Vbar_r, :2688-2750): the sum over positions of
+//     ((r2 / c) / ((r1 r1) / (c c))) - 1, r1 and r2 the ring sums of |psi| and
+//     |psi|^2 (zero on the direct beam), c*c an integer product.
+// Bound by latency: a bin's positions are a serial chain.  A workgroup takes
+// 64 bins; its four wavefronts read and divide kStatChunk positions at a time
+// into LDS (all loads of a chunk in flight, the next chunk's issued before
+// this one's chain), the first wavefront runs the chain, whose steps are two
+// dependent FP64 operations (1/n formed beside the loads, so mean += d / n is
+// one fma).  One lane per bin that loaded, divided and chained one position
+// after another took 34 us for 853 bins x 64 positions and 76 us for
+// 42 x 256, and d2 and the final V a launch each; this form 12 and 15 us.
+constexpr int kStatBins = 64, kStatChunk = 32;
 
-hipError_t launch_collect_adf(const double* partial, int groups, int batch, double* adf,
-                              hipStream_t s)
+__global__ void __launch_bounds__(256) fem_stats_kernel(
+    const double* partial, int groups, int batch, int nbins, int which0, int off_abs, int off_sqr,
+    const int32_t* counts, const uint8_t* zeroed, double* state, double* v, double* vsum)
 {
-    hipLaunchKernelGGL(collect_adf_kernel, dim3((batch + 255) / 256), dim3(256), 0, s, partial,
-                       groups, batch, adf);
-    return hipGetLastError();
-}
-
-// r = radial sum / count (adfstem.cpp:2591-2599), direct-beam bins zeroed
-// first (:2518-2522); Welford over positions in raster order.
-__global__ void fem_welford_kernel(const double* partial, int groups, int batch, int nbins,
-                                   const int32_t* counts, const uint8_t* zeroed, double* state)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= nbins) return;
-    double n = state[3 * k], mean = state[3 * k + 1], m2 = state[3 * k + 2];
-    const double c = (double)counts[k];
-    const bool z = zeroed[k] != 0;
-    for (int b = 0; b < batch; ++b) {
-        const double r = z ? 0.0 : partial[(int64_t)b * groups + 1 + k];
-        const double x = r / c;
-        n += 1.0;
-        const double d = x - mean;
-        mean += d / n;
-        m2 += d * (x - mean);
+    constexpr int PW = kStatChunk / 4; // positions per wavefront and chunk
+    __shared__ double s_x[2][kStatChunk][kStatBins];
+    __shared__ double s_inv[2][kStatChunk];
+    const bool d1 = which0 + (int)blockIdx.y == 0;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int k = blockIdx.x * kStatBins + lane;
+    const int kc = min(k, nbins - 1); // lanes past the last bin repeat it and store nothing
+    const int c = counts[kc];
+    const double cd = (double)c, cc = (double)(c * c);
+    const bool z = zeroed[kc] != 0;
+    // positions before this batch: equal in every bin (own bin: another workgroup's may be updated already)
+    const double n0 = d1 ? state[3 * kc] : 0.0;
+    double r1[PW], r2[PW];
+    auto load = [&](int b0) {
+#pragma unroll
+        for (int j = 0; j < PW; ++j) {
+            const double* p = partial + (int64_t)min(b0 + wv * PW + j, batch - 1) * groups + kc;
+            r1[j] = p[off_abs];
+            r2[j] = d1 ? 0.0 : p[off_sqr];
+        }
+    };
+    auto put = [&](int b0, int buf) {
+#pragma unroll
+        for (int j = 0; j < PW; ++j) {
+            const double a = z ? 0.0 : r1[j], q = z ? 0.0 : r2[j];
+            s_x[buf][wv * PW + j][lane] = d1 ? a / cd : ((q / cd) / ((a * a) / cc)) - 1.0;
+        }
+        if (threadIdx.x < kStatChunk) s_inv[buf][threadIdx.x] = 1.0 / (n0 + b0 + (threadIdx.x + 1.0));
+    };
+    double mean = 0.0, m2 = 0.0, acc = 0.0;
+    if (wv == 0) {
+        if (d1) {
+            mean = state[3 * kc + 1];
+            m2 = state[3 * kc + 2];
+        } else {
+            acc = vsum[kc];
+        }
     }
-    state[3 * k] = n;
-    state[3 * k + 1] = mean;
-    state[3 * k + 2] = m2;
-}
-
-hipError_t launch_fem_welford(const double* partial, int groups, int batch, int nbins,
-                              const int32_t* counts, const uint8_t* zeroed, double* state,
-                              hipStream_t s)
-{
-    if (nbins <= 0) return hipSuccess;
-    hipLaunchKernelGGL(fem_welford_kernel, dim3((nbins + 255) / 256), dim3(256), 0, s, partial,
-                       groups, batch, nbins, counts, zeroed, state);
-    return hipGetLastError();
-}
-
-// V = Npos sum r^2 / (sum r)^2 - 1 = M2 / (n mean^2); 0 when sum r == 0
-// (adfstem.cpp:2837-2856)
-__global__ void fem_finalize_kernel(const double* state, int nbins, double* v)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= nbins) return;
-    const double n = state[3 * k], mean = state[3 * k + 1], m2 = state[3 * k + 2];
-    v[k] = (mean == 0.0) ? 0.0 : m2 / (n * mean * mean);
-}
-
-hipError_t launch_fem_finalize(const double* state, int nbins, double* v, hipStream_t s)
-{
-    if (nbins <= 0) return hipSuccess;
-    hipLaunchKernelGGL(fem_finalize_kernel, dim3((nbins + 255) / 256), dim3(256), 0, s, state,
-                       nbins, v);
-    return hipGetLastError();
-}
-
-// Vbar_r (adfstem.cpp:2688-2750): per position and bin
-//   ((r2 / c) / ((r1 r1) / (c c))) - 1
-// with r1, r2 the ring sums of |psi| and |psi|^2 (zero on the direct beam)
-// and c*c an integer product, summed over positions in raster order.
-__global__ void fem_vbar_kernel(const double* partial, int groups, int batch, int nbins,
-                                int off_abs, int off_sqr, const int32_t* counts,
-                                const uint8_t* zeroed, double* vsum)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= nbins) return;
-    const int c = counts[k];
-    const double cc = (double)(c * c);
-    const bool z = zeroed[k] != 0;
-    double acc = vsum[k];
-    for (int b = 0; b < batch; ++b) {
-        const double r1 = z ? 0.0 : partial[(int64_t)b * groups + off_abs + k];
-        const double r2 = z ? 0.0 : partial[(int64_t)b * groups + off_sqr + k];
-        acc += ((r2 / (double)c) / ((r1 * r1) / cc)) - 1.0;
+    load(0);
+    put(0, 0);
+    __syncthreads();
+    for (int b0 = 0, buf = 0; b0 < batch; b0 += kStatChunk, buf ^= 1) {
+        const bool more = b0 + kStatChunk < batch;
+        if (more) load(b0 + kStatChunk);
+        if (wv == 0) {
+            const int n = min(kStatChunk, batch - b0);
+            if (d1) {
+                for (int j = 0; j < n; ++j) {
+                    const double x = s_x[buf][j][lane], d = x - mean;
+                    mean = fma(d, s_inv[buf][j], mean);
+                    m2 = fma(d, x - mean, m2);
+                }
+            } else {
+                for (int j = 0; j < n; ++j) acc += s_x[buf][j][lane];
+            }
+        }
+        if (more) put(b0 + kStatChunk, buf ^ 1);
+        __syncthreads();
     }
-    vsum[k] = acc;
+    if (wv != 0 || k >= nbins) return;
+    if (d1) {
+        const double n = n0 + batch;
+        state[3 * k] = n;
+        state[3 * k + 1] = mean;
+        state[3 * k + 2] = m2;
+        v[k] = (mean == 0.0) ? 0.0 : m2 / (n * mean * mean);
+    } else {
+        vsum[k] = acc;
+    }
 }
 
-hipError_t launch_fem_vbar(const double* partial, int groups, int batch, int nbins, int off_abs,
-                           int off_sqr, const int32_t* counts, const uint8_t* zeroed,
-                           double* vsum, hipStream_t s)
+hipError_t launch_fem_stats(const double* partial, int groups, int batch, int nbins, bool d1,
+                            bool d2, int off_abs, int off_sqr, const int32_t* counts,
+                            const uint8_t* zeroed, double* state, double* v, double* vsum,
+                            hipStream_t s)
 {
-    if (nbins <= 0 || batch <= 0) return hipSuccess;
-    hipLaunchKernelGGL(fem_vbar_kernel, dim3((nbins + 255) / 256), dim3(256), 0, s, partial,
-                       groups, batch, nbins, off_abs, off_sqr, counts, zeroed, vsum);
+    if (nbins <= 0 || batch <= 0 || !(d1 || d2)) return hipSuccess;
+    hipLaunchKernelGGL(fem_stats_kernel,
+                       dim3((unsigned)((nbins + kStatBins - 1) / kStatBins), d1 && d2 ? 2u : 1u),
+                       dim3(256), 0, s, partial, groups, batch, nbins, d1 ? 0 : 1, off_abs, off_sqr,
+                       counts, zeroed, state, v, vsum);
     return hipGetLastError();
 }
 
@@ -609,11 +631,12 @@ hipError_t launch_fem_vbar(const double* partial, int groups, int batch, int nbi
 // jj, c = count_ii * I_ii,jj / r_ii - 1 when that ratio is >= 1 and count,
 // I and r are all non-zero, else 0; I and r are the sector and ring sums of
 // |psi| (zero on direct-beam rings).  Sums of c and c^2 over positions in
-// raster order, stored [ii + jj * nbins].
-__global__ void fem_correlograph_kernel(const double* partial, int groups, int batch, int nbins,
-                                        int nphi, int off_abs, int off_corr,
-                                        const int32_t* counts, const uint8_t* zeroed,
-                                        double* csum, double* csqr, double* each)
+// raster order, stored [ii + jj * nbins].  The sums of 8 positions are read
+// ahead of their products: one at a time the pass waited for each position's
+// loads (61 -> 41 us for 853 rings x 159 sectors x 64 positions, 69 MB).
+__global__ void __launch_bounds__(256) fem_correlograph_kernel(
+    const double* partial, int groups, int batch, int nbins, int nphi, int off_abs, int off_corr,
+    const int32_t* counts, const uint8_t* zeroed, double* csum, double* csqr, double* each)
 {
     const int k = blockIdx.x * blockDim.x + threadIdx.x; // ii * nphi + jj
     if (k >= nbins * nphi) return;
@@ -622,16 +645,29 @@ __global__ void fem_correlograph_kernel(const double* partial, int groups, int b
     const int c = counts[ii];
     const bool z = zeroed[ii] != 0;
     double a = csum[o], q = csqr[o];
-    for (int b = 0; b < batch; ++b) {
-        const double r = z ? 0.0 : partial[(int64_t)b * groups + off_abs + ii];
-        const double I = z ? 0.0 : partial[(int64_t)b * groups + off_corr + k];
+    auto add = [&](int b, double r, double I) {
+        if (z) r = I = 0.0;
         const double t = (c * I / r);
         double v = 0.0;
         if ((t >= 1) && (c != 0) && (I != 0) && (r != 0)) v = t - 1;
         a += v;
         q += v * v;
         if (each) each[(int64_t)b * nbins * nphi + o] = v; // per position (optional)
+    };
+    constexpr int C = 8;
+    const double* w = partial;
+    int b = 0;
+    for (; b + C <= batch; b += C, w += (int64_t)C * groups) {
+        double r[C], I[C];
+#pragma unroll
+        for (int j = 0; j < C; ++j) {
+            r[j] = w[(int64_t)j * groups + off_abs + ii];
+            I[j] = w[(int64_t)j * groups + off_corr + k];
+        }
+#pragma unroll
+        for (int j = 0; j < C; ++j) add(b + j, r[j], I[j]);
     }
+    for (; b < batch; ++b, w += groups) add(b, w[off_abs + ii], w[off_corr + k]);
     csum[o] = a;
     csqr[o] = q;
 }
@@ -790,20 +826,32 @@ hipError_t launch_div_f64(double2* a, int64_t n, double d, hipStream_t s)
 }
 
 // Per-pixel sums over positions of |psi| and |psi|^2 in raster order, FP64
-// (adfstem.cpp:2753-2781), on the compact plane of the exit waves.
-__global__ void pixel_moments_kernel(const float2* psi, int64_t plane, int batch, double* s1,
-                                     double* s2)
+// (adfstem.cpp:2753-2781), on the compact plane of the exit waves.  8
+// positions' waves are read ahead of their sums (56 -> 32 us for 512 x 352
+// pixels x 64 positions, 92 MB).
+__global__ void __launch_bounds__(256) pixel_moments_kernel(const float2* psi, int64_t plane,
+                                                            int batch, double* s1, double* s2)
 {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= plane) return;
     double a = s1[p], q = s2[p];
-    for (int b = 0; b < batch; ++b) {
-        const float2 v = psi[(int64_t)b * plane + p];
+    auto add = [&](float2 v) {
         const double re = v.x, im = v.y;
         const double m2 = re * re + im * im;
         a += sqrt(m2);
         q += m2;
+    };
+    constexpr int C = 8;
+    const float2* w = psi + p;
+    int b = 0;
+    for (; b + C <= batch; b += C, w += C * plane) {
+        float2 v[C];
+#pragma unroll
+        for (int j = 0; j < C; ++j) v[j] = w[j * plane];
+#pragma unroll
+        for (int j = 0; j < C; ++j) add(v[j]);
     }
+    for (; b < batch; ++b, w += plane) add(*w);
     s1[p] = a;
     s2[p] = q;
 }

@@ -680,9 +680,9 @@ int msf_fem_accumulate(msf_ctx* c, const msf_grid* grid, const msf_fem* fem, dou
             HIPCHK(c, st.alloc((size_t)nb * 3 * sizeof(double)));
             HIPCHK(c, v.alloc((size_t)nb * sizeof(double)));
             HIPCHK(c, hipMemsetAsync(st.p, 0, (size_t)nb * 3 * sizeof(double), c->stream));
-            HIPCHK(c, msf::launch_fem_welford(dp.as<double>(), G, (int)count, nb, dc.as<int32_t>(),
-                                              dz.as<uint8_t>(), st.as<double>(), c->stream));
-            HIPCHK(c, msf::launch_fem_finalize(st.as<double>(), nb, v.as<double>(), c->stream));
+            HIPCHK(c, msf::launch_fem_stats(dp.as<double>(), G, (int)count, nb, true, false,
+                                            g.fem_abs, 0, dc.as<int32_t>(), dz.as<uint8_t>(),
+                                            st.as<double>(), v.as<double>(), nullptr, c->stream));
             HIPCHK(c, hipMemcpyAsync(v_omega, v.p, (size_t)nb * sizeof(double), hipMemcpyDeviceToHost,
                                      c->stream));
             HIPCHK(c, hipStreamSynchronize(c->stream));

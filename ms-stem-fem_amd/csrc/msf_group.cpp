@@ -214,14 +214,6 @@ int run_group(msf_ctx* c, std::vector<GroupRun>& runs, GroupInfo* info)
             if (a.k + 1 < s.sh.n_batches) start(a.r, a.k + 1);
         }
     }
-    for (int r = 0; r < R && rc == MSF_OK; ++r) {
-        const GroupState& s = gs[(size_t)r];
-        if (s.ok && s.f.want_d1)
-            rc = msf::launch_fem_finalize(s.v.state, c->gplans[(size_t)r]->nbins, s.v.femv, st) ==
-                         hipSuccess
-                     ? MSF_OK
-                     : fail(c, MSF_ERR_DEVICE, "fem_finalize launch failed");
-    }
     for (hipStream_t q : {su, st}) {
         const hipError_t e = hipStreamSynchronize(q);
         if (e != hipSuccess && rc == MSF_OK) {

@@ -777,17 +777,21 @@ int enqueue_batch_tail(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, co
     float2* bpsi = v.psi[ch];
     double* bpart = v.part[ch];
     double* bsegp = v.segp[ch];
-    auto combine = [&](const double* sg, int n, double* out, hipStream_t st) {
-        return msf::launch_combine_segments(sg, pl.n_tiles * 64, pl.seg_of_group, pl.grp_small,
-                                            (int)pl.small_ids.size(), pl.grp_large,
-                                            (int)pl.large_ids.size(), G, n, out, st);
+    auto sums = [&](double* adf) {
+        const hipError_t e = msf::launch_reduce_segments(bpsi, plane, pl.seg_pix, pl.tile_off,
+                                                         pl.seg_kind, pl.n_tiles, nb, bsegp, s);
+        return e != hipSuccess
+                   ? e
+                   : msf::launch_combine_segments(bsegp, pl.n_tiles * 64, pl.seg_of_group,
+                                                  pl.grp_small, (int)pl.small_ids.size(),
+                                                  pl.grp_large, (int)pl.large_ids.size(), G, nb,
+                                                  bpart, adf, s);
     };
-    HIPCHK(c, prof.begin(K_RED));
-    HIPCHK(c, msf::launch_reduce_segments(bpsi, plane, pl.seg_pix, pl.tile_off, pl.seg_kind,
-                                          pl.n_tiles, nb, bsegp, s));
-    HIPCHK(c, combine(bsegp, nb, bpart, s));
-    HIPCHK(c, prof.end());
-    if (f.want_adf) HIPCHK(c, msf::launch_collect_adf(bpart, G, nb, v.adf + b0, s));
+    if (f.want_adf || f.want_fem) { // exit waves alone need no sums
+        HIPCHK(c, prof.begin(K_RED));
+        HIPCHK(c, sums(f.want_adf ? v.adf + b0 : nullptr));
+        HIPCHK(c, prof.end());
+    }
     if (f.want_mtf) {
         // adfstem.cpp:2272-2385 after the ADF sum: |psi| outside the
         // aperture, BACKWARD FFT, x MTF / s (in-place update), FORWARD
@@ -799,17 +803,12 @@ int enqueue_batch_tail(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, co
         HIPCHK(c, msf::fft2d_f64(full, nx, ny, nb, false, v.twx.f64, v.twy.f64, s));
         HIPCHK(c, msf::launch_mtf_compact(full, nx, ny, ncp, ka, kb, sp->dkeep.as<int2>(),
                                           d.sqrt_nxny, nb, bpsi, s));
-        HIPCHK(c, msf::launch_reduce_segments(bpsi, plane, pl.seg_pix, pl.tile_off,
-                                              pl.seg_kind, pl.n_tiles, nb, bsegp, s));
-        HIPCHK(c, combine(bsegp, nb, bpart, s));
+        HIPCHK(c, sums(nullptr));
     }
     // the FEM accumulators are shared: batch k updates them after batch k-1
     if (chains == 2 && k > 0) HIPCHK(c, hipStreamWaitEvent(s, c->ev_fem[(k - 1) % 2], 0));
-    if (f.want_d1)
-        HIPCHK(c, msf::launch_fem_welford(bpart, G, nb, nbins, pl.cnt, pl.zero, v.state, s));
-    if (f.want_d2)
-        HIPCHK(c, msf::launch_fem_vbar(bpart, G, nb, nbins, pl.hg.fem_abs, pl.hg.fem_sqr, pl.cnt,
-                                       pl.zero, v.vsum, s));
+    HIPCHK(c, msf::launch_fem_stats(bpart, G, nb, nbins, f.want_d1, f.want_d2, pl.hg.fem_abs,
+                                    pl.hg.fem_sqr, pl.cnt, pl.zero, v.state, v.femv, v.vsum, s));
     if (f.want_corr)
         HIPCHK(c, msf::launch_fem_correlograph(
                       bpart, G, nb, nbins, nphi, pl.hg.fem_abs, pl.hg.corr, pl.cnt, pl.zero,
@@ -909,7 +908,6 @@ int enqueue_job(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, const Run
             k += 2;
             b0 = b1 + nbB;
         }
-        if (f.want_d1) HIPCHK(c, msf::launch_fem_finalize(v.state, pl.nbins, v.femv, c->stream));
         return MSF_OK;
     }
     if (chains == 2) { // fork: the second stream starts after everything issued so far
@@ -931,7 +929,6 @@ int enqueue_job(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, const Run
         HIPCHK(c, hipEventRecord(c->ev_join, c->stream2));
         HIPCHK(c, hipStreamWaitEvent(c->stream, c->ev_join, 0));
     }
-    if (f.want_d1) HIPCHK(c, msf::launch_fem_finalize(v.state, pl.nbins, v.femv, c->stream));
     return MSF_OK;
 }
 
