@@ -452,12 +452,12 @@ hipError_t launch_reduce_segments(const float2* psi, int64_t plane, const int32_
 // to adf as well, where there were three launches of ~4.5 us each.
 constexpr int kWaveGroup = 64;
 
-constexpr int kCombinePos = 4; // positions per lane of a small group: its index loads serve them all
+constexpr int kCombinePos = 4; // positions per workgroup: a small group's index loads serve them all
 
 __global__ void __launch_bounds__(256) combine_segments_kernel(
     const double* seg_in, int n_seg_stride, const int32_t* seg_of_group, const int32_t* small,
-    int n_small, int small_blocks, const int32_t* large, int n_large, int groups, int batch,
-    double* out, double* adf)
+    int n_small, int small_blocks, const int32_t* large, int groups, int batch, double* out,
+    double* adf)
 {
     if ((int)blockIdx.x < small_blocks) {
         const int id = (int)blockIdx.x * 256 + (int)threadIdx.x;
@@ -481,21 +481,21 @@ __global__ void __launch_bounds__(256) combine_segments_kernel(
             }
         return;
     }
-    const int id = ((int)blockIdx.x - small_blocks) * 4 + (int)(threadIdx.x >> 6);
-    if (id >= n_large) return; // whole wavefronts
+    // one large group per workgroup, one position per wavefront
+    const int b = (int)blockIdx.y * kCombinePos + (int)(threadIdx.x >> 6);
+    if (b >= batch) return; // whole wavefronts
     const int lane = threadIdx.x & 63;
-    const int g = large[id];
+    const int g = large[(int)blockIdx.x - small_blocks];
     const int s1 = seg_of_group[g + 1];
-    for (int b = (int)blockIdx.y * kCombinePos; b < min(batch, ((int)blockIdx.y + 1) * kCombinePos); ++b) {
-        const double* in = seg_in + (int64_t)b * n_seg_stride;
-        double acc = 0.0;
-        for (int k = seg_of_group[g] + lane; k < s1; k += 64) acc += in[k];
+    const double* in = seg_in + (int64_t)b * n_seg_stride;
+    double acc = 0.0;
+#pragma unroll 8
+    for (int k = seg_of_group[g] + lane; k < s1; k += 64) acc += in[k];
 #pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off);
-        if (lane == 0) {
-            out[(int64_t)b * groups + g] = acc;
-            if (adf && g == 0) adf[b] = acc;
-        }
+    for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off);
+    if (lane == 0) {
+        out[(int64_t)b * groups + g] = acc;
+        if (adf && g == 0) adf[b] = acc;
     }
 }
 
@@ -514,10 +514,10 @@ hipError_t launch_combine_segments(const double* seg_in, int n_seg_stride,
                                    double* out, double* adf, hipStream_t s)
 {
     if (batch <= 0 || n_small + n_large <= 0) return hipSuccess;
-    const int sb = (n_small + 255) / 256, lb = (n_large + 3) / 4;
-    hipLaunchKernelGGL(combine_segments_kernel, dim3((unsigned)(sb + lb), (unsigned)((batch + kCombinePos - 1) / kCombinePos)),
+    const int sb = (n_small + 255) / 256;
+    hipLaunchKernelGGL(combine_segments_kernel, dim3((unsigned)(sb + n_large), (unsigned)((batch + kCombinePos - 1) / kCombinePos)),
                        dim3(256), 0, s, seg_in, n_seg_stride, seg_of_group, small, n_small, sb,
-                       large, n_large, groups, batch, out, adf);
+                       large, groups, batch, out, adf);
     return hipGetLastError();
 }
 
