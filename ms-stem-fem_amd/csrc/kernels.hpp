@@ -182,16 +182,15 @@ bool setup_lengths_ok(int n);
 // stage twiddle tables)
 hipError_t fft2d_f64(double2* data, int nx, int ny, int count, bool inverse, const double2* twx,
                      const double2* twy, hipStream_t s);
+struct ProbeOptics {
+    int corrected;
+    double cs3, cs5, defocus, lambda, x0, y0;
+};
 // probe H(k) of probe_wavefunction.cpp:37-239 inside the aperture ranges
 hipError_t launch_probe_k(double2* h, const double* kx, const double* ky, int nx, int ny,
-                          const int2* aperture, int corrected, double cs3, double cs5,
-                          double defocus, double lambda, double x0, double y0,
-                          hipStream_t s);
+                          const int2* aperture, const ProbeOptics& o, hipStream_t s);
 // sum |a|^2 over n values (one workgroup, fixed order)
 hipError_t launch_norm2(const double2* a, int64_t n, double* out, hipStream_t s);
-// probe_s = (float) (a * scale)
-hipError_t launch_scale_to_f32(const double2* a, int64_t n, const double* norm2,
-                               double numerator, float2* out, hipStream_t s);
 hipError_t launch_fill_f64(double2* a, int64_t n, hipStream_t s);
 // out[0, n16) = in[0, n16), 16-byte vectors; n16 a multiple of 1024
 hipError_t launch_stream_copy(const float4* in, float4* out, int64_t n16, hipStream_t s);
@@ -218,12 +217,25 @@ hipError_t launch_vacuum_step(double2* a, int nx, int ny, const double2* px, con
 // FP64 transmission update of `count` real-space waves by one slice's t
 hipError_t launch_transmit_f64(double2* a, const double2* t, int64_t m, int count, int mode,
                                double s, hipStream_t st);
-// FP64 [nx][ny] -> FP32 [ny][nx]
-hipError_t launch_to_f32_transposed(const double2* a, int nx, int ny, float2* out, hipStream_t s);
-// out[i][2r + h] = (float2) a[i][(r + h ny/2) mod ny], r < ny, h = 0, 1: the
-// pair of elements r and r + ny/2 for every shift r of a row (u0 rows)
-hipError_t launch_to_f32_shift_pairs(const double2* a, int nx, int ny, float2* out, hipStream_t s);
-// a *= f / sqrt(*norm2)
-hipError_t launch_scale_f64(double2* a, int64_t n, const double* norm2, double f, hipStream_t s);
+// row stride of an FP64 array of nc <= ny columns: an odd number of 128-byte
+// lines where that fits in ny columns (fft64_passes.hpp)
+int col_stride64(int nc, int ny);
+// Vacuum waves entering slices [n0, n1) of S, and with n1 == S the exit wave.
+// The aperture's bounding box: rows [0, ra) U [nx - rb, nx), columns [0, ca)
+// U [ny - cb, ny).
+struct VacuumArgs {
+    double2* w;              // work: [n1 - n0][nx][ld], ld = col_stride64(ca + cb, ny)
+    float2* psi0;            // [ny][nx] k-space exit wave; pixels off the box are not written
+    const double *kx, *ky;
+    const int2 *ap, *keep;   // aperture and slice-step ranges per row
+    const double2 *px, *py;  // [S][nx], [S][ny]
+    ProbeOptics o;
+    double norm;             // of H(k): s over the norm of its inverse transform
+    int nx, ny, ld, ra, rb, ca, cb, n0, n1, S;
+};
+// u0: the waves of slices n0, n0 + 1, ... in real space as rows of FP32 shift
+// pairs [nx][ny][2] (pair r of a row holds elements r and (r + ny/2) mod ny)
+hipError_t launch_vacuum(const VacuumArgs& a, float2* u0, const double2* twx, const double2* twy,
+                         hipStream_t s);
 
 } // namespace msf

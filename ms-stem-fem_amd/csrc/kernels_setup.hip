@@ -11,8 +11,9 @@
 // bw_limit, BACKWARD FFT, / NxNy.  Everything here is FP64.
 //
 // Probe (adfstem.cpp:586-817): H(k) inside the aperture, BACKWARD FFT, norm.
-#include "fft_engine.hpp"
-#include "kernels.hpp"
+#include <algorithm>
+
+#include "fft64_passes.hpp"
 
 namespace msf {
 
@@ -124,40 +125,41 @@ hipError_t fft2d_f64(double2* data, int nx, int ny, int count, bool inverse, con
 constexpr double kPi = 3.14159265369; // the reference's PI
 
 // probe_wavefunction.cpp:37-137 / :139-239 with lenses.cpp:249-290
+__device__ __forceinline__ double2 probe_h(double kx, double ky, const ProbeOptics& o)
+{
+    const double lsq = o.lambda * o.lambda;
+    const double ksqr = kx * kx + ky * ky;
+    double chi;
+    if (o.corrected) {
+        const double kl = ksqr * lsq;
+        chi = kPi * o.lambda * ksqr * (-o.defocus + 0.5 * o.cs3 * kl + (1.0 / 3.0) * o.cs5 * (kl * kl));
+    } else {
+        chi = kPi * o.lambda * ksqr * (0.5 * o.cs3 * lsq * ksqr - o.defocus);
+    }
+    const double trig = chi + 2 * kPi * ((kx * o.x0) + (ky * o.y0));
+    double sn, cs;
+    sincos(trig, &sn, &cs);
+    return double2{cs, -1.0 * sn};
+}
+
 __global__ void probe_k_kernel(double2* h, const double* kx, const double* ky, int nx, int ny,
-                               const int2* ap, int corrected, double cs3, double cs5,
-                               double defocus, double lambda, double x0, double y0)
+                               const int2* ap, ProbeOptics o)
 {
     const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (int64_t)nx * ny) return;
     const int i = (int)(idx / ny), j = (int)(idx % ny);
     const int2 r = ap[i];
     double2 v{0.0, 0.0};
-    if (j < r.x || j >= ny - r.y) {
-        const double lsq = lambda * lambda;
-        const double ksqr = kx[i] * kx[i] + ky[j] * ky[j];
-        double chi;
-        if (corrected) {
-            const double kl = ksqr * lsq;
-            chi = kPi * lambda * ksqr * (-defocus + 0.5 * cs3 * kl + (1.0 / 3.0) * cs5 * (kl * kl));
-        } else {
-            chi = kPi * lambda * ksqr * (0.5 * cs3 * lsq * ksqr - defocus);
-        }
-        const double trig = chi + 2 * kPi * ((kx[i] * x0) + (ky[j] * y0));
-        double sn, cs;
-        sincos(trig, &sn, &cs);
-        v = double2{cs, -1.0 * sn};
-    }
+    if (j < r.x || j >= ny - r.y) v = probe_h(kx[i], ky[j], o);
     h[idx] = v;
 }
 
 hipError_t launch_probe_k(double2* h, const double* kx, const double* ky, int nx, int ny,
-                          const int2* aperture, int corrected, double cs3, double cs5,
-                          double defocus, double lambda, double x0, double y0, hipStream_t s)
+                          const int2* aperture, const ProbeOptics& o, hipStream_t s)
 {
     const int64_t n = (int64_t)nx * ny;
     hipLaunchKernelGGL(probe_k_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, h, kx,
-                       ky, nx, ny, aperture, corrected, cs3, cs5, defocus, lambda, x0, y0);
+                       ky, nx, ny, aperture, o);
     return hipGetLastError();
 }
 
@@ -179,23 +181,6 @@ __global__ void __launch_bounds__(1024) norm2_kernel(const double2* a, int64_t n
 hipError_t launch_norm2(const double2* a, int64_t n, double* out, hipStream_t s)
 {
     hipLaunchKernelGGL(norm2_kernel, dim3(1), dim3(1024), 0, s, a, n, out);
-    return hipGetLastError();
-}
-
-__global__ void scale_to_f32_kernel(const double2* a, int64_t n, const double* norm2,
-                                    double numerator, float2* out)
-{
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const double f = numerator / sqrt(*norm2);
-    out[k] = float2{(float)(a[k].x * f), (float)(a[k].y * f)};
-}
-
-hipError_t launch_scale_to_f32(const double2* a, int64_t n, const double* norm2,
-                               double numerator, float2* out, hipStream_t s)
-{
-    hipLaunchKernelGGL(scale_to_f32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a,
-                       n, norm2, numerator, out);
     return hipGetLastError();
 }
 
@@ -389,61 +374,108 @@ hipError_t launch_vacuum_step(double2* a, int nx, int ny, const double2* px, con
 }
 
 
-
-// out[j * nx + i] = a[i * ny + j]: the column-major copy a column pass reads
-// along its column
-__global__ void to_f32_transposed_kernel(const double2* a, int nx, int ny, float2* out)
+// -------------------------------------------------------- vacuum waves
+int col_stride64(int nc, int ny)
 {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= (int64_t)nx * ny) return;
-    const int64_t j = k / nx;
-    const int i = (int)(k % nx);
-    const double2 v = a[(int64_t)i * ny + j];
-    out[k] = float2{(float)v.x, (float)v.y};
+    const int pad = (nc + 7) / 8 * 8;
+    const int ld = pad % 16 == 8 ? pad : pad + 8;
+    return ld <= ny ? ld : nc;
 }
 
-hipError_t launch_to_f32_transposed(const double2* a, int nx, int ny, float2* out, hipStream_t s)
+// The vacuum wave (t = 1) entering every slice (adfstem.cpp:586-817,
+// :1986-2043): u0_0 = s * probe, w_n = M P_n FFT(u0_n) / s^2, u0_{n+1} =
+// IFFT(w_n).  FFT(IFFT(w)) = s^2 w, so w_n is H(k) times the product of the
+// slices' masks and propagators, and non-zero inside the aperture only: one
+// lane per pixel of the aperture's bounding box ([0, ra) U [nx - rb, nx) x
+// [0, ca) U [ny - cb, ny)) forms every slice's wave, columns of the box are
+// transformed for all slices at once, then the rows, whose last stage writes
+// the FP32 shift pairs.  The probe's norm is sqrt(n_ap s^2) by Parseval,
+// |H| = 1 on the n_ap aperture pixels, so no sum over the grid is needed.
+// A transform pair per slice on one plane at a time took 5 launches a slice
+// and a single-workgroup norm: 0.43 ms of set-up at 256^2 with 12 slices and
+// 2.7 ms at 1024^2 with 25, bound by launches; now 0.02 and 0.17 ms of kernels.
+__global__ void __launch_bounds__(256) vacuum_box_kernel(VacuumArgs a)
 {
-    const int64_t n = (int64_t)nx * ny;
-    hipLaunchKernelGGL(to_f32_transposed_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                       s, a, nx, ny, out);
-    return hipGetLastError();
+    const int nc = a.ca + a.cb;
+    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= (int64_t)(a.ra + a.rb) * nc) return;
+    const int ib = (int)(idx / nc), c = (int)(idx - (int64_t)ib * nc);
+    const int i = ib < a.ra ? ib : a.nx - a.rb - a.ra + ib;
+    const int j = c < a.ca ? c : a.ny - a.cb - a.ca + c;
+    const int2 r = a.ap[i];
+    double2 v{0.0, 0.0};
+    if (j < r.x || j >= a.ny - r.y) v = probe_h(a.kx[i], a.ky[j], a.o);
+    v = double2{v.x * a.norm, v.y * a.norm};
+    const int2 k = a.keep[i];
+    const bool keep = j < k.x || j >= a.ny - k.y;
+    double2* __restrict__ out = a.w + (int64_t)i * a.ld + c;
+    const int64_t plane = (int64_t)a.nx * a.ld;
+#pragma unroll 4
+    for (int n = 0; n < a.n1; ++n) {
+        if (n >= a.n0) out[(n - a.n0) * plane] = v;
+        const double2 px = a.px[(int64_t)n * a.nx + i], py = a.py[(int64_t)n * a.ny + j];
+        const double pr = px.x * py.x - px.y * py.y;
+        const double pi = px.x * py.y + px.y * py.x;
+        v = keep ? double2{pr * v.x - pi * v.y, pr * v.y + pi * v.x} : double2{0.0, 0.0};
+    }
+    if (a.n1 == a.S) a.psi0[(int64_t)j * a.nx + i] = float2{(float)v.x, (float)v.y};
 }
 
-__global__ void to_f32_shift_pairs_kernel(const double2* a, int nx, int ny, float2* out)
-{
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= (int64_t)nx * 2 * ny) return;
-    const int64_t i = k / (2 * ny);
-    const int m = (int)(k % (2 * ny));
-    // pair r = m / 2 holds a[i][r] and a[i][(r + ny/2) mod ny]
-    int j = m / 2 + (m % 2) * (ny / 2);
-    if (j >= ny) j -= ny;
-    const double2 v = a[i * ny + j];
-    out[k] = float2{(float)v.x, (float)v.y};
-}
+struct VacuumCols {
+    static constexpr int inputs = 1;
+    double2* w;
+    int nx, ld, ra, rb;
+    __device__ __forceinline__ double2 load(int plane, int, int i, int c) const
+    {
+        return (i < ra || i >= nx - rb) ? w[((int64_t)plane * nx + i) * ld + c] : double2{0.0, 0.0};
+    }
+    __device__ __forceinline__ void store(int plane, int i, int c, double2 v) const
+    {
+        w[((int64_t)plane * nx + i) * ld + c] = v;
+    }
+};
 
-hipError_t launch_to_f32_shift_pairs(const double2* a, int nx, int ny, float2* out, hipStream_t s)
-{
-    const int64_t n = (int64_t)nx * 2 * ny;
-    hipLaunchKernelGGL(to_f32_shift_pairs_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                       s, a, nx, ny, out);
-    return hipGetLastError();
-}
+// rows from the aperture's columns; out[i][2r + h] = a[i][(r + h ny/2) mod ny]:
+// a lane's elements p and p + E/2 are j and j + ny/2, one 16-byte store each
+// for the shifts r = j and r = j + ny/2
+struct VacuumRows {
+    const double2* w;
+    float2* u0;
+    int nx, ny, ld, ca, cb;
+    __device__ __forceinline__ double2 load(int plane, int i, int j) const
+    {
+        const int c = j < ca ? j : j - ny + ca + cb;
+        return (j < ca || j >= ny - cb) ? w[((int64_t)plane * nx + i) * ld + c] : double2{0.0, 0.0};
+    }
+    template <int E, int T>
+    __device__ __forceinline__ void store(int plane, int i, int t, const double2 (&x)[E]) const
+    {
+        float4* row = reinterpret_cast<float4*>(u0 + ((int64_t)plane * nx + i) * (2 * ny));
+#pragma unroll
+        for (int p = 0; p < E / 2; ++p) {
+            const double2 a = x[p], b = x[p + E / 2];
+            const float4 f{(float)a.x, (float)a.y, (float)b.x, (float)b.y};
+            row[t + T * p] = f;
+            row[t + T * p + ny / 2] = float4{f.z, f.w, f.x, f.y};
+        }
+    }
+};
 
-__global__ void scale_f64_kernel(double2* a, int64_t n, const double* norm2, double f)
+hipError_t launch_vacuum(const VacuumArgs& a, float2* u0, const double2* twx, const double2* twy,
+                         hipStream_t s)
 {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const double g = f / sqrt(*norm2);
-    a[k] = double2{a[k].x * g, a[k].y * g};
-}
-
-hipError_t launch_scale_f64(double2* a, int64_t n, const double* norm2, double f, hipStream_t s)
-{
-    hipLaunchKernelGGL(scale_f64_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, n,
-                       norm2, f);
-    return hipGetLastError();
+    const int64_t box = (int64_t)(a.ra + a.rb) * (a.ca + a.cb);
+    const int planes = a.n1 - a.n0;
+    if (box <= 0 || planes <= 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(vacuum_box_kernel, dim3((unsigned)((box + 255) / 256)), dim3(256), 0, s, a);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess)
+        e = launch_cols64<Fft64::Inverse>(a.nx, VacuumCols{a.w, a.nx, a.ld, a.ra, a.rb}, a.ca + a.cb,
+                                          planes, twx, s);
+    if (e == hipSuccess)
+        e = launch_rows64<Fft64::Inverse>(a.ny, VacuumRows{a.w, u0, a.nx, a.ny, a.ld, a.ca, a.cb},
+                                          a.nx, planes, twy, s);
+    return e;
 }
 
 // FP64 transmission update of one slice on `count` real-space waves

@@ -315,10 +315,10 @@ int msf_specimen_build(msf_ctx* c, const msf_grid* grid, const double* q, const 
         if ((rc = twiddles(c, heap, nx, tx))) return bail(rc);
         if ((rc = twiddles(c, heap, ny, ty))) return bail(rc);
         const double2 *twx = tx.f64, *twy = ty.f64;
-        DevBuf dkx, dky, dsup, dbw, dpar, dmaps, datoms;
+        DevBuf dsup, dbw, dpar, dmaps, datoms;
         hipError_t e = hipSuccess;
-        if (!e) e = upload(dkx, d.kx, c->stream);
-        if (!e) e = upload(dky, d.ky, c->stream);
+        if (!e) e = upload(sp->dkx, d.kx, c->stream);
+        if (!e) e = upload(sp->dky, d.ky, c->stream);
         if (!e) e = upload(dsup, to_int2(sup), c->stream);
         if (!e) e = upload(dbw, to_int2(bw), c->stream);
         if (!e) e = upload(dpar, params, c->stream);
@@ -353,8 +353,8 @@ int msf_specimen_build(msf_ctx* c, const msf_grid* grid, const double* q, const 
             if (!e) e = msf::launch_scatter_atoms(maps, datoms.as<int4>(), (int)chunk.size(), nx, ny,
                                                   std::max(nsp, 1), c->stream);
             if (!e && nsp > 0) e = msf::fft2d_f64(maps, nx, ny, k * nsp, false, twx, twy, c->stream);
-            if (!e) e = msf::launch_combine_species(maps, sig, k, nsp, dpar.as<double>(), dkx.as<double>(),
-                                                    dky.as<double>(), nx, ny, dsup.as<int2>(), lgab,
+            if (!e) e = msf::launch_combine_species(maps, sig, k, nsp, dpar.as<double>(),
+                                                    sp->dkx.as<double>(), sp->dky.as<double>(), nx, ny, dsup.as<int2>(), lgab,
                                                     grid->xmin, grid->ymin, c->stream);
             if (!e) e = msf::fft2d_f64(sig, nx, ny, k, true, twx, twy, c->stream);
             if (!e) e = msf::launch_exp_transmit(sig, (int64_t)k * M, 1.0 / std::sqrt((double)M), c->stream);

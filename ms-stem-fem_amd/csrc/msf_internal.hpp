@@ -79,7 +79,7 @@ struct RunPlan {
     // vacuum waves: u0 of every slice [S][nx][ny] pairs (s * real space; for
     // every shift r of a row, u0[r] and u0[(r + ny/2) mod ny]: pair_pos) and
     // the k-space vacuum exit wave, column-major [ny][nx], FP32
-    DevBuf U0, Psi0;
+    DevBuf U0, Psi0, vac_b; // vac_b: work array of their build, at most 32 MiB or one plane
     float2* u0 = nullptr;
     float2* psi0 = nullptr;
     // reduction groups (host tables and their device copies); they depend on
@@ -138,7 +138,7 @@ struct RunPlan {
         drop_graph();
         valid = false;
         spec_id = 0;
-        for (DevBuf* b : {&U0, &Psi0, &state_b, &femv_b, &adf_b, &shift_b, &exit_b, &vsum_b,
+        for (DevBuf* b : {&U0, &Psi0, &vac_b, &state_b, &femv_b, &adf_b, &shift_b, &exit_b, &vsum_b,
                           &pm1_b, &pm2_b, &csum_b, &csqr_b, &ceach_b})
             b->release();
         for (int k = 0; k < 2; ++k)
@@ -274,6 +274,7 @@ struct msf_specimen {
     msf_impl::DevBuf py;   // [S][ny] float2, P_y / sqrtNxNy
     msf_impl::DevBuf px64; // [S][nx] double2
     msf_impl::DevBuf py64; // [S][ny] double2
+    msf_impl::DevBuf dkx, dky; // [nx], [ny] spatial frequencies, FP64
     uint64_t id = 0;           // unique per build, keys the run-plan cache
     msf::RowRanges keep;       // columns the slice step keeps (bw_limit + propagate)
     msf_impl::DevBuf dkeep;    // keep as int2 [nx]

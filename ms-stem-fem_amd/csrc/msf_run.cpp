@@ -198,6 +198,11 @@ int check_mtf(msf_ctx* c, const msf_fem* fem)
     return MSF_OK;
 }
 
+static msf::ProbeOptics probe_optics(const msf::Domain& d, const msf_optics* o)
+{
+    return {o->corrected, o->cs3, o->cs5, o->defocus, d.lambda, d.xx[0], d.yy[0]};
+}
+
 int probe_device(msf_ctx* c, Mem& m, const msf::Domain& d, const msf_optics* o, DevBuf& hb,
                  double2** h, DevBuf& nb, double** norm2)
 {
@@ -215,8 +220,7 @@ int probe_device(msf_ctx* c, Mem& m, const msf::Domain& d, const msf_optics* o, 
     if (int r = put(c, m, ap_b, to_int2(ap), &apr)) return r;
     if (int r = take_as<double2>(c, m, hb, (size_t)nx * ny, h)) return r;
     if (int r = take_as<double>(c, m, nb, 1, norm2)) return r;
-    HIPCHK(c, msf::launch_probe_k(*h, kx, ky, nx, ny, apr, o->corrected, o->cs3, o->cs5,
-                                  o->defocus, d.lambda, d.xx[0], d.yy[0], c->stream));
+    HIPCHK(c, msf::launch_probe_k(*h, kx, ky, nx, ny, apr, probe_optics(d, o), c->stream));
     HIPCHK(c, msf::fft2d_f64(*h, nx, ny, 1, true, twx.f64, twy.f64, c->stream));
     HIPCHK(c, msf::launch_norm2(*h, (int64_t)nx * ny, *norm2, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -485,8 +489,7 @@ int prepare_groups(msf_ctx* c, Mem& m, RunPlan& pl, const msf_specimen* sp, cons
 }
 
 // Vacuum wave (t = 1) of every slice, FP64, from the probe of
-// adfstem.cpp:586-817: u0_0 = s * A_p * IFFT(H)/s; then per slice
-// w = FFT(u0_n) / s^2 * M P_n (adfstem.cpp:1986-2043), u0_{n+1} = IFFT(w).
+// adfstem.cpp:586-817 (launch_vacuum).
 // Kept while specimen and optics are unchanged (ordinary runs).
 int prepare_vacuum(msf_ctx* c, Mem& m, RunPlan& pl, const msf_specimen* sp, const msf_optics* o,
                    const RunFlags& f)
@@ -498,26 +501,51 @@ int prepare_vacuum(msf_ctx* c, Mem& m, RunPlan& pl, const msf_specimen* sp, cons
     const msf::Domain& d = sp->dom;
     const int nx = f.nx, ny = f.ny, S = f.S;
     const int64_t M = f.M;
-    DevBuf hb, nb;
-    double2* v = nullptr;
-    double* norm2 = nullptr;
-    if (int r = probe_device(c, m, d, o, hb, &v, nb, &norm2)) return r;
+    const msf::RowRanges ap = msf::aperture_keep_ranges(d, o->alpha_max);
+    if (!ap.ok) return fail(c, MSF_ERR_INVALID, "aperture is not a disk in FFT order");
+    msf::VacuumArgs va{};
+    int64_t n_ap = 0;
+    for (int i = 0; i < nx; ++i) {
+        const int n = ap.ab[2 * i] + ap.ab[2 * i + 1];
+        n_ap += n;
+        if (n > 0 && i < nx / 2) va.ra = i + 1;
+        if (n > 0 && i >= nx / 2 && va.rb == 0) va.rb = nx - i;
+    }
+    va.ca = ap.amax;
+    va.cb = std::min(ap.bmax, ny - ap.amax);
+    if (n_ap == 0) va.ra = va.ca = 1; // no probe: 0 / 0 in every pixel
+    va.nx = nx;
+    va.ny = ny;
+    va.S = S;
+    va.ld = msf::col_stride64(va.ca + va.cb, ny);
+    va.o = probe_optics(d, o);
+    va.norm = d.sqrt_nxny / std::sqrt((double)n_ap * d.nxny);
     Twiddles twx, twy;
     if (int r = twiddles(c, m, nx, twx)) return r;
     if (int r = twiddles(c, m, ny, twy)) return r;
+    DevBuf ap_b;
+    int2* apr = nullptr;
+    if (int r = put(c, m, ap_b, to_int2(ap), &apr)) return r;
+    // slices per pass: a work array of 32 MiB, or in the scratch region no
+    // more than one plane of the grid
+    const int64_t per = (int64_t)nx * va.ld * (int64_t)sizeof(double2);
+    const int64_t room = m.scratch() ? M * (int64_t)sizeof(double2) : (32ll << 20);
+    const int K = (int)std::max<int64_t>(1, std::min<int64_t>(S, room / per));
+    if (int r = take_as<double2>(c, m, pl.vac_b, (size_t)K * nx * va.ld, &va.w)) return r;
     if (int r = take_as<float2>(c, m, pl.U0, (size_t)S * 2 * M, &pl.u0)) return r;
     if (int r = take_as<float2>(c, m, pl.Psi0, (size_t)M, &pl.psi0)) return r;
-    HIPCHK(c, msf::launch_scale_f64(v, M, norm2, d.sqrt_nxny, c->stream));
-    for (int n = 0; n < S; ++n) {
-        HIPCHK(c, msf::launch_to_f32_shift_pairs(v, nx, ny, pl.u0 + (int64_t)n * 2 * M, c->stream));
-        HIPCHK(c, msf::fft2d_f64(v, nx, ny, 1, false, twx.f64, twy.f64, c->stream));
-        HIPCHK(c, msf::launch_vacuum_step(v, nx, ny, sp->px64.as<double2>() + (int64_t)n * nx,
-                                          sp->py64.as<double2>() + (int64_t)n * ny,
-                                          sp->dkeep.as<int2>(), 1.0 / (d.sqrt_nxny * d.sqrt_nxny),
-                                          c->stream));
-        if (n + 1 < S) HIPCHK(c, msf::fft2d_f64(v, nx, ny, 1, true, twx.f64, twy.f64, c->stream));
+    HIPCHK(c, hipMemsetAsync(pl.psi0, 0, (size_t)M * sizeof(float2), c->stream));
+    va.psi0 = pl.psi0;
+    va.kx = sp->dkx.as<double>();
+    va.ky = sp->dky.as<double>();
+    va.ap = apr;
+    va.keep = sp->dkeep.as<int2>();
+    va.px = sp->px64.as<double2>();
+    va.py = sp->py64.as<double2>();
+    for (va.n0 = 0; va.n0 < S; va.n0 = va.n1) {
+        va.n1 = std::min(S, va.n0 + K);
+        HIPCHK(c, msf::launch_vacuum(va, pl.u0 + (int64_t)va.n0 * 2 * M, twx.f64, twy.f64, c->stream));
     }
-    HIPCHK(c, msf::launch_to_f32_transposed(v, nx, ny, pl.psi0, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     pl.spec_id = sp->id;
     pl.optics = *o;
