@@ -191,26 +191,33 @@ hipError_t launch_probe_k(double2* h, const double* kx, const double* ky, int nx
                           const int2* aperture, const ProbeOptics& o, hipStream_t s);
 // sum |a|^2 over n values (one workgroup, fixed order)
 hipError_t launch_norm2(const double2* a, int64_t n, double* out, hipStream_t s);
-hipError_t launch_fill_f64(double2* a, int64_t n, hipStream_t s);
 // out[0, n16) = in[0, n16), 16-byte vectors; n16 a multiple of 1024
 hipError_t launch_stream_copy(const float4* in, float4* out, int64_t n16, hipStream_t s);
-// atom count maps: maps[(slot*nsp + sp)][sx][sy] += 1
-hipError_t launch_scatter_atoms(double2* maps, const int4* atoms, int n_atoms, int nx, int ny,
-                                int nsp, hipStream_t s);
-// sigma_k[slot] = sum_sp T_sp(k) C_sp(k)   (scatterer_pap.hpp:104-130 template)
-hipError_t launch_combine_species(const double2* maps, double2* sigma, int slots, int nsp,
-                                  const double* params /* nsp*12 */, const double* kx,
-                                  const double* ky, int nx, int ny, const int2* support,
-                                  double lgab, double xmin, double ymin, hipStream_t s);
-// t = exp(-Im v) (cos Re v, sin Re v), v = sigma * scale
-hipError_t launch_exp_transmit(double2* a, int64_t n, double scale, hipStream_t s);
+// Transmission functions of a chunk of slices [s0, s0 + k).
+struct BuildArgs {
+    int nx, ny, nsp, k, s0;
+    bool half;               // spectra on ky >= 0 only (sb == 0), the rest by conjugation
+    int sa, sb, lds;         // columns of the template support [0, sa) U [ny - sb, ny), stride
+    int ba, bb, ldb;         // columns of the band limit, stride
+    double2* spec;           // [k][nsp][nx][lds]
+    double2* band;           // [k][nx][ldb]
+    uint32_t* maps;          // [k][nsp][nx][ny] atom counts, zeroed by the caller
+    double* tmpl;            // [nsp][nx][lds] f_e lambda gamma / (a b), 0 outside the support
+    const int4* atoms;       // (slice, species, sx, sy) of the chunk
+    int n_atoms;
+    const int2 *support, *bw; // per row
+    const double *kx, *ky, *params /* nsp * 12 */;
+    double xmin, ymin, lgab, s /* sqrt(nx ny) */, nxny, sqrt_nxny;
+    double2* t64;            // [k][nx][ny] t
+    float2* t32;             // [k][nx][ny] (t_re/s - 1/s, t_im/s), rows in the pair layout
+};
+// tmpl for every species (projected_atomic_potential.cpp:169-225)
+hipError_t launch_templates(const BuildArgs& a, hipStream_t s);
+// t64 and t32 of the chunk
+hipError_t launch_build(const BuildArgs& a, const double2* twx, const double2* twy, hipStream_t s);
 // zero outside the kept ranges
 hipError_t launch_apply_keep(double2* a, int nx, int ny, int count, const int2* keep,
                              hipStream_t s);
-// t = a / nxny (FP64, kept for queries); t32 = (t_re/s - 1/s, t_im/s) in FP32,
-// each row of ny in the pair layout (pair_pos)
-hipError_t launch_finish_transmit(double2* a, int64_t n, int ny, double nxny, double s,
-                                  float2* t32, hipStream_t st);
 // one vacuum slice step in k-space: a *= keep ? P_x[i] P_y[j] * scale : 0
 hipError_t launch_vacuum_step(double2* a, int nx, int ny, const double2* px, const double2* py,
                               const int2* keep, double scale, hipStream_t s);

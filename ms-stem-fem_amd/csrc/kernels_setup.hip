@@ -184,18 +184,6 @@ hipError_t launch_norm2(const double2* a, int64_t n, double* out, hipStream_t s)
     return hipGetLastError();
 }
 
-__global__ void fill_f64_kernel(double2* a, int64_t n)
-{
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) a[k] = double2{0.0, 0.0};
-}
-
-hipError_t launch_fill_f64(double2* a, int64_t n, hipStream_t s)
-{
-    hipLaunchKernelGGL(fill_f64_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, n);
-    return hipGetLastError();
-}
-
 // ------------------------------------------------------------ measurement
 // A streaming copy at the rate HBM sustains for a plain read + write: each
 // lane moves four 16-byte vectors, the four loads issued before the stores.
@@ -220,88 +208,234 @@ hipError_t launch_stream_copy(const float4* in, float4* out, int64_t n16, hipStr
 }
 
 // ------------------------------------------------------------ transmission
-// atoms[k] = (slot, species, sx, sy); counts are small integers, so the FP64
-// atomic sums are exact and order-independent
-__global__ void scatter_atoms_kernel(double2* maps, const int4* atoms, int n_atoms, int nx,
-                                     int ny, int nsp)
+// Passes of one chunk of slices (columns of `spec` and `band` only):
+//   scatter  atoms -> count maps (small integers, so the atomic sums are exact
+//            and order-independent)
+//   rows     FFT_y of the maps                              -> spec
+//   columns  sum_sp T_sp(k) FFT_x(spec), IFFT_x             -> spec
+//   rows     IFFT_y, t = exp(-Im v)(cos Re v, sin Re v), FFT_y -> band
+//   columns  FFT_x, bw_limit, IFFT_x                        -> band (in place)
+//   rows     IFFT_y, / NxNy                                 -> t64, t32
+// Each transform pair shares a pass with the element-wise work between and
+// around it, and only columns that carry data are stored (half the spectrum
+// of a real map, 2/3 of a band-limited plane): 25 slices of 1024^2 with one
+// species move 2.8 GB instead of 7.5 GB in eleven passes over full planes,
+// whose column passes also lost half of each 128-byte line to another XCD;
+// the kernels of that build went from 3.6 to 1.2 ms.
+__global__ void scatter_atoms_kernel(BuildArgs a)
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n_atoms) return;
-    const int4 a = atoms[k];
-    double* dst = &maps[(((int64_t)a.x * nsp + a.y) * nx + a.z) * ny + a.w].x;
-    atomicAdd(dst, 1.0);
+    const int n = blockIdx.x * blockDim.x + threadIdx.x;
+    if (n >= a.n_atoms) return;
+    const int4 at = a.atoms[n];
+    atomicAdd(&a.maps[(((int64_t)(at.x - a.s0) * a.nsp + at.y) * a.nx + at.z) * a.ny + at.w], 1u);
 }
 
-hipError_t launch_scatter_atoms(double2* maps, const int4* atoms, int n_atoms, int nx, int ny,
-                                int nsp, hipStream_t s)
+// projected_atomic_potential.cpp:169-225: lambda*gamma/(ab) * f_e(|k|^2)
+// inside the template support
+__global__ void __launch_bounds__(256) template_kernel(BuildArgs a)
 {
-    if (n_atoms <= 0) return hipSuccess;
-    hipLaunchKernelGGL(scatter_atoms_kernel, dim3((n_atoms + 255) / 256), dim3(256), 0, s, maps,
-                       atoms, n_atoms, nx, ny, nsp);
+    const int nc = a.sa + a.sb;
+    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= (int64_t)a.nsp * a.nx * nc) return;
+    const int c = (int)(idx % nc);
+    const int64_t r = idx / nc;
+    const int i = (int)(r % a.nx), sp = (int)(r / a.nx);
+    const int j = c < a.sa ? c : c + a.ny - nc;
+    const int2 k = a.support[i];
+    double t = 0.0;
+    if (j < k.x || j >= a.ny - k.y) {
+        const double ksq = (a.kx[i] * a.kx[i]) + (a.ky[j] * a.ky[j]);
+        const double* p = a.params + 12 * sp;
+        t = a.lgab * (p[0] / (ksq + p[3]) + p[1] / (ksq + p[4]) + p[2] / (ksq + p[5])
+                      + p[6] * exp(-p[9] * ksq) + p[7] * exp(-p[10] * ksq)
+                      + p[8] * exp(-p[11] * ksq));
+    }
+    a.tmpl[r * a.lds + c] = t;
+}
+
+hipError_t launch_templates(const BuildArgs& a, hipStream_t s)
+{
+    const int64_t n = (int64_t)a.nsp * a.nx * (a.sa + a.sb);
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(template_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
-// projected_atomic_potential.cpp:169-225: lambda*gamma/(ab) * f_e(|k|^2) *
-// e^{2 pi i k.(xmin, ymin)} inside the template support
-__global__ void combine_species_kernel(const double2* maps, double2* sigma, int slots, int nsp,
-                                       const double* params, const double* kx, const double* ky,
-                                       int nx, int ny, const int2* support, double lgab,
-                                       double xmin, double ymin)
-{
-    const int64_t plane = (int64_t)nx * ny;
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= plane * slots) return;
-    const int64_t pix = idx % plane;
-    const int64_t slot = idx / plane;
-    const int i = (int)(pix / ny), j = (int)(pix % ny);
-    const int2 r = support[i];
-    double2 acc{0.0, 0.0};
-    if (j < r.x || j >= ny - r.y) {
-        const double ksq = (kx[i] * kx[i]) + (ky[j] * ky[j]);
-        double sn, cs;
-        sincos(2 * kPi * (kx[i] * xmin + ky[j] * ymin), &sn, &cs);
-        for (int sp = 0; sp < nsp; ++sp) {
-            const double* p = params + 12 * sp;
-            const double fe = p[0] / (ksq + p[3]) + p[1] / (ksq + p[4]) + p[2] / (ksq + p[5])
-                              + p[6] * exp(-p[9] * ksq) + p[7] * exp(-p[10] * ksq)
-                              + p[8] * exp(-p[11] * ksq);
-            const double2 tk{lgab * fe * cs, lgab * fe * sn};
-            const double2 c = maps[(slot * nsp + sp) * plane + pix];
-            acc.x += tk.x * c.x - tk.y * c.y;
-            acc.y += tk.x * c.y + tk.y * c.x;
+struct MapRows {
+    const uint32_t* maps;
+    double2* spec;
+    int nx, ny, sa, sb, lds;
+    __device__ __forceinline__ double2 load(int plane, int i, int j) const
+    {
+        return double2{(double)maps[((int64_t)plane * nx + i) * ny + j], 0.0};
+    }
+    template <int E, int T>
+    __device__ __forceinline__ void store(int plane, int i, int t, const double2 (&x)[E]) const
+    {
+        double2* row = spec + ((int64_t)plane * nx + i) * lds;
+#pragma unroll
+        for (int p = 0; p < E; ++p) {
+            const int j = t + T * p;
+            if (j < sa) row[j] = x[p];
+            else if (j >= ny - sb) row[j - ny + sa + sb] = x[p];
         }
     }
-    sigma[idx] = acc;
-}
+};
 
-hipError_t launch_combine_species(const double2* maps, double2* sigma, int slots, int nsp,
-                                  const double* params, const double* kx, const double* ky,
-                                  int nx, int ny, const int2* support, double lgab, double xmin,
-                                  double ymin, hipStream_t s)
-{
-    const int64_t n = (int64_t)nx * ny * slots;
-    hipLaunchKernelGGL(combine_species_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
-                       maps, sigma, slots, nsp, params, kx, ky, nx, ny, support, lgab, xmin, ymin);
-    return hipGetLastError();
-}
+struct SpeciesCols {
+    int inputs;
+    double2* spec;
+    const double *tmpl, *kx, *ky;
+    int nx, ny, sa, sb, lds;
+    bool origin; // domain minima at 0: the template's phase is 1
+    double xmin, ymin;
+    __device__ __forceinline__ double2 load(int plane, int in, int i, int c) const
+    {
+        return spec[(((int64_t)plane * inputs + in) * nx + i) * lds + c];
+    }
+    __device__ __forceinline__ double2 mid(int, int in, int i, int c, double2 v) const
+    {
+        const double f = tmpl[((int64_t)in * nx + i) * lds + c];
+        if (origin) return double2{f * v.x, f * v.y};
+        const int j = c < sa ? c : c + ny - sa - sb;
+        double sn, cs;
+        sincos(2 * kPi * (kx[i] * xmin + ky[j] * ymin), &sn, &cs);
+        const double2 t{f * cs, f * sn};
+        return double2{t.x * v.x - t.y * v.y, t.x * v.y + t.y * v.x};
+    }
+    __device__ __forceinline__ void store(int plane, int i, int c, double2 v) const
+    {
+        spec[((int64_t)plane * inputs * nx + i) * lds + c] = v; // over species 0
+    }
+};
 
 // slice.cpp:1700-1725
-__global__ void exp_transmit_kernel(double2* a, int64_t n, double scale)
-{
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const double re = a[k].x * scale, im = a[k].y * scale;
-    const double e = exp(-im);
-    double sn, cs;
-    sincos(re, &sn, &cs);
-    a[k] = double2{e * cs, e * sn};
-}
+struct TransmitRows {
+    const double2* spec; // null: no atoms
+    double2* band;
+    int nsp, nx, ny, sa, sb, lds, ba, bb, ldb;
+    bool half;
+    double scale;
+    __device__ __forceinline__ double2 load(int plane, int i, int j) const
+    {
+        if (!spec) return double2{0.0, 0.0};
+        const double2* row = spec + ((int64_t)plane * nsp * nx + i) * lds;
+        if (j < sa) return row[j];
+        if (half) {
+            if (ny - j >= sa) return double2{0.0, 0.0};
+            const double2 v = row[ny - j];
+            return double2{v.x, -v.y};
+        }
+        return j >= ny - sb ? row[j - ny + sa + sb] : double2{0.0, 0.0};
+    }
+    __device__ __forceinline__ double2 mid(int, int, int, double2 v) const
+    {
+        const double re = v.x * scale, im = v.y * scale;
+        // Im v is rounding of a real sum; exp of so small a value by its
+        // series (the next term is below 2e-19)
+        const double e = fabs(im) < 1e-6 ? 1.0 - im + 0.5 * im * im : exp(-im);
+        double sn, cs;
+        sincos(re, &sn, &cs);
+        return double2{e * cs, e * sn};
+    }
+    template <int E, int T>
+    __device__ __forceinline__ void store(int plane, int i, int t, const double2 (&x)[E]) const
+    {
+        double2* row = band + ((int64_t)plane * nx + i) * ldb;
+#pragma unroll
+        for (int p = 0; p < E; ++p) {
+            const int j = t + T * p;
+            if (j < ba) row[j] = x[p];
+            else if (j >= ny - bb) row[j - ny + ba + bb] = x[p];
+        }
+    }
+};
 
-hipError_t launch_exp_transmit(double2* a, int64_t n, double scale, hipStream_t s)
+struct BandCols {
+    static constexpr int inputs = 1;
+    double2* band;
+    const int2* bw;
+    int nx, ny, ba, bb, ldb;
+    __device__ __forceinline__ double2 load(int plane, int, int i, int c) const
+    {
+        return band[((int64_t)plane * nx + i) * ldb + c];
+    }
+    __device__ __forceinline__ double2 mid(int, int, int i, int c, double2 v) const
+    {
+        const int j = c < ba ? c : c + ny - ba - bb;
+        const int2 r = bw[i];
+        return (j < r.x || j >= ny - r.y) ? v : double2{0.0, 0.0};
+    }
+    __device__ __forceinline__ void store(int plane, int i, int c, double2 v) const
+    {
+        band[((int64_t)plane * nx + i) * ldb + c] = v;
+    }
+};
+
+// slice.cpp:1741-1748 (/ NxNy).  The FP32 copy used by the slice loop holds
+// t' = t/s (adfstem.cpp:1936,1949 divide by sqrtNxNy) as (t're - 1/s, t'im):
+// the deviation from vacuum keeps full FP32 relative precision.
+struct FinishRows {
+    const double2* band;
+    double2* t64;
+    float2* t32;
+    int nx, ny, ba, bb, ldb;
+    double nxny, s;
+    __device__ __forceinline__ double2 load(int plane, int i, int j) const
+    {
+        const double2* row = band + ((int64_t)plane * nx + i) * ldb;
+        if (j < ba) return row[j];
+        return j >= ny - bb ? row[j - ny + ba + bb] : double2{0.0, 0.0};
+    }
+    template <int E, int T>
+    __device__ __forceinline__ void store(int plane, int i, int t, const double2 (&x)[E]) const
+    {
+        const int64_t r = (int64_t)plane * nx + i;
+        double2* row = t64 + r * ny;
+        float4* pairs = reinterpret_cast<float4*>(t32 + r * ny); // elements j and j + ny/2 (pair_pos)
+#pragma unroll
+        for (int p = 0; p < E / 2; ++p) {
+            const int j = t + T * p;
+            const double2 a{x[p].x / nxny, x[p].y / nxny};
+            const double2 b{x[p + E / 2].x / nxny, x[p + E / 2].y / nxny};
+            row[j] = a;
+            row[j + ny / 2] = b;
+            pairs[j] = float4{(float)(a.x / s - 1.0 / s), (float)(a.y / s),
+                              (float)(b.x / s - 1.0 / s), (float)(b.y / s)};
+        }
+    }
+};
+
+hipError_t launch_build(const BuildArgs& a, const double2* twx, const double2* twy, hipStream_t s)
 {
-    hipLaunchKernelGGL(exp_transmit_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a,
-                       n, scale);
-    return hipGetLastError();
+    hipError_t e = hipSuccess;
+    if (a.nsp > 0) {
+        if (a.n_atoms > 0) {
+            hipLaunchKernelGGL(scatter_atoms_kernel, dim3((a.n_atoms + 255) / 256), dim3(256), 0, s, a);
+            e = hipGetLastError();
+        }
+        if (e == hipSuccess)
+            e = launch_rows64<Fft64::Forward>(
+                a.ny, MapRows{a.maps, a.spec, a.nx, a.ny, a.sa, a.sb, a.lds}, a.nx, a.k * a.nsp, twy, s);
+        if (e == hipSuccess)
+            e = launch_cols64<Fft64::ForwardInverse>(
+                a.nx, SpeciesCols{a.nsp, a.spec, a.tmpl, a.kx, a.ky, a.nx, a.ny, a.sa, a.sb, a.lds,
+                                  a.xmin == 0.0 && a.ymin == 0.0, a.xmin, a.ymin},
+                a.sa + a.sb, a.k, twx, s);
+    }
+    if (e == hipSuccess)
+        e = launch_rows64<Fft64::InverseForward>(
+            a.ny, TransmitRows{a.nsp > 0 ? a.spec : nullptr, a.band, a.nsp, a.nx, a.ny, a.sa, a.sb,
+                               a.lds, a.ba, a.bb, a.ldb, a.half, 1.0 / a.s},
+            a.nx, a.k, twy, s);
+    if (e == hipSuccess)
+        e = launch_cols64<Fft64::ForwardInverse>(
+            a.nx, BandCols{a.band, a.bw, a.nx, a.ny, a.ba, a.bb, a.ldb}, a.ba + a.bb, a.k, twx, s);
+    if (e == hipSuccess)
+        e = launch_rows64<Fft64::Inverse>(
+            a.ny, FinishRows{a.band, a.t64, a.t32, a.nx, a.ny, a.ba, a.bb, a.ldb, a.nxny, a.sqrt_nxny},
+            a.nx, a.k, twy, s);
+    return e;
 }
 
 __global__ void apply_keep_kernel(double2* a, int nx, int ny, int64_t total, const int2* keep)
@@ -320,28 +454,6 @@ hipError_t launch_apply_keep(double2* a, int nx, int ny, int count, const int2* 
     const int64_t n = (int64_t)nx * ny * count;
     hipLaunchKernelGGL(apply_keep_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, nx,
                        ny, n, keep);
-    return hipGetLastError();
-}
-
-// slice.cpp:1741-1748 (/ NxNy).  The FP32 copy used by the slice loop holds
-// t' = t/s (adfstem.cpp:1936,1949 divide by sqrtNxNy) as (t're - 1/s, t'im):
-// the deviation from vacuum keeps full FP32 relative precision.
-__global__ void finish_transmit_kernel(double2* a, int64_t n, int ny, double nxny, double s,
-                                       float2* t32)
-{
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const double2 t{a[k].x / nxny, a[k].y / nxny};
-    a[k] = t;
-    const int j = (int)(k % ny);
-    t32[k - j + pair_pos(j, ny)] = float2{(float)(t.x / s - 1.0 / s), (float)(t.y / s)};
-}
-
-hipError_t launch_finish_transmit(double2* a, int64_t n, int ny, double nxny, double s,
-                                  float2* t32, hipStream_t st)
-{
-    hipLaunchKernelGGL(finish_transmit_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                       a, n, ny, nxny, s, t32);
     return hipGetLastError();
 }
 

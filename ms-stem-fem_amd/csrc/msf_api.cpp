@@ -219,23 +219,13 @@ int msf_specimen_build(msf_ctx* c, const msf_grid* grid, const double* q, const 
             delete sp;
             return fail(c, MSF_ERR_INVALID, "band limit is not a disk in FFT order");
         }
-        if (hipError_t e = upload(sp->dkeep, to_int2(sp->keep), c->stream)) {
+        // the column pass's view of the same set, per compact column
+        const int W = msf::col_tile(nx);
+        const int ncp = std::max(W, ((sp->keep.amax + sp->keep.bmax + W - 1) / W) * W);
+        const msf::RowRanges ck = msf::column_keep_ranges(sp->keep, nx, ny, ncp);
+        if (!ck.ok) {
             delete sp;
-            return fail(c, MSF_ERR_DEVICE, hipGetErrorString(e));
-        }
-        {   // the column pass's view of the same set, per compact column
-            const int W = msf::col_tile(nx);
-            const int ncp = std::max(W, ((sp->keep.amax + sp->keep.bmax + W - 1) / W) * W);
-            const msf::RowRanges ck = msf::column_keep_ranges(sp->keep, nx, ny, ncp);
-            if (!ck.ok) {
-                delete sp;
-                return fail(c, MSF_ERR_UNSUPPORTED, "band limit is not a disk by column");
-            }
-            if (hipError_t e = upload(sp->dcolkeep, to_int2(ck), c->stream)) {
-                (void)hipGetLastError();
-                delete sp;
-                return fail(c, MSF_ERR_DEVICE, hipGetErrorString(e));
-            }
+            return fail(c, MSF_ERR_UNSUPPORTED, "band limit is not a disk by column");
         }
 
         // species present, ascending Z (tem.cpp:944-972)
@@ -279,29 +269,29 @@ int msf_specimen_build(msf_ctx* c, const msf_grid* grid, const double* q, const 
         // propagators (slice.cpp:1293-1363), FP64 -> FP32; P_y carries 1/sqrtNxNy
         std::vector<float2> pxs((size_t)S * nx), pys((size_t)S * ny);
         std::vector<double2> pxd((size_t)S * nx), pyd((size_t)S * ny);
+        const bool same_axes = d.kx == d.ky;
+        std::vector<double> p;
         for (int s = 0; s < S; ++s) {
-            std::vector<double> p;
             msf::propagator(d.lambda, sl.thick[s], d.kx, d.bw_t, p);
             for (int i = 0; i < nx; ++i) {
                 pxd[(size_t)s * nx + i] = double2{p[2 * i], p[2 * i + 1]};
                 pxs[(size_t)s * nx + i] = float2{(float)p[2 * i], (float)p[2 * i + 1]};
             }
-            msf::propagator(d.lambda, sl.thick[s], d.ky, d.bw_t, p);
+            if (!same_axes) msf::propagator(d.lambda, sl.thick[s], d.ky, d.bw_t, p);
             for (int j = 0; j < ny; ++j) {
                 pyd[(size_t)s * ny + j] = double2{p[2 * j], p[2 * j + 1]};
                 pys[(size_t)s * ny + j] = float2{(float)(p[2 * j] / d.sqrt_nxny), (float)(p[2 * j + 1] / d.sqrt_nxny)};
             }
         }
-        int rc = MSF_OK;
         auto bail = [&](int code) {
             (void)hipGetLastError(); // the failure is reported here, not by a later launch
             delete sp;
             return code;
         };
-        if (hipError_t e = upload(sp->px, pxs, c->stream)) return bail(fail(c, MSF_ERR_DEVICE, hipGetErrorString(e)));
-        if (hipError_t e = upload(sp->py, pys, c->stream)) return bail(fail(c, MSF_ERR_DEVICE, hipGetErrorString(e)));
-        if (hipError_t e = upload(sp->px64, pxd, c->stream)) return bail(fail(c, MSF_ERR_DEVICE, hipGetErrorString(e)));
-        if (hipError_t e = upload(sp->py64, pyd, c->stream)) return bail(fail(c, MSF_ERR_DEVICE, hipGetErrorString(e)));
+        auto device_error = [&](hipError_t e) {
+            return bail(fail(c, e == hipErrorOutOfMemory ? MSF_ERR_MEMORY : MSF_ERR_DEVICE,
+                             std::string("specimen build: ") + hipGetErrorString(e)));
+        };
 
         // transmission functions, FP64 on the device, in chunks of slices
         const msf::RowRanges sup = msf::template_keep_ranges(d);
@@ -312,66 +302,98 @@ int msf_specimen_build(msf_ctx* c, const msf_grid* grid, const double* q, const 
         const int64_t M = (int64_t)nx * ny;
         Mem heap;
         Twiddles tx, ty;
-        if ((rc = twiddles(c, heap, nx, tx))) return bail(rc);
-        if ((rc = twiddles(c, heap, ny, ty))) return bail(rc);
-        const double2 *twx = tx.f64, *twy = ty.f64;
-        DevBuf dsup, dbw, dpar, dmaps, datoms;
-        hipError_t e = hipSuccess;
-        if (!e) e = upload(sp->dkx, d.kx, c->stream);
-        if (!e) e = upload(sp->dky, d.ky, c->stream);
-        if (!e) e = upload(dsup, to_int2(sup), c->stream);
-        if (!e) e = upload(dbw, to_int2(bw), c->stream);
-        if (!e) e = upload(dpar, params, c->stream);
+        if (int rc = twiddles(c, heap, nx, tx)) return bail(rc);
+        if (int rc = twiddles(c, heap, ny, ty)) return bail(rc);
+
+        // every small table of the specimen and of its build in one copy
+        std::vector<char> blob;
+        std::vector<std::pair<DevBuf*, std::pair<size_t, size_t>>> views;
+        auto pack = [&](DevBuf& b, const auto& v) {
+            const size_t at = (blob.size() + 255) & ~size_t(255), n = v.size() * sizeof(v[0]);
+            blob.resize(at + std::max<size_t>(n, 16));
+            if (n) std::memcpy(blob.data() + at, v.data(), n);
+            views.push_back({&b, {at, std::max<size_t>(n, 16)}});
+        };
+        DevBuf dsup, dbw, dpar, datoms;
+        pack(sp->dkeep, to_int2(sp->keep));
+        pack(sp->dcolkeep, to_int2(ck));
+        pack(sp->px, pxs);
+        pack(sp->py, pys);
+        pack(sp->px64, pxd);
+        pack(sp->py64, pyd);
+        pack(sp->dkx, d.kx);
+        pack(sp->dky, d.ky);
+        pack(dsup, to_int2(sup));
+        pack(dbw, to_int2(bw));
+        pack(dpar, params);
+        pack(datoms, atoms);
+        hipError_t e = upload(sp->tables, blob, c->stream);
+        if (e) return device_error(e);
+        for (auto& v : views) v.first->view(sp->tables.as<char>() + v.second.first, v.second.second);
         if (!e) e = sp->t64.alloc((size_t)S * M * sizeof(double2));
         if (!e) e = sp->t32.alloc((size_t)S * M * sizeof(float2));
-        const int64_t per_slot = (int64_t)std::max(nsp, 1) * M * (int64_t)sizeof(double2);
-        const int K = (int)std::max<int64_t>(1, std::min<int64_t>(S, (256ll << 20) / per_slot));
-        if (!e) e = dmaps.alloc((size_t)K * per_slot);
-        if (!e) e = datoms.alloc(std::max<size_t>(atoms.size(), 1) * sizeof(int4));
-        if (!e && !atoms.empty())
-            e = hipMemcpyAsync(datoms.p, atoms.data(), atoms.size() * sizeof(int4), hipMemcpyHostToDevice,
-                               c->stream);
-        if (e) {
-            (void)hipGetLastError();
-            return bail(fail(c, e == hipErrorOutOfMemory ? MSF_ERR_MEMORY : MSF_ERR_DEVICE, hipGetErrorString(e)));
+
+        msf::BuildArgs ba{};
+        ba.nx = nx;
+        ba.ny = ny;
+        ba.nsp = nsp;
+        // Count maps are real, so the template spectra on either side of
+        // ky = 0 are conjugates and one side is transformed, provided the
+        // template's support (decided pixel by pixel) is symmetric too.
+        ba.half = sup.amax <= ny / 2;
+        for (int i = 0; i < nx && ba.half; ++i) {
+            const int a = sup.ab[2 * i], b = sup.ab[2 * ((nx - i) % nx) + 1];
+            ba.half = std::max(a - 1, 0) == b;
         }
-        const double lgab = d.lambda * d.gamma * (1 / (grid->xperiod * grid->yperiod));
+        ba.sa = sup.amax;
+        ba.sb = ba.half ? 0 : std::min(sup.bmax, ny - sup.amax);
+        ba.ba = bw.amax;
+        ba.bb = bw.bmax;
+        ba.lds = msf::col_stride64(ba.sa + ba.sb, ny);
+        ba.ldb = msf::col_stride64(ba.ba + ba.bb, ny);
+        ba.support = dsup.as<int2>();
+        ba.bw = dbw.as<int2>();
+        ba.kx = sp->dkx.as<double>();
+        ba.ky = sp->dky.as<double>();
+        ba.params = dpar.as<double>();
+        ba.xmin = grid->xmin;
+        ba.ymin = grid->ymin;
+        ba.lgab = d.lambda * d.gamma * (1 / (grid->xperiod * grid->yperiod));
+        ba.s = std::sqrt((double)M);
+        ba.nxny = d.nxny;
+        ba.sqrt_nxny = d.sqrt_nxny;
+        // slices per chunk: work arrays of 96 MiB, which stay in the 256 MB
+        // Infinity Cache between the passes
+        const int64_t spectra = (int64_t)std::max(nsp, 1) * nx * ba.lds * (int64_t)sizeof(double2);
+        const int64_t band = (int64_t)nx * ba.ldb * (int64_t)sizeof(double2);
+        const int64_t maps = (int64_t)std::max(nsp, 1) * M * (int64_t)sizeof(uint32_t);
+        const int K = (int)std::max<int64_t>(1, std::min<int64_t>(S, (96ll << 20) / (spectra + band + maps)));
+        const int64_t tmpl = (int64_t)std::max(nsp, 1) * nx * ba.lds * (int64_t)sizeof(double);
+        DevBuf work;
+        if (!e) e = work.alloc((size_t)(K * (spectra + band + maps) + tmpl));
+        if (e) return device_error(e);
+        ba.spec = work.as<double2>();
+        ba.band = reinterpret_cast<double2*>(work.as<char>() + K * spectra);
+        ba.maps = reinterpret_cast<uint32_t*>(work.as<char>() + K * (spectra + band));
+        ba.tmpl = reinterpret_cast<double*>(work.as<char>() + K * (spectra + band + maps));
+        if (nsp > 0) e = msf::launch_templates(ba, c->stream);
         size_t a0 = 0;
         for (int s0 = 0; s0 < S && !e; s0 += K) {
-            const int k = std::min(K, S - s0);
+            ba.s0 = s0;
+            ba.k = std::min(K, S - s0);
             size_t a1 = a0;
-            while (a1 < atoms.size() && atoms[a1].x < s0 + k) ++a1;
-            // slots are relative to the chunk
-            std::vector<int4> chunk(atoms.begin() + a0, atoms.begin() + a1);
-            for (auto& at : chunk) at.x -= s0;
-            if (!chunk.empty())
-                e = hipMemcpyAsync(datoms.p, chunk.data(), chunk.size() * sizeof(int4), hipMemcpyHostToDevice,
-                                   c->stream);
-            double2* maps = dmaps.as<double2>();
-            double2* sig = sp->t64.as<double2>() + (int64_t)s0 * M;
-            if (!e) e = msf::launch_fill_f64(maps, (int64_t)k * std::max(nsp, 1) * M, c->stream);
-            if (!e) e = msf::launch_scatter_atoms(maps, datoms.as<int4>(), (int)chunk.size(), nx, ny,
-                                                  std::max(nsp, 1), c->stream);
-            if (!e && nsp > 0) e = msf::fft2d_f64(maps, nx, ny, k * nsp, false, twx, twy, c->stream);
-            if (!e) e = msf::launch_combine_species(maps, sig, k, nsp, dpar.as<double>(),
-                                                    sp->dkx.as<double>(), sp->dky.as<double>(), nx, ny, dsup.as<int2>(), lgab,
-                                                    grid->xmin, grid->ymin, c->stream);
-            if (!e) e = msf::fft2d_f64(sig, nx, ny, k, true, twx, twy, c->stream);
-            if (!e) e = msf::launch_exp_transmit(sig, (int64_t)k * M, 1.0 / std::sqrt((double)M), c->stream);
-            if (!e) e = msf::fft2d_f64(sig, nx, ny, k, false, twx, twy, c->stream);
-            if (!e) e = msf::launch_apply_keep(sig, nx, ny, k, dbw.as<int2>(), c->stream);
-            if (!e) e = msf::fft2d_f64(sig, nx, ny, k, true, twx, twy, c->stream);
-            if (!e) e = msf::launch_finish_transmit(sig, (int64_t)k * M, ny, d.nxny, d.sqrt_nxny,
-                                                    sp->t32.as<float2>() + (int64_t)s0 * M, c->stream);
-            // the atom list buffer is reused by the next chunk
-            if (!e) e = hipStreamSynchronize(c->stream);
+            while (a1 < atoms.size() && atoms[a1].x < s0 + ba.k) ++a1;
+            ba.atoms = datoms.as<int4>() + a0;
+            ba.n_atoms = (int)(a1 - a0);
+            ba.t64 = sp->t64.as<double2>() + (int64_t)s0 * M;
+            ba.t32 = sp->t32.as<float2>() + (int64_t)s0 * M;
+            if (nsp > 0) e = hipMemsetAsync(ba.maps, 0, (size_t)(ba.k * maps), c->stream);
+            if (!e) e = msf::launch_build(ba, tx.f64, ty.f64, c->stream);
             a0 = a1;
         }
         if (!e) e = hipStreamSynchronize(c->stream);
-        if (e) {
-            (void)hipGetLastError();
-            return bail(fail(c, MSF_ERR_DEVICE, std::string("transmission build: ") + hipGetErrorString(e)));
-        }
+        for (DevBuf* b : {&dsup, &dbw, &dpar, &datoms}) b->release();
+        if (e) return device_error(e);
         c->specimens.insert(sp);
         *out = sp;
         return MSF_OK;

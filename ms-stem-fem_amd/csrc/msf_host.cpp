@@ -85,23 +85,9 @@ RowRanges column_keep_ranges(const RowRanges& rows, int nx, int ny, int ncp)
 {
     const int ka = rows.amax, kb = rows.bmax, nc = ka + kb;
     auto kept = [&](int i, int j) { return j < rows.ab[2 * i] || j >= ny - rows.ab[2 * i + 1]; };
-    RowRanges r;
-    r.ab.assign(2 * (size_t)ncp, 0);
-    for (int jc = 0; jc < ncp && jc < nc; ++jc) {
-        const int j = jc < ka ? jc : jc - nc + ny;
-        int c = 0;
-        while (c < nx && kept(c, j)) ++c;
-        int d = 0;
-        if (c < nx)
-            while (d < nx - c && kept(nx - 1 - d, j)) ++d;
-        for (int i = c; i < nx - d; ++i)
-            if (kept(i, j)) r.ok = false;
-        r.ab[2 * jc] = c;
-        r.ab[2 * jc + 1] = d;
-        r.amax = std::max(r.amax, c);
-        r.bmax = std::max(r.bmax, d);
-    }
-    return r;
+    return row_ranges(ncp, nx, [&](int jc, int i) {
+        return jc < nc && kept(i, jc < ka ? jc : jc - nc + ny);
+    });
 }
 
 RowRanges bwlimit_keep_ranges(const Domain& d)
@@ -132,15 +118,15 @@ int64_t shift_index(const std::vector<double>& grid, double q, int64_t previous)
 {
     // The reference scans for the first i with grid[i] - q >= half.  The grid
     // is non-decreasing and rounded subtraction of a fixed q is monotone, so
-    // the test holds from that index on and a bisection finds the same i.
-    const double half = 0.5 * (grid[1] - grid[0]);
-    size_t lo = 0, hi = grid.size();
-    while (lo < hi) {
-        const size_t mid = lo + (hi - lo) / 2;
-        if (grid[mid] - q >= half) hi = mid;
-        else lo = mid + 1;
-    }
-    return lo < grid.size() ? (int64_t)lo - 1 : previous;
+    // the test holds from that index on: start where an even spacing puts it
+    // and step to it.
+    const double step = grid[1] - grid[0], half = 0.5 * step;
+    const size_t n = grid.size();
+    const double at = (q + half - grid[0]) / step;
+    size_t lo = at > 0.0 ? (at < (double)n ? (size_t)at : n) : 0;
+    while (lo > 0 && grid[lo - 1] - q >= half) --lo;
+    while (lo < n && !(grid[lo] - q >= half)) ++lo;
+    return lo < n ? (int64_t)lo - 1 : previous;
 }
 
 Slices autoslice(const double* q, uint32_t n, double zmin, double zperiod, double min_thickness)

@@ -38,25 +38,40 @@ Domain make_domain(int nx, int ny, double xperiod, double yperiod, double xmin, 
                    double voltage);
 
 // Row-wise membership of a disk-like pixel set in FFT order: for row i the
-// kept columns are [0, a_i) U [ny - b_i, ny).  Built by testing every pixel
-// with the caller's predicate; ok == false if a row is not of that form.
+// kept columns are [0, a_i) U [ny - b_i, ny); ok == false if a set is not of
+// that form.
 struct RowRanges {
     std::vector<int32_t> ab; // 2*nx: a_i, b_i
     int amax = 0, bmax = 0;  // union over rows
     bool ok = true;
 };
+// keep(i, j) holds from j = 0 up to some j and from some j on to ny - 1 when
+// it tests a rounded sum that grows with |k_y|: k_y rises over [0, ny/2) and
+// -k_y falls over [ny/2, ny), and IEEE rounding is monotone.  A bisection of
+// each half then finds the same ranges as a test of every pixel.
 template <typename Pred> RowRanges row_ranges(int nx, int ny, Pred keep)
 {
     RowRanges r;
     r.ab.assign(2 * (size_t)nx, 0);
+    const int h = ny / 2;
     for (int i = 0; i < nx; ++i) {
-        int a = 0;
-        while (a < ny && keep(i, a)) ++a;
-        int b = 0;
-        if (a < ny)
-            while (b < ny - a && keep(i, ny - 1 - b)) ++b;
-        for (int j = a; j < ny - b; ++j)
-            if (keep(i, j)) r.ok = false;
+        int a = 0, end = h; // first j of the low half that is not kept
+        while (a < end) {
+            const int m = a + (end - a) / 2;
+            if (keep(i, m)) a = m + 1;
+            else end = m;
+        }
+        int lo = h, hi = ny; // first j of the high half that is kept
+        while (lo < hi) {
+            const int m = lo + (hi - lo) / 2;
+            if (keep(i, m)) hi = m;
+            else lo = m + 1;
+        }
+        int b = ny - lo;
+        if (a == h && lo == h) { // the whole row
+            a = ny;
+            b = 0;
+        }
         r.ab[2 * i] = a;
         r.ab[2 * i + 1] = b;
         if (a > r.amax) r.amax = a;

@@ -28,19 +28,29 @@
 
 namespace msf_impl {
 
-// A device allocation owned by the library (hipMalloc / hipFree).
+// A device allocation owned by the library (hipMalloc / hipFree), or a view
+// into another one that outlives it.
 struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
+    bool owned = true;
     DevBuf() = default;
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
     ~DevBuf() { release(); }
     void release()
     {
-        if (p) (void)hipFree(p);
+        if (p && owned) (void)hipFree(p);
         p = nullptr;
         bytes = 0;
+        owned = true;
+    }
+    void view(void* q, size_t n)
+    {
+        release();
+        p = q;
+        bytes = n;
+        owned = false;
     }
     hipError_t alloc(size_t n)
     {
@@ -268,6 +278,7 @@ struct msf_specimen {
     int n_slices = 0;
     std::vector<double> lower, thick;
     std::vector<uint32_t> counts;
+    msf_impl::DevBuf tables; // the small tables below, one allocation
     msf_impl::DevBuf t32;  // [S][nx][ny] float2, t / sqrtNxNy, rows in the pair layout (pair_pos)
     msf_impl::DevBuf t64;  // [S][nx][ny] double2, t as built
     msf_impl::DevBuf px;   // [S][nx] float2
