@@ -153,15 +153,9 @@ hipError_t launch_fem_stats(const double* partial, int groups, int batch, int nb
 hipError_t launch_group_sums_f64(const double2* psi, int64_t plane, const int32_t* offsets,
                                  const int32_t* pixels, const int32_t* kind, int groups,
                                  int count, double* out, hipStream_t s);
-// detector MTF steps: |psi| outside the aperture from the compact FP32 planes
-// into full FP64 planes; the same in place on full FP64 planes; / s with the
-// band limit back into compact FP32 planes; a /= d
-hipError_t launch_mtf_magnitude(const float2* psi, int nx, int ny, int ncp, int ka, int kb,
-                                const uint8_t* outside, int batch, double2* out, hipStream_t s);
+// |psi| outside the aperture of full FP64 planes in place; a /= d
 hipError_t launch_mtf_magnitude_f64(double2* a, int64_t m, int count, const uint8_t* outside,
                                     hipStream_t s);
-hipError_t launch_mtf_compact(const double2* full, int nx, int ny, int ncp, int ka, int kb,
-                              const int2* keep, double s, int batch, float2* psi, hipStream_t st);
 hipError_t launch_div_f64(double2* a, int64_t n, double d, hipStream_t s);
 // correlograph sums of c and c^2 per (ring, phi sector) over a batch; with
 // `each`, also c of every position of the batch ([b][ii + jj * nbins])
@@ -224,6 +218,18 @@ hipError_t launch_vacuum_step(double2* a, int nx, int ny, const double2* px, con
 // FP64 transmission update of `count` real-space waves by one slice's t
 hipError_t launch_transmit_f64(double2* a, const double2* t, int64_t m, int count, int mode,
                                double s, hipStream_t st);
+// The detector MTF on a batch of compact FP32 exit waves in place
+// (adfstem.cpp:2272-2385).
+struct MtfArgs {
+    float2* psi;             // [batch][nx][ncp]
+    double2* work;           // [batch][nx][ld], ld = col_stride64(ka + kb, ny)
+    const double2* mtf;      // [nx][ny] 2-D MTF
+    const uint8_t* outside;  // [nx][ny] 1 outside the aperture
+    const int2* keep;        // band limit per row
+    int nx, ny, ncp, ka, kb, ld, batch;
+    double s;                // sqrt(nx ny)
+};
+hipError_t launch_mtf(const MtfArgs& a, const double2* twx, const double2* twy, hipStream_t s);
 // row stride of an FP64 array of nc <= ny columns: an odd number of 128-byte
 // lines where that fits in ny columns (fft64_passes.hpp)
 int col_stride64(int nc, int ny);

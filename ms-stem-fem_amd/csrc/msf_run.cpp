@@ -558,7 +558,8 @@ int64_t chain_bytes_per_position(const RunPlan& pl, const RunFlags& f)
 {
     int64_t b = f.plane * (int64_t)sizeof(float2) + (int64_t)pl.G * 8 +
                 (int64_t)std::max(pl.n_tiles, 1) * 64 * 8;
-    if (f.want_mtf) b += f.M * (int64_t)sizeof(double2);
+    if (f.want_mtf)
+        b += (int64_t)f.nx * msf::col_stride64(f.ka + f.kb, f.ny) * (int64_t)sizeof(double2);
     return b;
 }
 
@@ -695,7 +696,8 @@ int prepare_buffers(msf_ctx* c, Mem& m, RunPlan& pl, const RunFlags& f, const Sh
                                     &v.segp[k]))
             return r;
         if (f.want_mtf)
-            if (int r = take_as<double2>(c, m, pl.mtf_full_b[k], (size_t)B * f.M, &v.mtf_full[k]))
+            if (int r = take_as<double2>(c, m, pl.mtf_full_b[k], (size_t)B * f.nx * msf::col_stride64(f.ka + f.kb, f.ny),
+                                         &v.mtf_full[k]))
                 return r;
     }
     if (int r = take_as<double>(c, m, pl.adf_b, (size_t)P, &v.adf)) return r;
@@ -800,7 +802,7 @@ int enqueue_batch_tail(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, co
 {
     const msf::Domain& d = sp->dom;
     const int nx = f.nx, ny = f.ny, ka = f.ka, kb = f.kb, ncp = f.ncp;
-    const int64_t M = f.M, plane = f.plane;
+    const int64_t plane = f.plane;
     const int G = pl.G, nbins = pl.nbins, nphi = f.nphi;
     float2* bpsi = v.psi[ch];
     double* bpart = v.part[ch];
@@ -815,7 +817,8 @@ int enqueue_batch_tail(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, co
                                                   pl.grp_large, (int)pl.large_ids.size(), G, nb,
                                                   bpart, adf, s);
     };
-    if (f.want_adf || f.want_fem) { // exit waves alone need no sums
+    // exit waves alone need no sums, and FEM rings come after the MTF
+    if (f.want_adf || (f.want_fem && !f.want_mtf)) {
         HIPCHK(c, prof.begin(K_RED));
         HIPCHK(c, sums(f.want_adf ? v.adf + b0 : nullptr));
         HIPCHK(c, prof.end());
@@ -824,13 +827,21 @@ int enqueue_batch_tail(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, co
         // adfstem.cpp:2272-2385 after the ADF sum: |psi| outside the
         // aperture, BACKWARD FFT, x MTF / s (in-place update), FORWARD
         // FFT, / s, bw_limit; then the group sums again for the FEM
-        double2* full = v.mtf_full[ch];
-        HIPCHK(c, msf::launch_mtf_magnitude(bpsi, nx, ny, ncp, ka, kb, pl.mtf_out, nb, full, s));
-        HIPCHK(c, msf::fft2d_f64(full, nx, ny, nb, true, v.twx.f64, v.twy.f64, s));
-        HIPCHK(c, msf::launch_transmit_f64(full, pl.mtf2d, M, nb, 0, d.sqrt_nxny, s));
-        HIPCHK(c, msf::fft2d_f64(full, nx, ny, nb, false, v.twx.f64, v.twy.f64, s));
-        HIPCHK(c, msf::launch_mtf_compact(full, nx, ny, ncp, ka, kb, sp->dkeep.as<int2>(),
-                                          d.sqrt_nxny, nb, bpsi, s));
+        msf::MtfArgs ma{};
+        ma.psi = bpsi;
+        ma.work = v.mtf_full[ch];
+        ma.mtf = pl.mtf2d;
+        ma.outside = pl.mtf_out;
+        ma.keep = sp->dkeep.as<int2>();
+        ma.nx = nx;
+        ma.ny = ny;
+        ma.ncp = ncp;
+        ma.ka = ka;
+        ma.kb = kb;
+        ma.ld = msf::col_stride64(ka + kb, ny);
+        ma.batch = nb;
+        ma.s = d.sqrt_nxny;
+        HIPCHK(c, msf::launch_mtf(ma, v.twx.f64, v.twy.f64, s));
         HIPCHK(c, sums(nullptr));
     }
     // the FEM accumulators are shared: batch k updates them after batch k-1
