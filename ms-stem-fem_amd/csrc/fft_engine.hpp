@@ -218,15 +218,24 @@ template <bool INV, typename C> struct Dft<16, INV, C> {
 // one padding slot every 8 elements breaks the power-of-two strides of the
 // Stockham write pattern across LDS banks
 // (PS: one padding slot every 2^PS elements; 3 unless a kernel asks for a
-// sparser padding to fit more rows in LDS)
-template <int PS = 3> __host__ __device__ constexpr int lds_pad(int e) { return e + (e >> PS); }
+// sparser padding to fit more rows in LDS; PS < 0: elements -PS slots apart,
+// a column of an LDS plane whose rows are -PS slots long, shifted by one slot
+// every 8 rows)
+template <int PS = 3> __host__ __device__ constexpr int lds_pad(int e)
+{
+    if constexpr (PS < 0) return e * -PS + (e >> 3);
+    else return e + (e >> PS);
+}
 template <int PS = 3> __host__ __device__ constexpr int lds_len(int n) { return n + (n >> PS) + 1; }
 // lds_pad(r + S * p) for r >= 0: with S a multiple of 2^PS the padding of
 // the p-th element is (r >> PS) + p S / 2^PS, so the address is one per-lane
 // base plus a constant per p (an immediate offset, no address register per p)
 template <int S, int PS = 3> __device__ __forceinline__ int lds_pad_at(int r, int p)
 {
-    if constexpr (S % (1 << PS) == 0) {
+    if constexpr (PS < 0) {
+        if constexpr (S % 8 == 0) return lds_pad<PS>(r) + p * (S * -PS + S / 8);
+        else return lds_pad<PS>(r + S * p);
+    } else if constexpr (S % (1 << (PS < 0 ? 0 : PS)) == 0) {
         return (r + (r >> PS)) + p * (S + (S >> PS));
     } else {
         return lds_pad<PS>(r + S * p);
@@ -332,7 +341,7 @@ __device__ __forceinline__ void fft_stage(C (&x)[E], C* lds, const C* tw, int t)
         // plus constant offsets (fewer address registers: the 1024 column
         // pass 177 -> 120 registers); the 8-value plans measure faster with
         // an address per element (512 column pass 39.6 -> 37.1 us).
-        constexpr bool FOLD = E >= 16;
+        constexpr bool FOLD = E >= 16 || PS < 0;
 #pragma unroll
         for (int m = 0; m < BPT; ++m) {
             const int j = t + T * m;

@@ -75,6 +75,19 @@ bool fused_supported(int n, const RowPassArgs& ra, const ColPassArgs& ca);
 // column tile `tile` (0: the plan's default)
 bool fused_shape_ok(int n, int vr, int vc, int tile);
 
+// The whole slice loop of a batch in one launch, one workgroup per position
+// (kernels_loop.hip): both passes' arguments at slice 0, `slices` of them.
+// Results equal the passes' bit for bit.
+struct LoopArgs {
+    RowPassArgs row;
+    ColPassArgs col;
+    int slices;
+};
+// true when the grid has such a launch for these arguments and it is the
+// faster way for their batch
+bool loop_supported(int nx, int ny, const RowPassArgs& r, const ColPassArgs& c);
+hipError_t launch_slice_loop(int nx, int ny, int tmode, const LoopArgs& a, hipStream_t s);
+
 // Grouped launches: one launch runs the same pass over the batches of up to
 // kGroupMax runs of one transform length (each its own specimen, vacuum
 // waves, kept columns and buffers).  Entry k owns launch blocks

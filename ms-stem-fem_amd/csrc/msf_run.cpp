@@ -884,6 +884,12 @@ int enqueue_job(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, const Run
     };
     // the slice loop of one batch alone
     auto slices_alone = [&](msf::RowPassArgs& r, msf::ColPassArgs& cc, hipStream_t s) -> int {
+        if (!prof.on && msf::loop_supported(nx, ny, r, cc)) { // one launch, waves in LDS
+            row_at(r, 0);
+            col_at(cc, 0);
+            HIPCHK(c, msf::launch_slice_loop(nx, ny, f.tmode, msf::LoopArgs{r, cc, S}, s));
+            return MSF_OK;
+        }
         for (int n = 0; n < S; ++n) {
             row_at(r, n);
             HIPCHK(c, prof.kernel(n == 0 ? K_ROW0 : K_ROW));

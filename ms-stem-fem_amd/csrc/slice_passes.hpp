@@ -39,6 +39,21 @@ template <typename T> __device__ __forceinline__ T& elem32(T* base, uint32_t k)
 //   a  = t're u_re - ti u_im,            b  = t're u_im + ti a
 //   Da = tau u0_re - ti u0_im,           Db = tau u0_im + ti (u0_re/s + Da)
 // and TMODE 1 (exact product) uses b = t're u_im + ti u_re, Db = tau u0_im + ti u0_re.
+template <bool FIRST, int TMODE>
+__device__ __forceinline__ float2 transmit_point(float2 u, float2 tv, float2 u0, float is)
+{
+    const float da = tv.x * u0.x - tv.y * u0.y;
+    const float db = (TMODE == 0) ? tv.x * u0.y + tv.y * (u0.x * is + da) : tv.x * u0.y + tv.y * u0.x;
+    if constexpr (FIRST) {
+        return float2{da, db};
+    } else {
+        const float tr = tv.x + is;
+        const float re = tr * u.x - tv.y * u.y;
+        const float im = (TMODE == 0) ? tr * u.y + tv.y * re : tr * u.y + tv.y * u.x;
+        return float2{re + da, im + db};
+    }
+}
+
 // Lane element p (indices t + T*p) lies entirely inside the middle band
 // [3N/8, 5N/8), which the 2/3 band limit leaves empty in k-space (checked on
 // the host before a pruned variant is launched).
@@ -228,17 +243,7 @@ __device__ __forceinline__ void row_body(const RowPassArgs& a, int blk, float2* 
 
     const float is = a.inv_s;
     auto transmit = [&](int p, float2 tv, float2 u0) {
-        const float da = tv.x * u0.x - tv.y * u0.y;
-        const float db = (TMODE == 0) ? tv.x * u0.y + tv.y * (u0.x * is + da) : tv.x * u0.y + tv.y * u0.x;
-        if constexpr (FIRST) {
-            x[p] = float2{da, db};
-        } else {
-            const float tr = tv.x + is;
-            const float2 u = x[p];
-            const float re = tr * u.x - tv.y * u.y;
-            const float im = (TMODE == 0) ? tr * u.y + tv.y * re : tr * u.y + tv.y * u.x;
-            x[p] = float2{re + da, im + db};
-        }
+        x[p] = transmit_point<FIRST, TMODE>(x[p], tv, u0, is);
     };
     if constexpr (row_reads_ahead<NY, V>()) {
         // all reads issued before the first product: more of them in flight,
@@ -365,6 +370,21 @@ template <int NX, int V, int W> __host__ __device__ constexpr bool col_fits()
     return (size_t)W * col_len<NX, V, W>() * 8 + tables <= 160 * 1024 && W * P::T <= 1024;
 }
 
+// band limit and propagator P_x[i] * P_y[j] (which carries 1/sqrtNxNy) of one pixel
+__device__ __forceinline__ float2 propagate_point(float2 f, float2 pxi, float2 pyj, bool keep)
+{
+    const float2 pr = float2{pxi.x * pyj.x - pxi.y * pyj.y, pxi.x * pyj.y + pxi.y * pyj.x};
+    return keep ? float2{pr.x * f.x - pr.y * f.y, pr.x * f.y + pr.y * f.x} : float2{0.f, 0.f};
+}
+// the vacuum exit wave, shifted: psi0(k) e^{-2 pi i (i sx / nx + j sy / ny)}
+__device__ __forceinline__ float2 add_vacuum(float2 x, float2 v0, float2 wx, float2 wy)
+{
+    const float2 w = float2{wx.x * wy.x - wx.y * wy.y, wx.x * wy.y + wx.y * wy.x};
+    x.x += v0.x * w.x - v0.y * w.y;
+    x.y += v0.x * w.y + v0.y * w.x;
+    return x;
+}
+
 // One column-pass workgroup: logical block `blk` of `nblk` (XCD-banded over
 // the pass's own blocks), LDS at smem.
 template <int NX, int V, bool LAST, int W, bool PRUNE>
@@ -448,16 +468,12 @@ __device__ __forceinline__ void col_body(const ColPassArgs& a, int blk, int nblk
         }
         const int i = t + T * p;
         const bool keep = (i < ck.x) || (i >= NX - ck.y);
-        const float2 pxi = tpx[i];
-        const float2 pr = float2{pxi.x * pyj.x - pxi.y * pyj.y, pxi.x * pyj.y + pxi.y * pyj.x};
-        const float2 f = x[p];
-        x[p] = keep ? float2{pr.x * f.x - pr.y * f.y, pr.x * f.y + pr.y * f.x} : float2{0.f, 0.f};
+        x[p] = propagate_point(x[p], tpx[i], pyj, keep);
     }
 
     if constexpr (!LAST) {
         P::template run<true, float2, WAVE, PS>(x, lds, tw, t);
     } else if (active) {
-        // add the vacuum exit wave, shifted: psi0(k) e^{-2 pi i (i sx / nx + j sy / ny)}
         const int2 sh = a.shift[b];
         const float2 wy = a.twy[((uint32_t)j * (uint32_t)sh.y) % (uint32_t)a.ny];
 #pragma unroll
@@ -465,10 +481,7 @@ __device__ __forceinline__ void col_body(const ColPassArgs& a, int blk, int nblk
             if (PRUNE && in_zero_band<NX, E>(p)) continue;
             const uint32_t i = (uint32_t)(t + T * p);
             const float2 wx = s_nat[(i * (uint32_t)sh.x) % (uint32_t)NX];
-            const float2 w = float2{wx.x * wy.x - wx.y * wy.y, wx.x * wy.y + wx.y * wy.x};
-            const float2 v0 = a.psi0[(int64_t)j * NX + i];
-            x[p].x += v0.x * w.x - v0.y * w.y;
-            x[p].y += v0.x * w.y + v0.y * w.x;
+            x[p] = add_vacuum(x[p], a.psi0[(int64_t)j * NX + i], wx, wy);
         }
     }
 
