@@ -179,10 +179,6 @@ hipError_t launch_fem_correlograph(const double* partial, int groups, int batch,
 // per-pixel FP64 sums of |psi| and |psi|^2 over the positions of a batch
 hipError_t launch_pixel_moments(const float2* psi, int64_t plane, int batch, double* s1,
                                 double* s2, hipStream_t s);
-// compact exit wave -> full reference layout (FP32)
-hipError_t launch_expand_exit(const float2* psi, int nx, int ny, int ncp, int ka, int kb,
-                              int batch, float2* out, hipStream_t s);
-
 // ---------------------------------------------------------------- FP64 set-up
 bool setup_lengths_ok(int n);
 // in-place 2-D FFT of `count` planes of nx x ny complex doubles (twx, twy:

@@ -802,27 +802,4 @@ hipError_t launch_pixel_moments(const float2* psi, int64_t plane, int batch, dou
     return hipGetLastError();
 }
 
-__global__ void expand_exit_kernel(const float2* psi, int nx, int ny, int ncp, int ka, int kb,
-                                   int batch, float2* out)
-{
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t total = (int64_t)batch * nx * ny;
-    if (idx >= total) return;
-    const int j = (int)(idx % ny);
-    const int64_t r = idx / ny; // b * nx + i
-    float2 v{0.f, 0.f};
-    if (j < ka) v = psi[r * ncp + j];
-    else if (j >= ny - kb) v = psi[r * ncp + j - ny + ka + kb];
-    out[idx] = v;
-}
-
-hipError_t launch_expand_exit(const float2* psi, int nx, int ny, int ncp, int ka, int kb,
-                              int batch, float2* out, hipStream_t s)
-{
-    const int64_t total = (int64_t)batch * nx * ny;
-    hipLaunchKernelGGL(expand_exit_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
-                       psi, nx, ny, ncp, ka, kb, batch, out);
-    return hipGetLastError();
-}
-
 } // namespace msf

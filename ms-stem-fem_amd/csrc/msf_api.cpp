@@ -46,6 +46,7 @@ int msf_create(msf_ctx** out, int device)
             delete c;
             return MSF_ERR_DEVICE;
         }
+        exit_context(1);
         *out = c;
         return MSF_OK;
     }
@@ -90,6 +91,7 @@ int msf_destroy(msf_ctx* c)
             }
             (void)hipStreamDestroy(c->stream);
         }
+        exit_context(-1);
         delete c;
         return MSF_OK;
     }

@@ -123,7 +123,7 @@ struct RunPlan {
     // work buffers of the two batch chains and the run's accumulators
     int64_t cap_b = 0;       // batch depth the chain buffers were sized for
     DevBuf psi_b[2], part_b[2], segp_b[2], mtf_full_b[2];
-    DevBuf state_b, femv_b, adf_b, shift_b, exit_b, vsum_b, pm1_b, pm2_b, csum_b, csqr_b,
+    DevBuf state_b, femv_b, adf_b, shift_b, vsum_b, pm1_b, pm2_b, csum_b, csqr_b,
         ceach_b;
     // the job's launch sequence as an instantiated HIP graph, replayed while
     // every pointer and size it was captured with is unchanged
@@ -148,7 +148,7 @@ struct RunPlan {
         drop_graph();
         valid = false;
         spec_id = 0;
-        for (DevBuf* b : {&U0, &Psi0, &vac_b, &state_b, &femv_b, &adf_b, &shift_b, &exit_b, &vsum_b,
+        for (DevBuf* b : {&U0, &Psi0, &vac_b, &state_b, &femv_b, &adf_b, &shift_b, &vsum_b,
                           &pm1_b, &pm2_b, &csum_b, &csqr_b, &ceach_b})
             b->release();
         for (int k = 0; k < 2; ++k)
@@ -428,7 +428,6 @@ struct RunViews {
     double *state = nullptr, *femv = nullptr, *adf = nullptr, *vsum = nullptr, *pm1 = nullptr,
            *pm2 = nullptr, *csum = nullptr, *csqr = nullptr, *ceach = nullptr;
     int2* shift = nullptr;
-    float2* exit = nullptr;
     Twiddles twx, twy;
 };
 
@@ -548,6 +547,13 @@ struct GroupInfo {
 int run_group(msf_ctx* c, std::vector<GroupRun>& runs, GroupInfo* info);
 // frees the work buffers of the group's run plans (pixel groups stay)
 void release_group_plans(msf_ctx* c);
+
+// ---- exit waves (msf_exit.cpp)
+// `batch` compact planes of psi, after everything queued on s, into full rows
+// of the caller's memory
+int copy_exit_waves(msf_ctx* c, const float2* psi, int nx, int ny, int ncp, int ka, int kb,
+                    int64_t batch, hipStream_t s, float* dst);
+void exit_context(int delta); // a context begins (+1) or ends (-1)
 
 // ---- serving (msf_serve.cpp)
 // Blocks until no queued or running served job refers to the specimen.

@@ -634,7 +634,9 @@ int launch_shape(msf_ctx* c, Mem& m, RunPlan& pl, const msf_specimen* sp,
     // covers >= 4M pixels (512^2: +4 % over one chain, graph or not; the
     // runtime replays a two-branch graph's branches one after the other);
     // below that one chain replayed as a graph, where launch cost matters.
-    // Profiled, exit-wave and allocation-free runs use one chain.
+    // Profiled and allocation-free runs use one chain; exit-wave runs of
+    // several batches two, so that one batch's waves are copied to the host
+    // while the other's slices run.
     if (m.scratch()) {
         // what is left of the region after the per-position and fixed buffers
         int64_t fixed = P * (int64_t)(sizeof(double) + sizeof(int2)) +
@@ -654,10 +656,11 @@ int launch_shape(msf_ctx* c, Mem& m, RunPlan& pl, const msf_specimen* sp,
     sh.B = B;
     sh.n_batches = (P + B - 1) / B;
     const bool big_launch = B * f.plane >= (4ll << 20);
-    const int chains_req = chains_cfg ? chains_cfg : (big_launch ? 2 : 1);
+    const int chains_req = out.exit ? (chains_cfg == 1 ? 1 : 2)
+                                    : (chains_cfg ? chains_cfg : (big_launch ? 2 : 1));
     // chains 3: batches in pairs on one stream, row and column passes of the
     // pair's two batches fused into one launch per step
-    sh.chains = (chains_req >= 2 && sh.n_batches >= 2 && !prof && !out.exit && !m.scratch())
+    sh.chains = (chains_req >= 2 && sh.n_batches >= 2 && !prof && !m.scratch())
                     ? chains_req
                     : 1;
     sh.auto_eager = c->cfg.chains == 0 && sh.chains == 2;
@@ -683,7 +686,6 @@ int prepare_buffers(msf_ctx* c, Mem& m, RunPlan& pl, const RunFlags& f, const Sh
         for (int k = 0; k < 2; ++k)
             for (DevBuf* b : {&pl.psi_b[k], &pl.part_b[k], &pl.segp_b[k], &pl.mtf_full_b[k]})
                 b->release();
-        pl.exit_b.release();
         pl.cap_b = B;
     }
     for (int k = 0; k < std::min(sh.chains, 2); ++k) {
@@ -717,8 +719,6 @@ int prepare_buffers(msf_ctx* c, Mem& m, RunPlan& pl, const RunFlags& f, const Sh
         if (int r = take_as<double>(c, m, pl.pm1_b, (size_t)f.plane, &v.pm1)) return r;
         if (int r = take_as<double>(c, m, pl.pm2_b, (size_t)f.plane, &v.pm2)) return r;
     }
-    if (out.exit)
-        if (int r = take_as<float2>(c, m, pl.exit_b, (size_t)B * f.M, &v.exit)) return r;
     // accumulators start at zero (outside any captured graph)
     HIPCHK(c, hipMemsetAsync(v.state, 0, nb1 * 3 * sizeof(double), c->stream));
     if (f.want_d2) HIPCHK(c, hipMemsetAsync(v.vsum, 0, nb1 * sizeof(double), c->stream));
@@ -855,12 +855,6 @@ int enqueue_batch_tail(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, co
                       s));
     if (f.want_pix) HIPCHK(c, msf::launch_pixel_moments(bpsi, plane, nb, v.pm1, v.pm2, s));
     if (chains == 2) HIPCHK(c, hipEventRecord(c->ev_fem[k % 2], s));
-    if (out.exit) {
-        HIPCHK(c, msf::launch_expand_exit(bpsi, nx, ny, ncp, ka, kb, nb, v.exit, s));
-        HIPCHK(c, hipMemcpyAsync(out.exit + (size_t)b0 * nx * ny * 2, v.exit,
-                                 (size_t)nb * nx * ny * sizeof(float2), hipMemcpyDeviceToHost,
-                                 s));
-    }
     return MSF_OK;
 }
 
@@ -959,6 +953,19 @@ int enqueue_job(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, const Run
         HIPCHK(c, hipEventRecord(c->ev_fork, c->stream));
         HIPCHK(c, hipStreamWaitEvent(c->stream2, c->ev_fork, 0));
     }
+    // exit waves of a batch to the host, after the next batch's launches are
+    // queued when there are two chains
+    struct Pending {
+        int64_t b0 = 0;
+        int nb = 0, ch = 0;
+    } last;
+    auto drain = [&]() -> int {
+        if (!out.exit || last.nb == 0) return MSF_OK;
+        const Pending b = last;
+        last.nb = 0;
+        return copy_exit_waves(c, v.psi[b.ch], nx, ny, f.ncp, f.ka, f.kb, b.nb, streams[b.ch],
+                               out.exit + (size_t)b.b0 * nx * ny * 2);
+    };
     int64_t k = 0;
     for (int64_t b0 = 0; b0 < P; b0 += B, ++k) {
         const int nb = (int)std::min<int64_t>(B, P - b0);
@@ -969,7 +976,13 @@ int enqueue_job(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, const Run
         bind(b0, nb, ch, r, cc);
         if (int e = slices_alone(r, cc, s)) return e;
         if (int e = finish_batch(k, b0, nb, ch, s)) return e;
+        if (chains == 2)
+            if (int e = drain()) return e;
+        last = {b0, nb, ch};
+        if (chains != 2)
+            if (int e = drain()) return e;
     }
+    if (int e = drain()) return e;
     if (chains == 2) { // join: the first stream waits for everything on the second
         HIPCHK(c, hipEventRecord(c->ev_join, c->stream2));
         HIPCHK(c, hipStreamWaitEvent(c->stream, c->ev_join, 0));
