@@ -112,31 +112,32 @@ template <bool INV, typename C> struct Dft<3, INV, C> {
     }
 };
 
-template <bool INV, typename C> struct Dft<6, INV, C> {
-    static __device__ __forceinline__ void run(C* v)
-    {
-        using R = decltype(v[0].x);
-        const R s3 = R(0.86602540378443864676);
-        C e[3] = {v[0], v[2], v[4]};
-        C o[3] = {v[1], v[3], v[5]};
-        Dft<3, INV, C>::run(e);
-        Dft<3, INV, C>::run(o);
-        // W6 = 1/2 -/+ i sqrt(3)/2, W6^2 = -1/2 -/+ i sqrt(3)/2 (forward/inverse)
-        C o1, o2;
-        if (!INV) {
-            o1 = C{R(0.5) * o[1].x + s3 * o[1].y, R(0.5) * o[1].y - s3 * o[1].x};
-            o2 = C{-R(0.5) * o[2].x + s3 * o[2].y, -R(0.5) * o[2].y - s3 * o[2].x};
-        } else {
-            o1 = C{R(0.5) * o[1].x - s3 * o[1].y, R(0.5) * o[1].y + s3 * o[1].x};
-            o2 = C{-R(0.5) * o[2].x - s3 * o[2].y, -R(0.5) * o[2].y + s3 * o[2].x};
-        }
-        v[0] = cadd(e[0], o[0]);
-        v[3] = csub(e[0], o[0]);
-        v[1] = cadd(e[1], o1);
-        v[4] = csub(e[1], o1);
-        v[2] = cadd(e[2], o2);
-        v[5] = csub(e[2], o2);
+// Radices 6 and 12 as 2 x 3 and 4 x 3 by the prime-factor mapping: with
+// coprime factors A and B, n = (B a + A b) mod AB and k reduced modulo each
+// factor, W_AB^(nk) = W_A^(a k) W_B^(b k), so no twiddles stand between the
+// two steps, and the index maps are register names.
+template <int A, bool INV, typename C> __device__ __forceinline__ void dft_by_3(C* v)
+{
+    C y[A][3];
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+        C u[A];
+#pragma unroll
+        for (int a = 0; a < A; ++a) u[a] = v[(3 * a + A * b) % (3 * A)];
+        Dft<A, INV, C>::run(u);
+#pragma unroll
+        for (int a = 0; a < A; ++a) y[a][b] = u[a];
     }
+#pragma unroll
+    for (int a = 0; a < A; ++a) Dft<3, INV, C>::run(y[a]);
+#pragma unroll
+    for (int k = 0; k < 3 * A; ++k) v[k] = y[k % A][k % 3];
+}
+template <bool INV, typename C> struct Dft<6, INV, C> {
+    static __device__ __forceinline__ void run(C* v) { dft_by_3<2, INV, C>(v); }
+};
+template <bool INV, typename C> struct Dft<12, INV, C> {
+    static __device__ __forceinline__ void run(C* v) { dft_by_3<4, INV, C>(v); }
 };
 
 // multiplication by W16^e = exp(-/+ 2 pi i e / 16) (forward / inverse)
@@ -261,6 +262,60 @@ template <bool WAVE> __device__ __forceinline__ void lds_sync()
     }
 }
 
+// Where a stage's outputs go in the exchange buffer: butterfly j = t + T m,
+// output q is element e = (j / NS) NS R + j % NS + q NS, in slot
+// e * STRIDE + (e / PB) * PA, and lane t then reads elements t + T p.  When
+// the padding block PB and the spans divide one another (`fold`) a slot is
+// one per-lane base plus a constant for every (m, q) or p: an exchange needs
+// one address register for the writes and one for the reads.
+//
+// PS = 0 picks the padding of each exchange for 8-byte values, which the LDS
+// serves 16 lanes at a time without conflict when their slots differ modulo
+// 16: after the first stage (NS = 1) lane strides of 4, 8 or 16 become odd
+// over 16 lanes with one slot every 16; spans of 4 and 8 need their blocks of
+// NS R elements NS slots further on, so that 16 / NS blocks tile the banks;
+// longer spans need none.  The reads, 16 consecutive elements, then meet no
+// padding inside.  One slot every 8 elements for every exchange (PS = 3) took
+// two passes per read and up to four per write, and an address register per
+// element: per 112 positions of 384^2 the row pass went from 57 to 50 us and
+// the column pass from 47 to 40 us (registers 128 -> 100 and 126 -> 75), per
+// 496 of 192^2 50 -> 46 and 46 -> 40, per 272 of 256^2 41.2 -> 40.1 and
+// 35.5 -> 35.3, per 64 of 512^2 41.4 -> 40.3 and 37.5 -> 36.5 us.
+template <int T, int BPT, int R, int NS, int PS> struct LdsExchange {
+    static constexpr int STRIDE = PS < 0 ? -PS : 1;
+    static constexpr int PB = PS < 0 ? 8 : PS > 0 ? 1 << (PS > 0 ? PS : 0) : NS == 1 ? 16 : NS * R;
+    static constexpr int PA = PS != 0 || NS == 1 ? 1 : NS >= 16 ? 0 : NS;
+    static constexpr bool A = NS % PB == 0;                        // blocks within a span
+    static constexpr bool B = PB % NS == 0 && (NS * R) % PB == 0;  // spans within a block
+    static constexpr bool D = PB % (NS * R) == 0;                  // a butterfly within a block
+    static constexpr bool low = T % NS == 0 && (BPT == 1 || (T * R) % PB == 0) && (A || B || D);
+    static constexpr bool high = !low && NS % T == 0 && A && T % PB == 0;
+    static constexpr bool reads = PA == 0 || T % PB == 0 || PB % T == 0;
+    static constexpr bool fold = (low || high || PA == 0) && reads;
+    static __host__ __device__ constexpr int at(int e) { return e * STRIDE + (e / PB) * PA; }
+    static __device__ __forceinline__ int write_base(int t)
+    {
+        if constexpr (high) return t * STRIDE + (t / PB) * PA;
+        const int blk = t / NS, r = t % NS;
+        if constexpr (PA == 0) return (blk * NS * R + r) * STRIDE;
+        const int pad = A ? blk * (NS * R / PB) + r / PB : B ? blk * (NS * R / PB) : (blk * NS * R) / PB;
+        return (blk * NS * R + r) * STRIDE + pad * PA;
+    }
+    static __device__ __forceinline__ constexpr int write_off(int m, int q)
+    {
+        if constexpr (high) {
+            const int blk = (T * m) / NS, rm = (T * m) % NS;
+            return (blk * NS * R + rm + q * NS) * STRIDE + (blk * NS * R / PB + rm / PB + q * NS / PB) * PA;
+        }
+        return (m * T * R + q * NS) * STRIDE + ((m * T * R) / PB + (D && !A && !B ? 0 : (q * NS) / PB)) * PA;
+    }
+    static __device__ __forceinline__ int read_base(int t)
+    {
+        return t * STRIDE + (T % PB == 0 ? (t / PB) * PA : 0);
+    }
+    static __device__ __forceinline__ constexpr int read_off(int p) { return T * p * STRIDE + (T * p / PB) * PA; }
+};
+
 // ------------------------------------------------------------ one stage
 // Twiddles of stage s (radix R, span NS) come from a per-stage table laid out
 // [q-1][k], entry W_{NS R}^{q k}, q = 1..R-1, k = 0..NS-1, at offset TWO in
@@ -337,23 +392,47 @@ __device__ __forceinline__ void fft_stage(C (&x)[E], C* lds, const C* tw, int t)
             for (int q = 0; q < R; ++q) x[m + q * BPT] = y[m * R + q];
     } else {
         lds_sync<WAVE>(); // previous readers of this buffer are done
-        // Plans with 16 values per lane address the exchange as one base
-        // plus constant offsets (fewer address registers: the 1024 column
-        // pass 177 -> 120 registers); the 8-value plans measure faster with
-        // an address per element (512 column pass 39.6 -> 37.1 us).
-        constexpr bool FOLD = E >= 16 || PS < 0;
+        using X = LdsExchange<T, BPT, R, NS, PS>;
+        // (the 8-value FP64 transforms, padded alike in every exchange, keep
+        // an address per element)
+        static_assert(PS != 0 || X::fold, "per-exchange padding without constant offsets");
+        constexpr bool FOLD = X::fold && (PS <= 0 || E >= 12);
+        if constexpr (FOLD) {
+            C* w = lds + X::write_base(t);
 #pragma unroll
-        for (int m = 0; m < BPT; ++m) {
-            const int j = t + T * m;
-            const int base = (j / NS) * NS * R + (j % NS);
+            for (int m = 0; m < BPT; ++m)
 #pragma unroll
-            for (int q = 0; q < R; ++q)
-                lds[FOLD ? lds_pad_at<NS, PS>(base, q) : lds_pad<PS>(base + q * NS)] = y[m * R + q];
+                for (int q = 0; q < R; ++q) w[X::write_off(m, q)] = y[m * R + q];
+        } else {
+#pragma unroll
+            for (int m = 0; m < BPT; ++m) {
+                const int j = t + T * m;
+                const int base = (j / NS) * NS * R + (j % NS);
+#pragma unroll
+                for (int q = 0; q < R; ++q) lds[lds_pad<PS>(base + q * NS)] = y[m * R + q];
+            }
         }
         lds_sync<WAVE>();
+        if constexpr (FOLD) {
+            const C* r = lds + X::read_base(t);
 #pragma unroll
-        for (int p = 0; p < E; ++p)
-            x[p] = lds[FOLD ? lds_pad_at<T, PS>(t, p) : lds_pad<PS>(t + T * p)];
+            for (int p = 0; p < E; ++p) x[p] = r[X::read_off(p)];
+        } else {
+#pragma unroll
+            for (int p = 0; p < E; ++p) x[p] = lds[lds_pad<PS>(t + T * p)];
+        }
+    }
+}
+
+// slots of a plan's exchange buffer with per-exchange padding
+template <int T, int E, int NS, int R, int... Rest> constexpr int exchange_len()
+{
+    if constexpr (sizeof...(Rest) == 0) {
+        return T * E; // the last stage exchanges nothing
+    } else {
+        constexpr int here = LdsExchange<T, E / R, R, NS, 0>::at(T * E - 1) + 1;
+        constexpr int rest = exchange_len<T, E, NS * R, Rest...>();
+        return here > rest ? here : rest;
     }
 }
 
@@ -375,6 +454,12 @@ __device__ __forceinline__ void run_stages(C (&x)[E], C* lds, const C* tw, int t
 // schedule of each length (also used by the FP64 transforms); AltPlan<N>, where
 // it exists, a second schedule of the FP32 slice passes with 16 values per lane
 // and one fewer radix stage, chosen per run (configuration or autotuner).
+// Lengths with a factor 3 take 12 values per lane and their 4s first: the
+// spans of every exchange are then powers of two, which LdsExchange folds,
+// and butterflies of a lane share their twiddles.  24 values per lane (192 =
+// 6 8 4, 768 = 6 8 4 4) needed 170 to 207 registers: 192^2 row and column
+// pass 70 / 57 us per 496 positions against 46 / 40, 768^2 48 / 40 us per 16
+// against 36 / 28.
 template <int N> struct Plan;
 template <int N> struct AltPlan { static constexpr bool exists = false; };
 #define MSF_PLAN_AS(NAME, N_, E_, ...)                                                         \
@@ -383,6 +468,7 @@ template <int N> struct AltPlan { static constexpr bool exists = false; };
         static constexpr int N = N_, E = E_, T = N_ / E_;                                      \
         static constexpr int kRadix[] = {__VA_ARGS__};                                         \
         static constexpr int kStages = sizeof(kRadix) / sizeof(int);                           \
+        static constexpr int kExchangeLen = exchange_len<T, E, 1, __VA_ARGS__>();              \
         template <bool INV, typename C, bool WAVE = false, int PS = 3>                         \
         static __device__ __forceinline__ void run(C (&x)[E_], C* lds, const C* tw, int t)     \
         {                                                                                      \
@@ -394,13 +480,13 @@ template <int N> struct AltPlan { static constexpr bool exists = false; };
 MSF_PLAN(16, 8, 8, 2)
 MSF_PLAN(32, 8, 8, 4)
 MSF_PLAN(64, 8, 8, 8)
-MSF_PLAN(96, 12, 6, 4, 4)
+MSF_PLAN(96, 12, 4, 4, 6)
 MSF_PLAN(128, 8, 8, 4, 4)
-MSF_PLAN(192, 24, 6, 8, 4)
+MSF_PLAN(192, 12, 4, 4, 12)
 MSF_PLAN(256, 8, 8, 8, 4)
-MSF_PLAN(384, 12, 6, 4, 4, 4)
+MSF_PLAN(384, 12, 4, 4, 4, 6)
 MSF_PLAN(512, 8, 8, 8, 8)
-MSF_PLAN(768, 24, 6, 8, 4, 4)
+MSF_PLAN(768, 12, 4, 4, 4, 12)
 MSF_PLAN(1024, 8, 8, 8, 4, 4)
 MSF_ALT_PLAN(256, 16, 16, 16)
 MSF_ALT_PLAN(512, 16, 16, 8, 4)

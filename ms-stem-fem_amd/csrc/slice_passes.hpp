@@ -138,13 +138,13 @@ template <int NY, int V, int RT> __host__ __device__ constexpr bool row_is_lean(
     // one row per workgroup: nothing to share, tables are read from L2
     return row_lean<NY, V>() || RT / PlanV<NY, V>::T == 1;
 }
-// padding of a row's exchange buffer: one slot every 2^row_pad_shift values.
-// The alternate 1024 row pass pads every 32 (8.3 KB per row instead of
-// 9.2 KB): its pass takes as long, but the smaller workgroups leave room for
-// the other batch chain's column pass on the same CUs (1024^2 job +3 %).
-template <int NY, int V> __host__ __device__ constexpr int row_pad_shift()
+// slots of one row's exchange buffer (padded per exchange, LdsExchange); for
+// transforms of 8 lanes the two rows that 16 lanes cover start 8 slots apart
+// modulo 16
+template <int NY, int V> __host__ __device__ constexpr int row_len()
 {
-    return (NY == 1024 && V == 1) ? 5 : 3;
+    using P = PlanV<NY, V>;
+    return P::T >= 16 ? P::kExchangeLen : (P::kExchangeLen + 7) / 16 * 16 + 8;
 }
 // Row passes that read every transmission and u0 pair of a lane before the
 // first product (the alternate 1024 plan: row pass 57.5 -> 53.4 us; the
@@ -159,7 +159,7 @@ template <int NY, int V> __host__ __device__ constexpr bool row_reads_ahead()
 template <int NY, int V, int RT> __host__ __device__ constexpr int row_smem_len()
 {
     return (row_is_lean<NY, V, RT>() ? 0 : plan_tw_len<PlanV<NY, V>>() + NY) +
-           (RT / PlanV<NY, V>::T) * lds_len<row_pad_shift<NY, V>()>(NY);
+           (RT / PlanV<NY, V>::T) * row_len<NY, V>();
 }
 
 // One row-pass workgroup: logical block `blk` of the pass (XCD-banded over
@@ -170,8 +170,7 @@ __device__ __forceinline__ void row_body(const RowPassArgs& a, int blk, float2* 
     using P = PlanV<NY, V>;
     constexpr int E = P::E, T = P::T;
     constexpr int RPW = RT / T;
-    constexpr int PS = row_pad_shift<NY, V>();
-    constexpr int LEN = lds_len<PS>(NY);
+    constexpr int PS = 0, LEN = row_len<NY, V>();
     constexpr bool LEAN = row_is_lean<NY, V, RT>();
     float2* s_tw = smem;
     float2* s_t = smem + (LEAN ? 0 : plan_tw_len<P>());
@@ -310,23 +309,12 @@ template <int NX, int V = 0> struct ColTile {
     static constexpr int W = (NX == 1024 && V == 1) ? 4 : (16 * lds_len(NX) * 8 > 48 * 1024) ? 8 : 16;
 };
 
-// padding of a column in the tile: one slot every 2^col_pad_shift values.
-// The alternate 1024 column pass pads every 16 (a 4-column tile of 34.9 KB
-// instead of 37 KB): the pass 45.5 -> 44.0 us and the 1024^2 job +3-4 %
-// (every 32: +2 %), the smaller tiles sharing CUs with the other batch
-// chain's row pass; the primary 512 column pass likewise (the 512^2 job
-// +1.3 %; every 32: no better), and the alternate 256 one (its pass
-// 40.3-42.4 -> 39.0-39.5 us per 256 positions).
-template <int NX, int V> __host__ __device__ constexpr int col_pad_shift()
-{
-    return ((NX == 1024 && V == 1) || (NX == 512 && V == 0) || (NX == 256 && V == 1)) ? 4 : 3;
-}
 // column stride of the LDS tile: a 16-lane group of the coalesced load/store
 // phases covers W' = min(W, 16) columns x 16/W' rows; a stride congruent to
 // 16/W' modulo 16 (8-byte words) puts those 16 lanes on distinct bank pairs
 template <int NX, int V, int W> __host__ __device__ constexpr int col_len()
 {
-    constexpr int base = lds_len<col_pad_shift<NX, V>()>(NX);
+    constexpr int base = PlanV<NX, V>::kExchangeLen;
     constexpr int want = (16 / (W < 16 ? W : 16)) % 16;
     return base + ((want - base % 16) + 16) % 16;
 }
@@ -393,7 +381,8 @@ __device__ __forceinline__ void col_body(const ColPassArgs& a, int blk, int nblk
     using P = PlanV<NX, V>;
     constexpr int E = P::E, T = P::T;
     constexpr int LEN = col_len<NX, V, W>();
-    constexpr int PS = col_pad_shift<NX, V>();
+    constexpr int PS = 0;  // exchanges padded each its own way,
+    constexpr int SP = 4;  // the tile's loads and stores one slot every 16 rows
     constexpr bool LEAN = col_lean<NX, V, W>();
     // a column transform lies in one wavefront (wave-local exchanges) or
     // spans whole wavefronts (workgroup barriers)
@@ -438,7 +427,7 @@ __device__ __forceinline__ void col_body(const ColPassArgs& a, int blk, int nblk
         for (int p = 0; p < E; ++p) v[p] = elem32(tile, o0 + (uint32_t)p * step);
 #pragma unroll
         for (int p = 0; p < E; ++p)
-            s_buf[c * LEN + lds_pad_at<T, PS>(r0, p)] = ok ? v[p] : float2{0.f, 0.f};
+            s_buf[c * LEN + lds_pad_at<T, SP>(r0, p)] = ok ? v[p] : float2{0.f, 0.f};
     }
     __syncthreads();
 
@@ -450,7 +439,7 @@ __device__ __forceinline__ void col_body(const ColPassArgs& a, int blk, int nblk
     float2* lds = s_buf + c * LEN;
     float2 x[E];
 #pragma unroll
-    for (int p = 0; p < E; ++p) x[p] = lds[lds_pad_at<T, PS>(t, p)];
+    for (int p = 0; p < E; ++p) x[p] = lds[lds_pad_at<T, SP>(t, p)];
 
     P::template run<false, float2, WAVE, PS>(x, lds, tw, t);
 
@@ -487,7 +476,7 @@ __device__ __forceinline__ void col_body(const ColPassArgs& a, int blk, int nblk
 
     lds_sync<WAVE>();
 #pragma unroll
-    for (int p = 0; p < E; ++p) lds[lds_pad_at<T, PS>(t, p)] = x[p];
+    for (int p = 0; p < E; ++p) lds[lds_pad_at<T, SP>(t, p)] = x[p];
     __syncthreads();
 
     {   // coalesced store of the tile
@@ -498,7 +487,7 @@ __device__ __forceinline__ void col_body(const ColPassArgs& a, int blk, int nblk
         if (ok) {
 #pragma unroll
             for (int p = 0; p < E; ++p)
-                elem32(tile, o0 + (uint32_t)p * step) = s_buf[c2 * LEN + lds_pad_at<T, PS>(r0, p)];
+                elem32(tile, o0 + (uint32_t)p * step) = s_buf[c2 * LEN + lds_pad_at<T, SP>(r0, p)];
         }
     }
 }
