@@ -62,6 +62,7 @@ struct ColPassArgs {
     int tile;               // columns per workgroup (4, 8 or 16; 0 = default)
     int prune;              // 1: rows [3nx/8, 5nx/8) are masked for every column
     int plan;               // radix plan of length nx: 0 primary, 1 alternate (has_alt_plan)
+    int beside;             // 1: another chain of batches runs beside this one (col_tile_default)
 };
 
 // One launch with the row pass of one batch (ra) and the column pass of
@@ -123,11 +124,12 @@ bool stage_twiddles(int n, std::vector<double>& re_im, int v = 0);
 bool has_alt_plan(int n);
 // the column count of the compact wave is padded to a multiple of this
 int col_tile(int nx);
-// the column-pass tile width used when none is configured, for plan v
-int col_tile_default(int nx, int v = 0);
+// the column-pass tile width used when none is configured, for plan v, alone
+// or beside another chain of batches
+int col_tile_default(int nx, int v = 0, bool beside = false);
 // the tile used when none is configured: the default, or one column per
 // workgroup when the launch would not give every CU a workgroup
-int col_tile_auto(int nx, int v, int batch, int ncp);
+int col_tile_auto(int nx, int v, int batch, int ncp, bool beside);
 // true when the kept set leaves [3n/8, 5n/8) empty along the row (ka, kb) and
 // every row i in [3nx/8, 5nx/8) fully masked (keep ranges)
 bool row_prunable(int ny, int ka, int kb);

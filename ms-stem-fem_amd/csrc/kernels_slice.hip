@@ -147,15 +147,23 @@ int col_tile(int nx)
 // Launches of so few positions that the default tiles would leave CUs idle
 // (one position at 512^2: 44 workgroups of 8 columns for 256 CUs) take one
 // column per workgroup instead.
-int col_tile_auto(int nx, int v, int batch, int ncp)
+int col_tile_auto(int nx, int v, int batch, int ncp, bool beside)
 {
-    const int w = col_tile_default(nx, v);
+    const int w = col_tile_default(nx, v, beside);
     constexpr int64_t kCUs = 256;
     return (int64_t)batch * (ncp / std::max(w, 1)) < kCUs ? 1 : w;
 }
 
-int col_tile_default(int nx, int v)
+// The alternate 1024 plan takes 4 columns where its launches have the GPU to
+// themselves (64 positions of 1024 x 1024, 20 slices, one chain: 7.66 ms
+// against 7.81 with 8) and 8 beside the row passes of a second chain: those
+// hide what the larger tile loses in residency, and its 64-byte segments
+// leave them more of the memory (two chains: 1024 x 1024, 50 slices, 256
+// positions 72.7 -> 69.9 ms; 1024 x 512 13.4 -> 12.7, 1024 x 768 11.6 -> 11.0;
+// 1024 x 128 and 1024 x 256 within 2 % either way).
+int col_tile_default(int nx, int v, bool beside)
 {
+    if (nx == 1024 && v == 1 && beside) return 8;
     switch (nx) {
 #define MSF_CASE(N) case N: return v ? ColTile<N, 1>::W : ColTile<N>::W;
         MSF_CASE(16) MSF_CASE(32) MSF_CASE(64) MSF_CASE(96) MSF_CASE(128) MSF_CASE(192)
@@ -258,7 +266,7 @@ template <int NX, int V>
 static hipError_t col_pass_nv(bool last, const ColPassArgs& a, hipStream_t s, hipEvent_t ev0,
                               hipEvent_t ev1)
 {
-    int w = col_tile_auto(NX, V, a.batch, a.ncp);
+    int w = col_tile_auto(NX, V, a.batch, a.ncp, a.beside != 0);
     if (a.tile == 4 || a.tile == 8 || a.tile == 16) w = a.tile;
     if (w == 1) return col_pass_w<NX, V, 1>(last, a, s, ev0, ev1);
     if constexpr (col_fits<NX, V, 16>()) {

@@ -763,6 +763,7 @@ PassArgs pass_args(const RunPlan& pl, const msf_specimen* sp, const RunFlags& f,
     ca.twx_nat = v.twx.nat;
     ca.twy = v.twy.nat;
     ca.tile = sh.col_tile;
+    ca.beside = sh.chains == 2 ? 1 : 0;
     ca.prune = msf::col_prunable(f.nx, sp->keep.ab.data()) ? 1 : 0;
     p.t32 = sp->t32.as<float2>();
     p.px = sp->px.as<float2>();
@@ -1042,8 +1043,8 @@ int tune_shape(msf_ctx* c, RunPlan& pl, const msf_specimen* sp, const std::vecto
         << " " << (f.want_adf ? "a" : "") << (f.want_d1 ? "v" : "") << (f.want_d2 ? "b" : "")
         << (f.want_pix ? "p" : "") << (f.want_corr ? "c" : "") << (f.want_mtf ? "m" : "") << "-"
         << " " << (plans ? "plans" : "plan" + std::to_string(plan_rule));
-    const int tile0 = msf::col_tile_default(f.nx, plan_rule & 1);
     const int ch0 = (B * f.plane >= (4ll << 20) && (P + B - 1) / B >= 2) ? 2 : 1;
+    const int tile0 = msf::col_tile_default(f.nx, plan_rule & 1, ch0 == 2);
     const TunedShape rule = {(int)B, tile0, ch0, plan_rule};
     std::vector<int64_t> bs = {B};
     for (int64_t b : {B / 2, 2 * B}) {
@@ -1229,7 +1230,8 @@ int run_internal(msf_ctx* c, Mem& m, const msf_specimen* sp, const msf_optics* o
     st.chains = sh.chains;
     st.fused_launches = prof.fused;
     st.col_tile = sh.col_tile ? sh.col_tile
-                              : msf::col_tile_auto(f.nx, sh.plan_v & 1, (int)sh.B, f.ncp);
+                              : msf::col_tile_auto(f.nx, sh.plan_v & 1, (int)sh.B, f.ncp,
+                                                   sh.chains == 2);
     st.autotuned = sh.tuned_state;
     st.row_fft_plan = 1 + ((sh.plan_v >> 1) & 1);
     st.col_fft_plan = 1 + (sh.plan_v & 1);

@@ -46,3 +46,26 @@ def test_length_on_either_axis(msf, ctx, O, n, plan):
         finally:
             ctx.configure()
             spec.free()
+
+
+@pytest.mark.parametrize("plan", [1, 2])
+@pytest.mark.parametrize("batch", [6, 8])
+def test_two_chains_of_1024_rows_take_the_bits_of_one(msf, ctx, plan, batch):
+    # batches whose tiles fill the CUs, and a last one of fewer positions that does not
+    nx, ny = 1024, 512
+    cell = (nx * 0.09, ny * 0.09, 6.0)
+    q, Z = random_atoms(18, cell, seed=nx + plan, species=(14, 29))
+    q[:, 2] = 2.0 * (np.arange(18) // 6) + 0.1
+    c = Case(nx=nx, ny=ny, cell=cell, voltage=200e3, q=q, Z=Z, min_slice=1.0, cs3=1.2e7,
+             defocus=300.0, alpha_max=0.03, adf=True, fem=False)
+    xp, yp = np.linspace(0.1, 0.9, 13) * cell[0], np.array([0.3]) * cell[1]
+    spec, out = c.gpu_specimen(msf, ctx), []
+    try:
+        for chains in (1, 2):
+            ctx.configure(autotune=-1, fft_plan=plan, batch=batch, chains=chains)
+            out.append(ctx.adfstem(spec, c.optics(msf), xp, yp, detector=c.detector(msf)))
+            assert ctx.stats()["chains"] == chains
+    finally:
+        ctx.configure()
+        spec.free()
+    np.testing.assert_array_equal(out[0][0], out[1][0])
