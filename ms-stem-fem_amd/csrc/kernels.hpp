@@ -35,8 +35,7 @@ __host__ __device__ inline int pair_pos(int j, int n)
 
 struct RowPassArgs {
     float2* psi;            // [B][nx][ncp] scattered wave phi
-    const float2* t;        // [nx][ny] (t_re/s - 1/s, t_im/s) of this slice, rows in the
-                            // pair layout
+    const float2* t;        // [nx][ny] t - 1 of this slice, rows in the pair layout
     const float2* u0;       // [nx][ny][2] vacuum wave entering this slice, s * real space,
                             // rows as shift pairs (pair_pos)
 
@@ -46,12 +45,13 @@ struct RowPassArgs {
     int nx, ncp, ka, kb, batch;
     int prune;              // 1: columns [3ny/8, 5ny/8) are outside the kept band
     int plan;               // radix plan of length ny: 0 primary, 1 alternate (has_alt_plan)
+    uint32_t div;           // set by the launch: div_mul of the workgroups per row
 };
 
 struct ColPassArgs {
     float2* psi;            // [B][nx][ncp]
     const float2* px;       // [nx] propagator along x of this slice
-    const float2* py;       // [ny] propagator along y of this slice, scaled by 1/s
+    const float2* py;       // [ny] propagator along y of this slice, scaled by 1/(nx ny)
     const int2* colkeep;    // [ncp] (c, d): kept rows [0, c) U [nx - d, nx) of compact column jc
     const float2* tw;       // stage twiddle table of length nx (stage_twiddles)
     const float2* psi0;     // [ny][nx] vacuum exit wave in k-space, column-major (last pass only)
@@ -63,7 +63,10 @@ struct ColPassArgs {
     int prune;              // 1: rows [3nx/8, 5nx/8) are masked for every column
     int plan;               // radix plan of length nx: 0 primary, 1 alternate (has_alt_plan)
     int beside;             // 1: another chain of batches runs beside this one (col_tile_default)
+    uint32_t div;           // set by the launch: div_mul of the tiles per position
 };
+// multiplier for a kernel's division by d (1 <= d < 2^31)
+inline uint32_t div_mul(uint32_t d) { return 0xffffffffu / d; }
 
 // One launch with the row pass of one batch (ra) and the column pass of
 // another (ca), same transform length n = nx = ny: the rows' FIRST and the
@@ -120,6 +123,12 @@ bool slice_lengths_ok(int n);
 // concatenated per-stage twiddle tables of plan v (0 primary, 1 alternate) of
 // length n, (re, im) FP64
 bool stage_twiddles(int n, std::vector<double>& re_im, int v = 0);
+// What a forward and an inverse FP32 transform of length n together multiply
+// the mean amplitude by, against the exact n: 1 but for the rounding of
+// sin 60 degrees in the radix-3 step of lengths with a factor 3.  The scale of
+// one slice is rounded the same way at every pixel and every slice, so it
+// would add up: 4.8e-8 of the intensity per slice.
+double fp32_gain(int n);
 // true when length n has an alternate radix plan for the slice passes
 bool has_alt_plan(int n);
 // the column count of the compact wave is padded to a multiple of this
@@ -212,9 +221,9 @@ struct BuildArgs {
     int n_atoms;
     const int2 *support, *bw; // per row
     const double *kx, *ky, *params /* nsp * 12 */;
-    double xmin, ymin, lgab, s /* sqrt(nx ny) */, nxny, sqrt_nxny;
+    double xmin, ymin, lgab, s /* sqrt(nx ny) */, nxny;
     double2* t64;            // [k][nx][ny] t
-    float2* t32;             // [k][nx][ny] (t_re/s - 1/s, t_im/s), rows in the pair layout
+    float2* t32;             // [k][nx][ny] t - 1, rows in the pair layout
 };
 // tmpl for every species (projected_atomic_potential.cpp:169-225)
 hipError_t launch_templates(const BuildArgs& a, hipStream_t s);

@@ -80,9 +80,10 @@ int col_group_blocks(int nx, const ColPassArgs& a)
 }
 
 template <int NY, int V>
-static hipError_t row_group_nv(bool first, int tmode, const RowGroupArgs& g, hipStream_t s)
+static hipError_t row_group_nv(bool first, int tmode, RowGroupArgs g, hipStream_t s)
 {
-    constexpr int RT = row_threads<NY, V>();
+    constexpr int RT = row_threads<NY, V>(), RPW = RT / PlanV<NY, V>::T;
+    for (int k = 0; k < g.n; ++k) g.a[k].div = div_mul((uint32_t)((g.a[k].batch + RPW - 1) / RPW));
     const dim3 grid((unsigned)g.off[g.n]), block(RT);
     const bool pr = g.a[0].prune != 0;
 #define MSF_ROWG(F, M, PR)                                                                         \
@@ -136,10 +137,13 @@ hipError_t launch_row_group(int ny, bool first, int tmode, const RowGroupArgs& g
 }
 
 template <int NX, int V, int W>
-static hipError_t col_group_w(bool last, const ColGroupArgs& g, hipStream_t s)
+static hipError_t col_group_w(bool last, ColGroupArgs g, hipStream_t s)
 {
-    for (int k = 0; k < g.n; ++k)
-        if (g.a[k].ncp % W) return hipErrorInvalidValue;
+    for (int k = 0; k < g.n; ++k) {
+        const int tiles = (g.a[k].ka + g.a[k].kb + W - 1) / W;
+        if (g.a[k].ncp % W || tiles <= 0) return hipErrorInvalidValue;
+        g.a[k].div = div_mul((uint32_t)tiles);
+    }
     const dim3 grid((unsigned)g.off[g.n]), block(W * PlanV<NX, V>::T);
     const bool pr = g.a[0].prune != 0;
 #define MSF_COLG(L, PR)                                                                            \

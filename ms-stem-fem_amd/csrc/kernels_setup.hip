@@ -373,14 +373,14 @@ struct BandCols {
 };
 
 // slice.cpp:1741-1748 (/ NxNy).  The FP32 copy used by the slice loop holds
-// t' = t/s (adfstem.cpp:1936,1949 divide by sqrtNxNy) as (t're - 1/s, t'im):
-// the deviation from vacuum keeps full FP32 relative precision.
+// t - 1: the deviation from vacuum keeps full FP32 relative precision, and the
+// 1/sqrtNxNy of adfstem.cpp:1936,1949 is the column pass's.
 struct FinishRows {
     const double2* band;
     double2* t64;
     float2* t32;
     int nx, ny, ba, bb, ldb;
-    double nxny, s;
+    double nxny;
     __device__ __forceinline__ double2 load(int plane, int i, int j) const
     {
         const double2* row = band + ((int64_t)plane * nx + i) * ldb;
@@ -400,8 +400,7 @@ struct FinishRows {
             const double2 b{x[p + E / 2].x / nxny, x[p + E / 2].y / nxny};
             row[j] = a;
             row[j + ny / 2] = b;
-            pairs[j] = float4{(float)(a.x / s - 1.0 / s), (float)(a.y / s),
-                              (float)(b.x / s - 1.0 / s), (float)(b.y / s)};
+            pairs[j] = float4{(float)(a.x - 1.0), (float)a.y, (float)(b.x - 1.0), (float)b.y};
         }
     }
 };
@@ -433,7 +432,7 @@ hipError_t launch_build(const BuildArgs& a, const double2* twx, const double2* t
             a.nx, BandCols{a.band, a.bw, a.nx, a.ny, a.ba, a.bb, a.ldb}, a.ba + a.bb, a.k, twx, s);
     if (e == hipSuccess)
         e = launch_rows64<Fft64::Inverse>(
-            a.ny, FinishRows{a.band, a.t64, a.t32, a.nx, a.ny, a.ba, a.bb, a.ldb, a.nxny, a.sqrt_nxny},
+            a.ny, FinishRows{a.band, a.t64, a.t32, a.nx, a.ny, a.ba, a.bb, a.ldb, a.nxny},
             a.nx, a.k, twy, s);
     return e;
 }

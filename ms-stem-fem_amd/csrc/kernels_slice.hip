@@ -154,6 +154,15 @@ int col_tile_auto(int nx, int v, int batch, int ncp, bool beside)
     return (int64_t)batch * (ncp / std::max(w, 1)) < kCUs ? 1 : w;
 }
 
+// The difference of two of a 3-point step's inputs carries a third of the
+// energy and is the part scaled by sin 60 (squared amplitude 1 + 2 err); twice,
+// for the forward and the inverse step.
+double fp32_gain(int n)
+{
+    constexpr double s60 = 0.86602540378443864676;
+    return n % 3 == 0 ? 1.0 + 2.0 * ((double)(float)s60 / s60 - 1.0) / 3.0 : 1.0;
+}
+
 // The alternate 1024 plan takes 4 columns where its launches have the GPU to
 // themselves (64 positions of 1024 x 1024, 20 slices, one chain: 7.66 ms
 // against 7.81 with 8) and 8 beside the row passes of a second chain: those
@@ -177,11 +186,12 @@ int col_tile_default(int nx, int v, bool beside)
 // With ev0/ev1 the dispatch packet itself stamps the kernel's start and end
 // (hipExtLaunchKernelGGL), so profiled durations carry no marker overhead.
 template <int NY, int V, int RT>
-static hipError_t row_pass_rt(bool first, int tmode, const RowPassArgs& a, hipStream_t s,
+static hipError_t row_pass_rt(bool first, int tmode, RowPassArgs a, hipStream_t s,
                               hipEvent_t ev0, hipEvent_t ev1)
 {
     constexpr int RPW = RT / PlanV<NY, V>::T;
     const int64_t groups = (a.batch + RPW - 1) / RPW;
+    a.div = div_mul((uint32_t)groups);
     const dim3 grid((unsigned)(groups * a.nx));
     const dim3 block(RT);
 #define MSF_ROW(F, M, PR)                                                                          \
@@ -239,10 +249,11 @@ hipError_t launch_row_pass(int ny, bool first, int tmode, const RowPassArgs& a, 
 }
 
 template <int NX, int V, int W>
-static hipError_t col_pass_w(bool last, const ColPassArgs& a, hipStream_t s, hipEvent_t ev0,
+static hipError_t col_pass_w(bool last, ColPassArgs a, hipStream_t s, hipEvent_t ev0,
                              hipEvent_t ev1)
 {
-    if (a.ncp % W) return hipErrorInvalidValue;
+    if (a.ncp % W || a.ka + a.kb <= 0) return hipErrorInvalidValue;
+    a.div = div_mul((uint32_t)((a.ka + a.kb + W - 1) / W));
     const dim3 grid((unsigned)((int64_t)a.batch * ((a.ka + a.kb + W - 1) / W)));
     const dim3 block(W * PlanV<NX, V>::T);
 #define MSF_COL(L, PR)                                                                             \
@@ -354,8 +365,8 @@ bool fused_supported(int n, const RowPassArgs& ra, const ColPassArgs& ca)
 }
 
 template <int N>
-static hipError_t fused_n(bool first, bool last, int tmode, const RowPassArgs& ra,
-                          const ColPassArgs& ca, hipStream_t s)
+static hipError_t fused_n(bool first, bool last, int tmode, RowPassArgs ra, ColPassArgs ca,
+                          hipStream_t s)
 {
     if constexpr (!FusedShape<N>::exists) {
         return hipErrorNotSupported;
@@ -366,6 +377,8 @@ static hipError_t fused_n(bool first, bool last, int tmode, const RowPassArgs& r
         constexpr int RPW = RT / PlanV<N, VR>::T;
         const int nr = ((ra.batch + RPW - 1) / RPW) * ra.nx;
         const int nc = ca.batch * ((ca.ka + ca.kb + W - 1) / W);
+        ra.div = div_mul((uint32_t)((ra.batch + RPW - 1) / RPW));
+        ca.div = div_mul((uint32_t)((ca.ka + ca.kb + W - 1) / W));
         const dim3 grid((unsigned)(nr + nc)), block(RT);
 #define MSF_FUSED(F, L, M)                                                                         \
     hipLaunchKernelGGL((fused_pass_kernel<N, VR, VC, F, L, M, true, true, W, RT>), grid, block, 0,  \

@@ -268,7 +268,9 @@ int msf_specimen_build(msf_ctx* c, const msf_grid* grid, const double* q, const 
             }
         }
 
-        // propagators (slice.cpp:1293-1363), FP64 -> FP32; P_y carries 1/sqrtNxNy
+        // propagators (slice.cpp:1293-1363), FP64 -> FP32; P_y carries 1/NxNy,
+        // over what the FP32 transforms of a slice do to the wave's norm
+        const double gain = msf::fp32_gain(nx) * msf::fp32_gain(ny), py_div = d.nxny * gain;
         std::vector<float2> pxs((size_t)S * nx), pys((size_t)S * ny);
         std::vector<double2> pxd((size_t)S * nx), pyd((size_t)S * ny);
         const bool same_axes = d.kx == d.ky;
@@ -282,7 +284,7 @@ int msf_specimen_build(msf_ctx* c, const msf_grid* grid, const double* q, const 
             if (!same_axes) msf::propagator(d.lambda, sl.thick[s], d.ky, d.bw_t, p);
             for (int j = 0; j < ny; ++j) {
                 pyd[(size_t)s * ny + j] = double2{p[2 * j], p[2 * j + 1]};
-                pys[(size_t)s * ny + j] = float2{(float)(p[2 * j] / d.sqrt_nxny), (float)(p[2 * j + 1] / d.sqrt_nxny)};
+                pys[(size_t)s * ny + j] = float2{(float)(p[2 * j] / py_div), (float)(p[2 * j + 1] / py_div)};
             }
         }
         auto bail = [&](int code) {
@@ -363,7 +365,6 @@ int msf_specimen_build(msf_ctx* c, const msf_grid* grid, const double* q, const 
         ba.lgab = d.lambda * d.gamma * (1 / (grid->xperiod * grid->yperiod));
         ba.s = std::sqrt((double)M);
         ba.nxny = d.nxny;
-        ba.sqrt_nxny = d.sqrt_nxny;
         // slices per chunk: work arrays of 96 MiB, which stay in the 256 MB
         // Infinity Cache between the passes
         const int64_t spectra = (int64_t)std::max(nsp, 1) * nx * ba.lds * (int64_t)sizeof(double2);

@@ -279,10 +279,10 @@ struct msf_specimen {
     std::vector<double> lower, thick;
     std::vector<uint32_t> counts;
     msf_impl::DevBuf tables; // the small tables below, one allocation
-    msf_impl::DevBuf t32;  // [S][nx][ny] float2, t / sqrtNxNy, rows in the pair layout (pair_pos)
+    msf_impl::DevBuf t32;  // [S][nx][ny] float2, t - 1, rows in the pair layout (pair_pos)
     msf_impl::DevBuf t64;  // [S][nx][ny] double2, t as built
     msf_impl::DevBuf px;   // [S][nx] float2
-    msf_impl::DevBuf py;   // [S][ny] float2, P_y / sqrtNxNy
+    msf_impl::DevBuf py;   // [S][ny] float2, P_y / NxNy
     msf_impl::DevBuf px64; // [S][nx] double2
     msf_impl::DevBuf py64; // [S][ny] double2
     msf_impl::DevBuf dkx, dky; // [nx], [ny] spatial frequencies, FP64

@@ -31,26 +31,33 @@ template <typename T> __device__ __forceinline__ T& elem32(T* base, uint32_t k)
 {
     return *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + k * (uint32_t)sizeof(T));
 }
+template <typename T> __device__ __forceinline__ const T& elem32(const T* base, uint32_t k)
+{
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + k * (uint32_t)sizeof(T));
+}
 
 // ------------------------------------------------------------------ row pass
-// Transmission of one row.  With t' = t/s = (tau + 1/s, ti) and the
-// reference's in-place update (TMODE 0: Im uses the updated Re), for the
-// scattered wave u and the vacuum wave u0:
-//   a  = t're u_re - ti u_im,            b  = t're u_im + ti a
-//   Da = tau u0_re - ti u0_im,           Db = tau u0_im + ti (u0_re/s + Da)
-// and TMODE 1 (exact product) uses b = t're u_im + ti u_re, Db = tau u0_im + ti u0_re.
+// Transmission of one pixel, for the scattered wave u, the vacuum wave u0 and
+// U = u + u0, with (tau, ti) = t - 1 and everything times s = sqrt(nx ny)
+// (the column pass's P_y carries 1/s^2).  The scattered part of T(U) is
+//   A = tau U_re + u_re - ti U_im,
+//   B = tau U_im + u_im + ti (A + u0_re) / s     (TMODE 0)
+// since the reference's in-place update forms Im from the updated Re, whose
+// value is (A + u0_re) / s; TMODE 1 (exact product) has B = tau U_im + u_im +
+// ti U_re.  Eight operations a value: the row pass is bound by them, and the
+// products with u and u0 taken apart were twelve.
 template <bool FIRST, int TMODE>
-__device__ __forceinline__ float2 transmit_point(float2 u, float2 tv, float2 u0, float is)
+__device__ __forceinline__ float2 transmit_point(float2 u, float2 t, float2 u0, float is)
 {
-    const float da = tv.x * u0.x - tv.y * u0.y;
-    const float db = (TMODE == 0) ? tv.x * u0.y + tv.y * (u0.x * is + da) : tv.x * u0.y + tv.y * u0.x;
     if constexpr (FIRST) {
-        return float2{da, db};
+        const float a = fmaf(t.x, u0.x, -(t.y * u0.y));
+        return float2{a, TMODE == 0 ? fmaf(t.x, u0.y, (t.y * is) * (a + u0.x))
+                                    : fmaf(t.x, u0.y, t.y * u0.x)};
     } else {
-        const float tr = tv.x + is;
-        const float re = tr * u.x - tv.y * u.y;
-        const float im = (TMODE == 0) ? tr * u.y + tv.y * re : tr * u.y + tv.y * u.x;
-        return float2{re + da, im + db};
+        const float Ux = u.x + u0.x, Uy = u.y + u0.y;
+        const float a = fmaf(t.x, Ux, fmaf(-t.y, Uy, u.x));
+        return float2{a, TMODE == 0 ? fmaf(t.x, Uy, fmaf(t.y * is, a + u0.x, u.y))
+                                    : fmaf(t.x, Uy, fmaf(t.y, Ux, u.y))};
     }
 }
 
@@ -76,16 +83,6 @@ template <int N, int E> __host__ __device__ constexpr bool always_high(int p)
     return (N / E) * p >= N - N / 4;
 }
 
-template <int N> __device__ __forceinline__ int wrap_sub(int j, int s)
-{
-    if constexpr ((N & (N - 1)) == 0) {
-        return (j - s) & (N - 1);
-    } else {
-        const int d = j - s;
-        return d < 0 ? d + N : d;
-    }
-}
-
 // Workgroup -> (row i, group of RPW positions).  Consecutive launch indices go
 // to different XCDs round-robin; the permutation gives each XCD a contiguous
 // band of rows so that the t and u0 rows a band needs are fetched into that
@@ -100,6 +97,16 @@ __device__ __forceinline__ int xcd_band(int L, int G)
     const int q = G / kXcd, r = G % kXcd;
     const int x = L % kXcd, k = L / kXcd;
     return x * q + min(x, r) + k;
+}
+
+// g / d for uniform 0 <= g < 2^31 by the host's multiplier (2^32 - 1) / d:
+// the product's high word is the quotient or one less.  A handful of scalar
+// instructions; the compiler's own division of uniform values goes through
+// the vector unit and back.
+__device__ __forceinline__ int div_by(uint32_t g, uint32_t d, uint32_t mul)
+{
+    const uint32_t q = __umulhi(g, mul);
+    return (int)(g - q * d >= d ? q + 1 : q);
 }
 
 // lanes of a row-pass workgroup: RPW = row_threads / T rows share the staged
@@ -146,16 +153,16 @@ template <int NY, int V> __host__ __device__ constexpr int row_len()
     using P = PlanV<NY, V>;
     return P::T >= 16 ? P::kExchangeLen : (P::kExchangeLen + 7) / 16 * 16 + 8;
 }
-// Row passes that read every transmission and u0 pair of a lane before the
-// first product (the alternate 1024 plan: row pass 57.5 -> 53.4 us; the
-// primary 512 plan: the 512^2 job +0.7 %); the others interleave reads and
-// products, which keeps their registers lower (384: 128 against 149, the
-// alternate 256 plan: 101 against 128 with spills; the uneven 256-512 job
-// set +1 %).
-template <int NY, int V> __host__ __device__ constexpr bool row_reads_ahead()
-{
-    return (NY == 1024 && V == 1) || (NY == 512 && V == 0);
-}
+//
+// The row pass is bound by vector instructions (78-84 % of the cycles at 512
+// and 1024), so what is uniform or known at compile time stays out of the
+// vector unit: the workgroup's division, the row and u0 addresses (32-bit
+// offsets), the table staging in 16-byte words, the wrap of the shifted u0.
+// Together with transmit_point, and with every t and u0 read of a lane issued
+// before the first product, per pass: 128^2 39.4 -> 37.1 us (1024 positions),
+// 192^2 46.8 -> 43.9 (496), 256^2 40.1 -> 36.2 (272), 384^2 50.8 -> 47.4
+// (112), 512^2 41.5 -> 38.7 (64), 768^2 36.5 -> 32.5 (16), 1024^2 50.7 -> 50.1
+// (16; its tables come from L2, which bounds it now).
 template <int NY, int V, int RT> __host__ __device__ constexpr int row_smem_len()
 {
     return (row_is_lean<NY, V, RT>() ? 0 : plan_tw_len<PlanV<NY, V>>() + NY) +
@@ -172,53 +179,33 @@ __device__ __forceinline__ void row_body(const RowPassArgs& a, int blk, float2* 
     constexpr int RPW = RT / T;
     constexpr int PS = 0, LEN = row_len<NY, V>();
     constexpr bool LEAN = row_is_lean<NY, V, RT>();
+    constexpr int TW = plan_tw_len<P>();
     float2* s_tw = smem;
-    float2* s_t = smem + (LEAN ? 0 : plan_tw_len<P>());
-    float2* s_buf = smem + (LEAN ? 0 : plan_tw_len<P>() + NY);
+    float2* s_t = smem + (LEAN ? 0 : TW);
+    float2* s_buf = smem + (LEAN ? 0 : TW + NY);
 
     // workgroup-uniform decode (scalar unit)
     const int groups = (a.batch + RPW - 1) / RPW;
     const int g = xcd_band(blk, groups * a.nx);
-    const int i = g / groups;
+    const int i = div_by(g, groups, a.div);
     const int b0 = (g - i * groups) * RPW;
-
-    // twiddles and the transmission row i, shared by the RPW rows of the group
-    const float2* trow = a.t + (int64_t)i * NY;
-    if constexpr (!LEAN) {
-        for (int e = threadIdx.x; e < NY; e += blockDim.x) {
-            if (e < plan_tw_len<P>()) s_tw[e] = a.tw[e];
-            s_t[e] = trow[e];
-        }
-        __syncthreads();
-    }
-    const float2* tw = LEAN ? a.tw : s_tw;
-    const float2* tt = LEAN ? trow : s_t;
 
     // with T == 64 each row is one wavefront: keep its index in a scalar register
     const int lr = (T == 64) ? __builtin_amdgcn_readfirstlane(threadIdx.x / T) : threadIdx.x / T;
     const int t = threadIdx.x % T;
     const bool active = b0 + lr < a.batch;
-    const int b = active ? b0 + lr : a.batch - 1;
-    float2* row = a.psi + ((int64_t)b * a.nx + i) * a.ncp;
+    const int lb = active ? lr : a.batch - 1 - b0; // lanes past the batch repeat its last position
+    // rows and u0 pairs by 32-bit offsets from uniform bases: the rows of a
+    // workgroup lie within RPW planes, u0 within 16 MB
+    float2* base = a.psi + ((int64_t)b0 * a.nx + i) * a.ncp;
+    const uint32_t row = (uint32_t)lb * (uint32_t)(a.nx * a.ncp);
     float2* lds = s_buf + lr * LEN;
     const int hi = NY - a.kb;           // first kept column of the negative-ky band
     const int off = a.ka + a.kb - NY;   // compact index = j + off for j >= hi
+    const int2 sh = a.shift[b0 + lb];
 
-    // Transmission and u0 rows are stored as pairs (pair_pos): a lane's
-    // elements p and p + E/2 are j and j + NY/2, and one 16-byte read fetches
-    // both, of t at j and of u0 at the shifted r = (j - sy) mod NY.
-    const int2 sh = a.shift[b];
-    int ii = i - sh.x;
-    if (ii < 0) ii += a.nx;
-    const float2* urow = a.u0 + (int64_t)ii * (2 * NY);
-    auto pair_at = [&](int p, float4& tv, float4& uv) {
-        const int j = t + T * p;
-        int r = j - sh.y;
-        if (r < 0) r += NY;
-        tv = *reinterpret_cast<const float4*>(tt + 2 * j);
-        uv = *reinterpret_cast<const float4*>(urow + 2 * r);
-    };
-
+    // the wave is asked for before the tables, so that both are on their way
+    // when the workgroup meets at the barrier
     float2 x[E];
     if constexpr (!FIRST) {
 #pragma unroll
@@ -227,42 +214,61 @@ __device__ __forceinline__ void row_body(const RowPassArgs& a, int blk, float2* 
             if (PRUNE && in_zero_band<NY, E>(p)) {
                 x[p] = float2{0.f, 0.f};
             } else if (PRUNE && always_low<NY, E>(p)) {
-                x[p] = elem32(row, j);
+                x[p] = elem32(base, row + j);
             } else if (PRUNE && always_high<NY, E>(p)) {
-                x[p] = elem32(row, j + (uint32_t)off);
+                x[p] = elem32(base, row + j + (uint32_t)off);
             } else {
                 const bool lo = (int)j < a.ka, up = (int)j >= hi;
                 // lanes outside the kept band all read element 0 (one shared line)
-                const float2 v = elem32(row, lo ? j : (up ? j + (uint32_t)off : 0u));
+                const float2 v = elem32(base, row + (lo ? j : (up ? j + (uint32_t)off : 0u)));
                 x[p] = (lo || up) ? v : float2{0.f, 0.f};
             }
         }
-        P::template run<true, float2, (T <= 64), PS>(x, lds, tw, t);
     }
 
-    const float is = a.inv_s;
-    auto transmit = [&](int p, float2 tv, float2 u0) {
-        x[p] = transmit_point<FIRST, TMODE>(x[p], tv, u0, is);
-    };
-    if constexpr (row_reads_ahead<NY, V>()) {
-        // all reads issued before the first product: more of them in flight,
-        // for more registers
-        float4 tq[E / 2], uq[E / 2];
+    // twiddles and the transmission row i, shared by the RPW rows of the
+    // group: 16 bytes a lane, the two tables one after the other in LDS
+    const float2* trow = a.t + (int64_t)i * NY;
+    if constexpr (!LEAN) {
+        constexpr int NW = TW / 2, N4 = NW + NY / 2;
+        static_assert(TW % 2 == 0 && NY % 2 == 0, "tables in 16-byte words");
+        float4* dst = reinterpret_cast<float4*>(smem);
 #pragma unroll
-        for (int p = 0; p < E / 2; ++p) pair_at(p, tq[p], uq[p]);
-#pragma unroll
-        for (int p = 0; p < E / 2; ++p) {
-            transmit(p, float2{tq[p].x, tq[p].y}, float2{uq[p].x, uq[p].y});
-            transmit(p + E / 2, float2{tq[p].z, tq[p].w}, float2{uq[p].z, uq[p].w});
+        for (int k = 0; k < (N4 + RT - 1) / RT; ++k) {
+            const int e = (int)threadIdx.x + k * RT;
+            if (N4 % RT == 0 || e < N4)
+                dst[e] = e < NW ? reinterpret_cast<const float4*>(a.tw)[e]
+                                : reinterpret_cast<const float4*>(trow)[e - NW];
         }
-    } else {
+        __syncthreads();
+    }
+    const float2* tw = LEAN ? a.tw : s_tw;
+    const float4* tt = reinterpret_cast<const float4*>(LEAN ? trow : s_t);
+
+    if constexpr (!FIRST) P::template run<true, float2, (T <= 64), PS>(x, lds, tw, t);
+
+    // Transmission and u0 rows are stored as pairs (pair_pos): a lane's
+    // elements p and p + E/2 are j and j + NY/2, and one 16-byte read fetches
+    // both, of t at j and of u0 at the shifted r = (j - sy) mod NY.  All reads
+    // are issued before the first product.
+    int ii = i - sh.x;
+    if (ii < 0) ii += a.nx;
+    const uint32_t urow = (uint32_t)ii * (uint32_t)NY, u00 = (uint32_t)(t - sh.y);
+    const float4* u0 = reinterpret_cast<const float4*>(a.u0);
+    float4 tq[E / 2], uq[E / 2];
 #pragma unroll
-        for (int p = 0; p < E / 2; ++p) {
-            float4 tv, uv;
-            pair_at(p, tv, uv);
-            transmit(p, float2{tv.x, tv.y}, float2{uv.x, uv.y});
-            transmit(p + E / 2, float2{tv.z, tv.w}, float2{uv.z, uv.w});
-        }
+    for (int p = 0; p < E / 2; ++p) {
+        const uint32_t r0 = u00 + (uint32_t)(T * p); // negative (as unsigned: large) below the shift
+        const uint32_t r = (NY & (NY - 1)) == 0 ? r0 & (NY - 1) : min(r0, r0 + (uint32_t)NY);
+        tq[p] = tt[t + T * p];
+        uq[p] = elem32(u0, urow + r);
+    }
+#pragma unroll
+    for (int p = 0; p < E / 2; ++p) {
+        x[p] = transmit_point<FIRST, TMODE>(x[p], float2{tq[p].x, tq[p].y},
+                                            float2{uq[p].x, uq[p].y}, a.inv_s);
+        x[p + E / 2] = transmit_point<FIRST, TMODE>(x[p + E / 2], float2{tq[p].z, tq[p].w},
+                                                    float2{uq[p].z, uq[p].w}, a.inv_s);
     }
 
     P::template run<false, float2, (T <= 64), PS>(x, lds, tw, t);
@@ -273,12 +279,12 @@ __device__ __forceinline__ void row_body(const RowPassArgs& a, int blk, float2* 
             const uint32_t j = (uint32_t)(t + T * p);
             if (PRUNE && in_zero_band<NY, E>(p)) continue;
             if (PRUNE && always_low<NY, E>(p)) {
-                elem32(row, j) = x[p];
+                elem32(base, row + j) = x[p];
             } else if (PRUNE && always_high<NY, E>(p)) {
-                elem32(row, j + (uint32_t)off) = x[p];
+                elem32(base, row + j + (uint32_t)off) = x[p];
             } else {
-                if ((int)j < a.ka) elem32(row, j) = x[p];
-                else if ((int)j >= hi) elem32(row, j + (uint32_t)off) = x[p];
+                if ((int)j < a.ka) elem32(base, row + j) = x[p];
+                else if ((int)j >= hi) elem32(base, row + j + (uint32_t)off) = x[p];
             }
         }
     }
@@ -358,7 +364,7 @@ template <int NX, int V, int W> __host__ __device__ constexpr bool col_fits()
     return (size_t)W * col_len<NX, V, W>() * 8 + tables <= 160 * 1024 && W * P::T <= 1024;
 }
 
-// band limit and propagator P_x[i] * P_y[j] (which carries 1/sqrtNxNy) of one pixel
+// band limit and propagator P_x[i] * P_y[j] (which carries 1/(nx ny)) of one pixel
 __device__ __forceinline__ float2 propagate_point(float2 f, float2 pxi, float2 pyj, bool keep)
 {
     const float2 pr = float2{pxi.x * pyj.x - pxi.y * pyj.y, pxi.x * pyj.y + pxi.y * pyj.x};
@@ -410,7 +416,7 @@ __device__ __forceinline__ void col_body(const ColPassArgs& a, int blk, int nblk
     const int nc = a.ka + a.kb;
     const int ntiles = (nc + W - 1) / W;
     const int g = xcd_band(blk, nblk);
-    const int b = g / ntiles;
+    const int b = div_by(g, ntiles, a.div);
     const int j0 = (g - b * ntiles) * W;
     float2* tile = a.psi + (int64_t)b * NX * a.ncp + j0;
 
@@ -444,7 +450,7 @@ __device__ __forceinline__ void col_body(const ColPassArgs& a, int blk, int nblk
     P::template run<false, float2, WAVE, PS>(x, lds, tw, t);
 
     // band limit (bw_limit + propagate's k^2 test, decided on the host) and
-    // propagator P_x[i] * P_y[j]; P_y carries the 1/sqrtNxNy of the FFT
+    // propagator P_x[i] * P_y[j]; P_y carries the 1/sqrtNxNy of the FFT and of the transmission
     const float2 pyj = active ? a.py[j] : float2{0.f, 0.f};
     // kept rows of this column, decided on the host (one pair per column
     // instead of a range table per row)
