@@ -281,7 +281,26 @@ template <bool WAVE> __device__ __forceinline__ void lds_sync()
 // the column pass from 47 to 40 us (registers 128 -> 100 and 126 -> 75), per
 // 496 of 192^2 50 -> 46 and 46 -> 40, per 272 of 256^2 41.2 -> 40.1 and
 // 35.5 -> 35.3, per 64 of 512^2 41.4 -> 40.3 and 37.5 -> 36.5 us.
+//
+// The first two stages of radix 4 on 16 lanes or more (spans 1 and 4) use no
+// padding but a swizzle, slot = e ^ ((e / 16) % 4 * NS): 16 lanes write
+// butterflies j .. j + 15 and the four that would share a bank differ in
+// (j / 4) % 4, which is (e / 16) % 4; reads of 16 elements see one constant.
+// The buffer is then the transform's length, where the span of 4 needed a
+// quarter more, and a CU holds four workgroups of the 768 row pass instead of
+// three and five at 192 and 384 instead of four: row passes 32.4 -> 30.2 us
+// (16 positions of 768^2), 46.8 -> 44.2 (112 of 384^2), 41.6 -> 40.2 (496 of
+// 192^2).
 template <int T, int BPT, int R, int NS, int PS> struct LdsExchange {
+    // swizzled: slot = (lane base ^ constant) + constant, four bases at most
+    static constexpr bool swizzle = PS == 0 && R == 4 && (NS == 1 || NS == 4) && T >= 16 && T % 16 == 0;
+    static __device__ __forceinline__ int swz_write_base(int t)
+    {
+        return 4 * NS * (t / NS) + t % NS + ((t >> 2) & 3) * NS;
+    }
+    static __device__ __forceinline__ int swz_read_base(int t) { return t ^ (((t >> 4) & 3) * NS); }
+    static __host__ __device__ constexpr int swz_write_xor(int q) { return q * NS; }
+    static __host__ __device__ constexpr int swz_read_xor(int p) { return ((T / 16 * p) & 3) * NS; }
     static constexpr int STRIDE = PS < 0 ? -PS : 1;
     static constexpr int PB = PS < 0 ? 8 : PS > 0 ? 1 << (PS > 0 ? PS : 0) : NS == 1 ? 16 : NS * R;
     static constexpr int PA = PS != 0 || NS == 1 ? 1 : NS >= 16 ? 0 : NS;
@@ -292,7 +311,7 @@ template <int T, int BPT, int R, int NS, int PS> struct LdsExchange {
     static constexpr bool high = !low && NS % T == 0 && A && T % PB == 0;
     static constexpr bool reads = PA == 0 || T % PB == 0 || PB % T == 0;
     static constexpr bool fold = (low || high || PA == 0) && reads;
-    static __host__ __device__ constexpr int at(int e) { return e * STRIDE + (e / PB) * PA; }
+    static __host__ __device__ constexpr int at(int e) { return swizzle ? e : e * STRIDE + (e / PB) * PA; }
     static __device__ __forceinline__ int write_base(int t)
     {
         if constexpr (high) return t * STRIDE + (t / PB) * PA;
@@ -397,7 +416,15 @@ __device__ __forceinline__ void fft_stage(C (&x)[E], C* lds, const C* tw, int t)
         // an address per element)
         static_assert(PS != 0 || X::fold, "per-exchange padding without constant offsets");
         constexpr bool FOLD = X::fold && (PS <= 0 || E >= 12);
-        if constexpr (FOLD) {
+        if constexpr (X::swizzle) {
+            const int w = X::swz_write_base(t);
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                C* wq = lds + (w ^ X::swz_write_xor(q));
+#pragma unroll
+                for (int m = 0; m < BPT; ++m) wq[m * T * R] = y[m * R + q];
+            }
+        } else if constexpr (FOLD) {
             C* w = lds + X::write_base(t);
 #pragma unroll
             for (int m = 0; m < BPT; ++m)
@@ -413,7 +440,11 @@ __device__ __forceinline__ void fft_stage(C (&x)[E], C* lds, const C* tw, int t)
             }
         }
         lds_sync<WAVE>();
-        if constexpr (FOLD) {
+        if constexpr (X::swizzle) {
+            const int r = X::swz_read_base(t);
+#pragma unroll
+            for (int p = 0; p < E; ++p) x[p] = (lds + (r ^ X::swz_read_xor(p)))[T * p];
+        } else if constexpr (FOLD) {
             const C* r = lds + X::read_base(t);
 #pragma unroll
             for (int p = 0; p < E; ++p) x[p] = r[X::read_off(p)];

@@ -127,12 +127,13 @@ template <int NY, int V> __host__ __device__ constexpr int row_threads()
 template <int NY, int V> __host__ __device__ constexpr bool row_lean() { return NY == 1024; }
 
 // Occupancy the row pass asks of the register allocator: 6 waves per SIMD for
-// the 8-value plans; the plans with 12 to 24 values per lane need more
-// registers, and ask for what they reach (their allocation is unchanged).
+// the 8-value plans; the plans with 12 and 16 values per lane need more
+// registers, and ask for what their LDS and registers allow (five workgroups
+// per CU at 192 and 384, where 98 registers would leave four waves).
 template <int NY, int V> __host__ __device__ constexpr int row_waves()
 {
     constexpr int E = PlanV<NY, V>::E;
-    return E <= 8 ? 6 : (E == 16 ? (NY == 512 ? 3 : 4) : (E == 12 ? 3 : 2));
+    return E <= 8 ? 6 : (E == 16 ? (NY == 512 ? 3 : 4) : (E == 12 ? (NY == 768 ? 4 : 5) : 2));
 }
 
 // RT lanes per workgroup: row_threads() for batches that fill it, or one
@@ -315,14 +316,29 @@ template <int NX, int V = 0> struct ColTile {
     static constexpr int W = (NX == 1024 && V == 1) ? 4 : (16 * lds_len(NX) * 8 > 48 * 1024) ? 8 : 16;
 };
 
+// Slot of row r + T p in a tile's column: the rows as they are where the
+// exchanges are swizzled (16 lanes read 16 rows without conflict), else one
+// slot more every 16 rows, as after the first stage of radix 8 or 16, whose
+// addresses it then shares.
+template <typename P> __host__ __device__ constexpr bool col_plain()
+{
+    return P::T >= 16 && P::kExchangeLen == P::N;
+}
+template <typename P> __device__ __forceinline__ int col_slot(int r, int p)
+{
+    if constexpr (col_plain<P>()) return r + P::T * p;
+    else return lds_pad_at<P::T, 4>(r, p);
+}
+
 // column stride of the LDS tile: a 16-lane group of the coalesced load/store
-// phases covers W' = min(W, 16) columns x 16/W' rows; a stride congruent to
-// 16/W' modulo 16 (8-byte words) puts those 16 lanes on distinct bank pairs
+// phases covers W' = min(W, 16) columns x g = 16/W' rows; a stride that is an
+// odd multiple of g puts those 16 lanes on distinct bank pairs
 template <int NX, int V, int W> __host__ __device__ constexpr int col_len()
 {
-    constexpr int base = PlanV<NX, V>::kExchangeLen;
-    constexpr int want = (16 / (W < 16 ? W : 16)) % 16;
-    return base + ((want - base % 16) + 16) % 16;
+    constexpr int tile = col_plain<PlanV<NX, V>>() ? NX : lds_len<4>(NX);
+    constexpr int base = PlanV<NX, V>::kExchangeLen > tile ? PlanV<NX, V>::kExchangeLen : tile;
+    constexpr int g = 16 / (W < 16 ? W : 16);
+    return (base + g - 1) / (2 * g) * (2 * g) + g;
 }
 
 // Lean tiles: when the twiddle and propagator tables would keep two
@@ -347,12 +363,30 @@ template <int NX, int V, int W> __host__ __device__ constexpr int col_bound()
     return (V || PlanV<NX, V>::E >= 12) ? W * PlanV<NX, V>::T : 1024;
 }
 
+// Workgroups of a column pass that a CU holds: by its 160 KB of LDS (given
+// out in steps of 1,280 bytes) and by waves (8 per SIMD, or 5 with the 75 to
+// 96 registers of the plans with 12 and 16 values per lane).
+template <int NX, int V, int W> __host__ __device__ constexpr int col_per_cu(bool px)
+{
+    constexpr int tile = (W * col_len<NX, V, W>() + plan_tw_len<PlanV<NX, V>>()) * 8;
+    constexpr int waves = PlanV<NX, V>::E <= 8 ? 32 : 20, lanes = W * PlanV<NX, V>::T;
+    const int by_lds = 160 * 1024 / ((tile + (px ? NX * 8 : 0) + 1279) / 1280 * 1280);
+    return by_lds < waves * 64 / lanes ? by_lds : waves * 64 / lanes;
+}
+// The propagator row, read once per element, stays in L2 where the CU then
+// holds a workgroup more: tiles of 8 columns of 512 rows take 40,512 bytes
+// and run four to a CU instead of three, 37.3 -> 35.0 us per 64 positions.
+template <int NX, int V, int W> __host__ __device__ constexpr bool col_px_lean()
+{
+    return col_lean<NX, V, W>() || col_per_cu<NX, V, W>(false) > col_per_cu<NX, V, W>(true);
+}
+
 // LDS of a column-pass workgroup in float2 units: the staged twiddle and
 // propagator tables (unless lean), the exit roots (last slice) and the tile.
 template <int NX, int V, bool LAST, int W> __host__ __device__ constexpr int col_smem_len()
 {
-    return (col_lean<NX, V, W>() ? 0 : plan_tw_len<PlanV<NX, V>>() + NX) + (LAST ? NX : 0) +
-           W * col_len<NX, V, W>();
+    return (col_lean<NX, V, W>() ? 0 : plan_tw_len<PlanV<NX, V>>()) +
+           (col_px_lean<NX, V, W>() ? 0 : NX) + (LAST ? NX : 0) + W * col_len<NX, V, W>();
 }
 
 // tile sizes whose LDS and workgroup fit a CU
@@ -387,27 +421,26 @@ __device__ __forceinline__ void col_body(const ColPassArgs& a, int blk, int nblk
     using P = PlanV<NX, V>;
     constexpr int E = P::E, T = P::T;
     constexpr int LEN = col_len<NX, V, W>();
-    constexpr int PS = 0;  // exchanges padded each its own way,
-    constexpr int SP = 4;  // the tile's loads and stores one slot every 16 rows
-    constexpr bool LEAN = col_lean<NX, V, W>();
+    constexpr int PS = 0; // exchanges padded each its own way
+    constexpr bool LEAN = col_lean<NX, V, W>(), LEANX = col_px_lean<NX, V, W>();
     // a column transform lies in one wavefront (wave-local exchanges) or
     // spans whole wavefronts (workgroup barriers)
     static_assert(64 % T == 0 || T % 64 == 0, "a column transform must align with wavefronts");
     constexpr bool WAVE = T <= 64;
     float2* s_tw = smem;
     float2* s_px = smem + (LEAN ? 0 : plan_tw_len<P>());
-    float2* s_nat = smem + (LEAN ? 0 : plan_tw_len<P>() + NX); // roots W_nx^e (last slice)
+    float2* s_nat = s_px + (LEANX ? 0 : NX); // roots W_nx^e (last slice)
     float2* s_buf = s_nat + (LAST ? NX : 0);
 
     for (int e = threadIdx.x; e < NX; e += blockDim.x) {
         if constexpr (!LEAN) {
             if (e < plan_tw_len<P>()) s_tw[e] = a.tw[e];
-            s_px[e] = a.px[e];
         }
+        if constexpr (!LEANX) s_px[e] = a.px[e];
         if constexpr (LAST) s_nat[e] = a.twx_nat[e];
     }
     const float2* tw = LEAN ? a.tw : s_tw;
-    const float2* tpx = LEAN ? a.px : s_px;
+    const float2* tpx = LEANX ? a.px : s_px;
 
     // neighbouring tiles share 128-byte lines (W = 8 reads 64 B per row): keep
     // them on one XCD, next to each other in dispatch order
@@ -433,7 +466,7 @@ __device__ __forceinline__ void col_body(const ColPassArgs& a, int blk, int nblk
         for (int p = 0; p < E; ++p) v[p] = elem32(tile, o0 + (uint32_t)p * step);
 #pragma unroll
         for (int p = 0; p < E; ++p)
-            s_buf[c * LEN + lds_pad_at<T, SP>(r0, p)] = ok ? v[p] : float2{0.f, 0.f};
+            s_buf[c * LEN + col_slot<P>(r0, p)] = ok ? v[p] : float2{0.f, 0.f};
     }
     __syncthreads();
 
@@ -445,7 +478,7 @@ __device__ __forceinline__ void col_body(const ColPassArgs& a, int blk, int nblk
     float2* lds = s_buf + c * LEN;
     float2 x[E];
 #pragma unroll
-    for (int p = 0; p < E; ++p) x[p] = lds[lds_pad_at<T, SP>(t, p)];
+    for (int p = 0; p < E; ++p) x[p] = lds[col_slot<P>(t, p)];
 
     P::template run<false, float2, WAVE, PS>(x, lds, tw, t);
 
@@ -482,7 +515,7 @@ __device__ __forceinline__ void col_body(const ColPassArgs& a, int blk, int nblk
 
     lds_sync<WAVE>();
 #pragma unroll
-    for (int p = 0; p < E; ++p) lds[lds_pad_at<T, SP>(t, p)] = x[p];
+    for (int p = 0; p < E; ++p) lds[col_slot<P>(t, p)] = x[p];
     __syncthreads();
 
     {   // coalesced store of the tile
@@ -493,7 +526,7 @@ __device__ __forceinline__ void col_body(const ColPassArgs& a, int blk, int nblk
         if (ok) {
 #pragma unroll
             for (int p = 0; p < E; ++p)
-                elem32(tile, o0 + (uint32_t)p * step) = s_buf[c2 * LEN + lds_pad_at<T, SP>(r0, p)];
+                elem32(tile, o0 + (uint32_t)p * step) = s_buf[c2 * LEN + col_slot<P>(r0, p)];
         }
     }
 }
