@@ -335,6 +335,16 @@ template <int T, int BPT, int R, int NS, int PS> struct LdsExchange {
     static __device__ __forceinline__ constexpr int read_off(int p) { return T * p * STRIDE + (T * p / PB) * PA; }
 };
 
+// A pointer into LDS whose value the compiler takes as given: the offsets of
+// an exchange's slots then stay in its instructions, which hold 64 KB, where
+// they were otherwise added into registers of their own.
+template <typename C> __device__ __forceinline__ C* lds_at(C* lds, int slot)
+{
+    auto p = (__attribute__((address_space(3))) C*)(lds + slot);
+    asm("" : "+v"(p));
+    return (C*)p;
+}
+
 // ------------------------------------------------------------ one stage
 // Twiddles of stage s (radix R, span NS) come from a per-stage table laid out
 // [q-1][k], entry W_{NS R}^{q k}, q = 1..R-1, k = 0..NS-1, at offset TWO in
@@ -425,7 +435,7 @@ __device__ __forceinline__ void fft_stage(C (&x)[E], C* lds, const C* tw, int t)
                 for (int m = 0; m < BPT; ++m) wq[m * T * R] = y[m * R + q];
             }
         } else if constexpr (FOLD) {
-            C* w = lds + X::write_base(t);
+            C* w = lds_at(lds, X::write_base(t));
 #pragma unroll
             for (int m = 0; m < BPT; ++m)
 #pragma unroll
@@ -445,7 +455,7 @@ __device__ __forceinline__ void fft_stage(C (&x)[E], C* lds, const C* tw, int t)
 #pragma unroll
             for (int p = 0; p < E; ++p) x[p] = (lds + (r ^ X::swz_read_xor(p)))[T * p];
         } else if constexpr (FOLD) {
-            const C* r = lds + X::read_base(t);
+            const C* r = lds_at(lds, X::read_base(t));
 #pragma unroll
             for (int p = 0; p < E; ++p) x[p] = r[X::read_off(p)];
         } else {

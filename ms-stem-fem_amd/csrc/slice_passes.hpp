@@ -36,6 +36,18 @@ template <typename T> __device__ __forceinline__ const T& elem32(const T* base, 
     return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + k * (uint32_t)sizeof(T));
 }
 
+// Element K past a lane's own (byte offset `lane`) of a uniform base: K goes
+// into the instruction, so all elements of a lane share one address register.
+template <typename T> __device__ __forceinline__ T& elem_at(T* base, uint32_t lane, int K)
+{
+    return *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + lane + (int64_t)K * (int)sizeof(T));
+}
+template <typename T> __device__ __forceinline__ const T& elem_at(const T* base, uint32_t lane, int K)
+{
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + lane +
+                                       (int64_t)K * (int)sizeof(T));
+}
+
 // ------------------------------------------------------------------ row pass
 // Transmission of one pixel, for the scattered wave u, the vacuum wave u0 and
 // U = u + u0, with (tau, ti) = t - 1 and everything times s = sqrt(nx ny)
@@ -192,17 +204,20 @@ __device__ __forceinline__ void row_body(const RowPassArgs& a, int blk, float2* 
     const int b0 = (g - i * groups) * RPW;
 
     // with T == 64 each row is one wavefront: keep its index in a scalar register
-    const int lr = (T == 64) ? __builtin_amdgcn_readfirstlane(threadIdx.x / T) : threadIdx.x / T;
+    const int lr = (T % 64 == 0) ? __builtin_amdgcn_readfirstlane(threadIdx.x / T) : threadIdx.x / T;
     const int t = threadIdx.x % T;
     const bool active = b0 + lr < a.batch;
     const int lb = active ? lr : a.batch - 1 - b0; // lanes past the batch repeat its last position
     // rows and u0 pairs by 32-bit offsets from uniform bases: the rows of a
-    // workgroup lie within RPW planes, u0 within 16 MB
-    float2* base = a.psi + ((int64_t)b0 * a.nx + i) * a.ncp;
-    const uint32_t row = (uint32_t)lb * (uint32_t)(a.nx * a.ncp);
+    // workgroup lie within RPW planes, u0 within 16 MB; a row that is a whole
+    // wavefront's has its own base
+    constexpr bool OWN = T % 64 == 0;
+    float2* base = a.psi + ((int64_t)(b0 + (OWN ? lb : 0)) * a.nx + i) * a.ncp;
+    const uint32_t lane = ((OWN ? 0u : (uint32_t)lb * (uint32_t)(a.nx * a.ncp)) + (uint32_t)t) * 8u;
     float2* lds = s_buf + lr * LEN;
     const int hi = NY - a.kb;           // first kept column of the negative-ky band
-    const int off = a.ka + a.kb - NY;   // compact index = j + off for j >= hi
+    // compact index = j + (ka + kb - NY) for j >= hi; that band's base
+    float2* up = base + (a.ka + a.kb - NY);
     const int2 sh = a.shift[b0 + lb];
 
     // the wave is asked for before the tables, so that both are on their way
@@ -211,18 +226,25 @@ __device__ __forceinline__ void row_body(const RowPassArgs& a, int blk, float2* 
     if constexpr (!FIRST) {
 #pragma unroll
         for (int p = 0; p < E; ++p) {
-            const uint32_t j = (uint32_t)(t + T * p);
-            if (PRUNE && in_zero_band<NY, E>(p)) {
-                x[p] = float2{0.f, 0.f};
-            } else if (PRUNE && always_low<NY, E>(p)) {
-                x[p] = elem32(base, row + j);
-            } else if (PRUNE && always_high<NY, E>(p)) {
-                x[p] = elem32(base, row + j + (uint32_t)off);
+            const int j = t + T * p;
+            if constexpr (PRUNE) {
+                // ka and kb lie in [N/4, 3N/8]: elements below N/2 belong to the
+                // low band or to none, and a read past its edge stays in the
+                // row's ka + kb >= N/2 stored columns, as one below the high
+                // band's edge does
+                if (in_zero_band<NY, E>(p)) {
+                    x[p] = float2{0.f, 0.f};
+                } else {
+                    const bool low = T * p < NY / 2;
+                    x[p] = elem_at(low ? base : up, lane, T * p);
+                    if (low ? !always_low<NY, E>(p) && j >= a.ka : !always_high<NY, E>(p) && j < hi)
+                        x[p] = float2{0.f, 0.f};
+                }
             } else {
-                const bool lo = (int)j < a.ka, up = (int)j >= hi;
+                const bool lo = j < a.ka, hi_band = j >= hi;
                 // lanes outside the kept band all read element 0 (one shared line)
-                const float2 v = elem32(base, row + (lo ? j : (up ? j + (uint32_t)off : 0u)));
-                x[p] = (lo || up) ? v : float2{0.f, 0.f};
+                const float2 v = elem32(base, lane / 8u - (uint32_t)t + (lo ? (uint32_t)j : hi_band ? (uint32_t)(j + a.ka + a.kb - NY) : 0u));
+                x[p] = (lo || hi_band) ? v : float2{0.f, 0.f};
             }
         }
     }
@@ -277,15 +299,15 @@ __device__ __forceinline__ void row_body(const RowPassArgs& a, int blk, float2* 
     if (active) {
 #pragma unroll
         for (int p = 0; p < E; ++p) {
-            const uint32_t j = (uint32_t)(t + T * p);
-            if (PRUNE && in_zero_band<NY, E>(p)) continue;
-            if (PRUNE && always_low<NY, E>(p)) {
-                elem32(base, row + j) = x[p];
-            } else if (PRUNE && always_high<NY, E>(p)) {
-                elem32(base, row + j + (uint32_t)off) = x[p];
+            const int j = t + T * p;
+            if constexpr (PRUNE) {
+                if (in_zero_band<NY, E>(p)) continue;
+                const bool low = T * p < NY / 2;
+                if (low ? always_low<NY, E>(p) || j < a.ka : always_high<NY, E>(p) || j >= hi)
+                    elem_at(low ? base : up, lane, T * p) = x[p];
             } else {
-                if ((int)j < a.ka) elem32(base, row + j) = x[p];
-                else if ((int)j >= hi) elem32(base, row + j + (uint32_t)off) = x[p];
+                if (j < a.ka) elem_at(base, lane, T * p) = x[p];
+                else if (j >= hi) elem_at(up, lane, T * p) = x[p];
             }
         }
     }
@@ -453,24 +475,24 @@ __device__ __forceinline__ void col_body(const ColPassArgs& a, int blk, int nblk
     const int j0 = (g - b * ntiles) * W;
     float2* tile = a.psi + (int64_t)b * NX * a.ncp + j0;
 
-    {   // coalesced load of the tile (32-bit offsets from the uniform tile base).
-        // Every load is in bounds (b < batch by the grid, padding columns
-        // jc >= nc exist in the buffer), so all E loads are issued before the
-        // first LDS write and overlap; padding columns are zeroed after.
+    {   // coalesced load of the tile: one 32-bit lane offset, and a uniform
+        // base per element.  Every load is in bounds (b < batch by the grid,
+        // padding columns jc >= nc exist in the buffer), so all E loads are
+        // issued before the first LDS write and overlap; what the padding
+        // columns hold stays in their own tile columns, which nothing stores.
         const int c = threadIdx.x % W, r0 = threadIdx.x / W;
-        const bool ok = j0 + c < nc;
         const uint32_t o0 = (uint32_t)(r0 * a.ncp + c);
-        const uint32_t step = (uint32_t)(T * a.ncp);
+        const int64_t step = (int64_t)T * a.ncp;
         float2 v[E];
 #pragma unroll
-        for (int p = 0; p < E; ++p) v[p] = elem32(tile, o0 + (uint32_t)p * step);
+        for (int p = 0; p < E; ++p) v[p] = elem32(tile + p * step, o0);
 #pragma unroll
-        for (int p = 0; p < E; ++p)
-            s_buf[c * LEN + col_slot<P>(r0, p)] = ok ? v[p] : float2{0.f, 0.f};
+        for (int p = 0; p < E; ++p) s_buf[c * LEN + col_slot<P>(r0, p)] = v[p];
     }
     __syncthreads();
 
-    const int c = threadIdx.x / T;
+    // with T a multiple of 64 a wavefront's column is uniform
+    const int c = T % 64 == 0 ? __builtin_amdgcn_readfirstlane(threadIdx.x / T) : threadIdx.x / T;
     const int t = threadIdx.x % T;
     const int jc = j0 + c;
     const bool active = (b < a.batch) && (jc < nc);
@@ -494,9 +516,12 @@ __device__ __forceinline__ void col_body(const ColPassArgs& a, int blk, int nblk
             x[p] = float2{0.f, 0.f};
             continue;
         }
+        // a pruned column keeps nothing of [3N/8, 5N/8), so its elements below
+        // N/2 can only be of the low band
         const int i = t + T * p;
-        const bool keep = (i < ck.x) || (i >= NX - ck.y);
-        x[p] = propagate_point(x[p], tpx[i], pyj, keep);
+        const bool keep = PRUNE ? (T * p < NX / 2 ? i < ck.x : i >= NX - ck.y)
+                                : (i < ck.x) || (i >= NX - ck.y);
+        x[p] = propagate_point(x[p], elem_at(tpx, (uint32_t)t * 8u, T * p), pyj, keep);
     }
 
     if constexpr (!LAST) {
@@ -522,11 +547,15 @@ __device__ __forceinline__ void col_body(const ColPassArgs& a, int blk, int nblk
         const int c2 = threadIdx.x % W, r0 = threadIdx.x / W;
         const bool ok = (b < a.batch) && (j0 + c2 < nc);
         const uint32_t o0 = (uint32_t)(r0 * a.ncp + c2);
-        const uint32_t step = (uint32_t)(T * a.ncp);
+        const int64_t step = (int64_t)T * a.ncp;
+        // formed anew: twelve or sixteen bases kept from the loads would not
+        // fit the scalar registers
+        auto out = (__attribute__((address_space(1))) float2*)tile;
+        asm("" : "+s"(out));
         if (ok) {
 #pragma unroll
             for (int p = 0; p < E; ++p)
-                elem32(tile, o0 + (uint32_t)p * step) = s_buf[c2 * LEN + col_slot<P>(r0, p)];
+                elem32((float2*)(out + p * step), o0) = s_buf[c2 * LEN + col_slot<P>(r0, p)];
         }
     }
 }
