@@ -144,14 +144,34 @@ int col_tile(int nx)
     }
 }
 
+// 16-column tiles of a length that a CU holds at once
+static int col_places16(int nx, int v)
+{
+    switch (nx) {
+#define MSF_CASE(N) case N: return v ? col_per_cu<N, AltPlan<N>::exists ? 1 : 0, 16>(true) : col_per_cu<N, 0, 16>(true);
+        MSF_CASE(16) MSF_CASE(32) MSF_CASE(64) MSF_CASE(96) MSF_CASE(128) MSF_CASE(192) MSF_CASE(256)
+#undef MSF_CASE
+    default:
+        return 0;
+    }
+}
+
 // Launches of so few positions that the default tiles would leave CUs idle
 // (one position at 512^2: 44 workgroups of 8 columns for 256 CUs) take one
 // column per workgroup instead.
+// Launches of less than two rounds of 16-column tiles take tiles of 8, whose
+// last round leaves fewer CUs idle: column pass of 99 positions of 256^2
+// (1,089 tiles of 16 for 1,024 places) 16.8 -> 16.0 us, of 192 26.8 -> 26.3,
+// of 91 positions of 192 x 96 10.2 -> 9.5; 256 positions (2.75 rounds) 32.5
+// against 33.0 with tiles of 8.  Row workgroups halved by the same rule: 3 %
+// faster at 192 x 96, 1 to 2 % slower at 256^2, not kept.
 int col_tile_auto(int nx, int v, int batch, int ncp, bool beside)
 {
     const int w = col_tile_default(nx, v, beside);
     constexpr int64_t kCUs = 256;
-    return (int64_t)batch * (ncp / std::max(w, 1)) < kCUs ? 1 : w;
+    const int64_t tiles = (int64_t)batch * (ncp / std::max(w, 1));
+    if (tiles < kCUs) return 1;
+    return w == 16 && tiles < 2 * kCUs * col_places16(nx, v) ? 8 : w;
 }
 
 // The difference of two of a 3-point step's inputs carries a third of the

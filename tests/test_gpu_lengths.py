@@ -69,3 +69,27 @@ def test_two_chains_of_1024_rows_take_the_bits_of_one(msf, ctx, plan, batch):
         ctx.configure()
         spec.free()
     np.testing.assert_array_equal(out[0][0], out[1][0])
+
+
+@pytest.mark.parametrize("nx,places", [(192, 5), (256, 4)])
+def test_column_tile_follows_the_rounds_of_a_launch(msf, ctx, nx, places):
+    # 4 tiles of 16 columns a position: tiles of 8 from a launch that fills the
+    # CUs to one of two rounds, and the bits of 16-column tiles
+    ny = 96
+    cell = (nx * 0.09, ny * 0.09, 4.0)
+    q, Z = random_atoms(12, cell, seed=nx, species=(14, 29))
+    q[:, 2] = 2.0 * (np.arange(12) // 6) + 0.1
+    c = Case(nx=nx, ny=ny, cell=cell, voltage=200e3, q=q, Z=Z, min_slice=1.0, cs3=1.2e7,
+             defocus=300.0, alpha_max=0.03, adf=True, fem=False)
+    spec, line = c.gpu_specimen(msf, ctx), 2 * 256 * places // 4
+    try:
+        for n, tile in ((63, 1), (64, 8), (line - 1, 8), (line, 16)):
+            xp, yp, img = np.linspace(0.05, 0.95, n) * cell[0], np.array([0.4]) * cell[1], []
+            for t in (0, 16):
+                ctx.configure(autotune=-1, batch=n, col_tile=t)
+                img.append(ctx.adfstem(spec, c.optics(msf), xp, yp, detector=c.detector(msf))[0])
+                assert ctx.stats()["col_tile"] == (t or tile)
+            np.testing.assert_array_equal(img[0], img[1])
+    finally:
+        ctx.configure()
+        spec.free()
