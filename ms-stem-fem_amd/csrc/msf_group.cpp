@@ -94,7 +94,7 @@ int run_group(msf_ctx* c, std::vector<GroupRun>& runs, GroupInfo* info)
         s.v.twy = twy;
         // launch shape: the rules (the radix plans of a run on its own), one chain
         s.sh.plan_v = plan_choice(c->cfg, nx, ny, twx, twy);
-        s.sh.B = std::min<int64_t>(c->cfg.batch ? (int64_t)c->cfg.batch : batch_rule(s.f), s.f.P);
+        s.sh.B = std::min<int64_t>(c->cfg.batch ? (int64_t)c->cfg.batch : batch_rule(s.f, false), s.f.P);
         s.sh.n_batches = (s.f.P + s.sh.B - 1) / s.sh.B;
         s.sh.col_tile = c->cfg.col_tile;
         s.sh.chains = 1;

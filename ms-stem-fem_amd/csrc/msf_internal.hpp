@@ -495,8 +495,9 @@ int prepare_groups(msf_ctx* c, Mem& m, RunPlan& pl, const msf_specimen* sp, cons
 int prepare_vacuum(msf_ctx* c, Mem& m, RunPlan& pl, const msf_specimen* sp, const msf_optics* o,
                    const RunFlags& f);
 // positions per batch by the rule: the fewest batches whose wave buffer stays
-// within 96 MiB, in whole groups of 16 positions
-int64_t batch_rule(const RunFlags& f);
+// within 96 MiB, an even number of three or more where two chains of batches
+// share them (pairs)
+int64_t batch_rule(const RunFlags& f, bool pairs);
 // the context's second stream and the events that order two batch chains
 // (created on first use)
 int ensure_stream2(msf_ctx* c);

@@ -572,15 +572,30 @@ int tune_shape(msf_ctx* c, RunPlan& pl, const msf_specimen* sp, const std::vecto
                const RunFlags& f, const Twiddles& twx, const Twiddles& twy, int64_t B,
                int plan_rule, int all_alt, TunedShape& pick, int& state);
 
-int64_t batch_rule(const RunFlags& f)
+// Pixels of a launch from which two chains of batches are the rule.
+constexpr int64_t kTwoChainPixels = 4ll << 20;
+
+// Positions per batch: the fewest batches whose waves stay within 96 MiB,
+// spread evenly.  On grids from 384^2 two chains (pairs) share an even number
+// of three or more, or the last one's passes run alone.  20 slices of 512^2:
+// 192 positions 4.65 -> 4.42 ms (four batches of 48 for three of 64), 150
+// 3.78 -> 3.58, 300 7.15 -> 6.99; 1024^2, 40 positions 4.83 -> 4.52; 384^2,
+// 300 positions, 15 slices 3.46 -> 3.29.  At 256^2 the smaller launches cost
+// more (600 positions, 10 slices 1.69 -> 1.75).
+int64_t batch_rule(const RunFlags& f, bool pairs)
 {
     const int64_t P = f.P;
     const int64_t per_pos = f.plane * (int64_t)sizeof(float2);
     int64_t bmax = std::max<int64_t>(1, (96ll << 20) / per_pos);
     if (bmax >= 32) bmax -= bmax % 16; // whole groups of 16 positions per launch
-    const int64_t nbat = (P + bmax - 1) / bmax;
+    int64_t nbat = (P + bmax - 1) / bmax, step = 16;
+    const int64_t even = (P + nbat) / (nbat + 1); // positions per batch with one batch more
+    if (pairs && f.M >= 384 * 384 && nbat >= 3 && nbat % 2 && even * f.plane >= kTwoChainPixels) {
+        ++nbat;
+        if (even < 96) step = 8;
+    }
     int64_t B = (P + nbat - 1) / nbat;
-    if (B > 16 && B % 16) B = std::min<int64_t>(bmax, B + 16 - B % 16);
+    if (B > 16 && B % step) B = std::min<int64_t>(bmax, B + step - B % step);
     return std::max<int64_t>(1, std::min<int64_t>(B, P));
 }
 
@@ -601,7 +616,8 @@ int launch_shape(msf_ctx* c, Mem& m, RunPlan& pl, const msf_specimen* sp,
     // partial sums then stay resident in the 256 MB Infinity Cache across the
     // two passes of a slice (512^2: 64 positions per batch, measured best of
     // 64..256).
-    int64_t B = c->cfg.batch ? (int64_t)c->cfg.batch : batch_rule(f);
+    int64_t B = c->cfg.batch ? (int64_t)c->cfg.batch
+                             : batch_rule(f, c->cfg.chains != 1 && !c->cfg.profile_kernels && !m.scratch());
     B = std::max<int64_t>(1, std::min<int64_t>(B, P));
     sh.col_tile = c->cfg.col_tile;
     int chains_cfg = c->cfg.chains;
@@ -655,7 +671,7 @@ int launch_shape(msf_ctx* c, Mem& m, RunPlan& pl, const msf_specimen* sp,
     }
     sh.B = B;
     sh.n_batches = (P + B - 1) / B;
-    const bool big_launch = B * f.plane >= (4ll << 20);
+    const bool big_launch = B * f.plane >= kTwoChainPixels;
     const int chains_req = out.exit ? (chains_cfg == 1 ? 1 : 2)
                                     : (chains_cfg ? chains_cfg : (big_launch ? 2 : 1));
     // chains 3: batches in pairs on one stream, row and column passes of the
