@@ -127,7 +127,7 @@ __device__ __forceinline__ int div_by(uint32_t g, uint32_t d, uint32_t mul)
 // positions); at 1024 the larger LDS footprint costs more than it saves.
 template <int NY, int V> __host__ __device__ constexpr int row_threads()
 {
-    // the alternate 1024 plan (16 values on 64 lanes, ~120 registers): two
+    // the alternate 1024 plan (16 values on 64 lanes, 95 registers): two
     // rows per 128-lane workgroup, 71 us against 76 us on 256 lanes per 17
     // positions
     return (NY == 512 && V == 0) ? 512 : (NY == 1024 && V == 1) ? 128 : 256;
@@ -167,15 +167,19 @@ template <int NY, int V> __host__ __device__ constexpr int row_len()
     return P::T >= 16 ? P::kExchangeLen : (P::kExchangeLen + 7) / 16 * 16 + 8;
 }
 //
-// The row pass is bound by vector instructions (78-84 % of the cycles at 512
-// and 1024), so what is uniform or known at compile time stays out of the
-// vector unit: the workgroup's division, the row and u0 addresses (32-bit
-// offsets), the table staging in 16-byte words, the wrap of the shifted u0.
-// Together with transmit_point, and with every t and u0 read of a lane issued
-// before the first product, per pass: 128^2 39.4 -> 37.1 us (1024 positions),
-// 192^2 46.8 -> 43.9 (496), 256^2 40.1 -> 36.2 (272), 384^2 50.8 -> 47.4
-// (112), 512^2 41.5 -> 38.7 (64), 768^2 36.5 -> 32.5 (16), 1024^2 50.7 -> 50.1
-// (16; its tables come from L2, which bounds it now).
+// The row pass keeps the vector unit busy for 70 to 80 % of its time and
+// waits for the rest between load, transforms and store, so what is uniform or
+// known at compile time stays out of the vector unit: the workgroup's
+// division, the row and u0 addresses (a base per wavefront, the element in the
+// instruction), the table staging in 16-byte words, the wrap of the shifted
+// u0.  Together with transmit_point, and with every t and u0 read of a lane
+// issued before the first product, per pass, before and now: 128^2 39.4 ->
+// 37.1 us (1024 positions), 192^2 46.8 -> 40.0 (496), 256^2 40.1 -> 35.2
+// (272), 384^2 50.8 -> 42.9 (112), 512^2 41.5 -> 37.0 (64), 768^2 36.5 -> 29.9
+// (16), 1024^2 50.7 -> 47.9 (16; its tables come from L2, which bounds it).
+// Not kept: 16 rows per workgroup at 512 (37.9 -> 39.9), two positions per
+// wavefront with the next row prefetched (512 36.3 -> 38.8, 384 42 -> 46,
+// 1024 47.9 -> 49.7), for the registers or waves that they cost.
 template <int NY, int V, int RT> __host__ __device__ constexpr int row_smem_len()
 {
     return (row_is_lean<NY, V, RT>() ? 0 : plan_tw_len<PlanV<NY, V>>() + NY) +
@@ -332,9 +336,9 @@ template <int NX, int V = 0> struct ColTile {
     static constexpr int WMAX = 16;  // ncp is a multiple of this
     // default tile: keep LDS (W * lds_len * 8 B) near 40 KiB so that several
     // workgroups share a CU
-    // The alternate 1024 plan (16 values on 64 lanes, ~190 registers) fits
-    // one 8-column tile per CU; 4-column tiles with lean tables fit two
-    // (column pass 83 -> 74.5 us per 17 positions).
+    // The alternate 1024 plan (16 values on 64 lanes, 72 registers) fits two
+    // 8-column tiles per CU, and four 4-column tiles with lean tables, which
+    // are faster where no second chain runs beside them.
     static constexpr int W = (NX == 1024 && V == 1) ? 4 : (16 * lds_len(NX) * 8 > 48 * 1024) ? 8 : 16;
 };
 
