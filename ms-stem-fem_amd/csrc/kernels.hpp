@@ -131,6 +131,8 @@ bool stage_twiddles(int n, std::vector<double>& re_im, int v = 0);
 double fp32_gain(int n);
 // true when length n has an alternate radix plan for the slice passes
 bool has_alt_plan(int n);
+// positions that a row-pass workgroup of length ny and plan v holds
+int row_positions(int ny, int v);
 // the column count of the compact wave is padded to a multiple of this
 int col_tile(int nx);
 // the column-pass tile width used when none is configured, for plan v, alone

@@ -132,6 +132,22 @@ bool col_prunable(int nx, const int32_t* ab)
     return true;
 }
 
+int row_positions(int ny, int v)
+{
+    switch (ny) {
+#define MSF_CASE(N)                                                                                \
+    case N: {                                                                                      \
+        constexpr int A = AltPlan<N>::exists ? 1 : 0;                                              \
+        return v ? row_threads<N, A>() / PlanV<N, A>::T : row_threads<N, 0>() / PlanV<N, 0>::T;    \
+    }
+        MSF_CASE(16) MSF_CASE(32) MSF_CASE(64) MSF_CASE(96) MSF_CASE(128) MSF_CASE(192)
+        MSF_CASE(256) MSF_CASE(384) MSF_CASE(512) MSF_CASE(768) MSF_CASE(1024)
+#undef MSF_CASE
+    default:
+        return 1;
+    }
+}
+
 int col_tile(int nx)
 {
     switch (nx) {

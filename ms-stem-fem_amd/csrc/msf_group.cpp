@@ -94,8 +94,8 @@ int run_group(msf_ctx* c, std::vector<GroupRun>& runs, GroupInfo* info)
         s.v.twy = twy;
         // launch shape: the rules (the radix plans of a run on its own), one chain
         s.sh.plan_v = plan_choice(c->cfg, nx, ny, twx, twy);
-        s.sh.B = std::min<int64_t>(c->cfg.batch ? (int64_t)c->cfg.batch : batch_rule(s.f, false), s.f.P);
-        s.sh.n_batches = (s.f.P + s.sh.B - 1) / s.sh.B;
+        s.sh.split = c->cfg.batch ? msf::batches_of(s.f.P, (int64_t)c->cfg.batch)
+                                  : batch_rule(s.f, false, s.sh.plan_v);
         s.sh.col_tile = c->cfg.col_tile;
         s.sh.chains = 1;
         if (int rc = prepare_buffers(c, heap, pl, s.f, s.sh, g.shifts, g.out, s.v)) return rc;
@@ -113,8 +113,8 @@ int run_group(msf_ctx* c, std::vector<GroupRun>& runs, GroupInfo* info)
         Active a{};
         a.r = r;
         a.k = k;
-        a.b0 = k * s.sh.B;
-        a.nb = (int)std::min<int64_t>(s.sh.B, s.f.P - a.b0);
+        a.b0 = s.sh.split.begin(k);
+        a.nb = (int)(s.sh.split.begin(k + 1) - a.b0);
         a.n = 0;
         s.pa.bind(s.v.psi[0], s.v.shift + a.b0, a.nb, a.ra, a.ca);
         act.push_back(a);
@@ -211,7 +211,7 @@ int run_group(msf_ctx* c, std::vector<GroupRun>& runs, GroupInfo* info)
             rc = enqueue_batch_tail(c, *c->gplans[(size_t)a.r], g.sp, s.f, s.v, g.out, prof, 1, a.k,
                                     a.b0, a.nb, 0, st);
             if (rc != MSF_OK) break;
-            if (a.k + 1 < s.sh.n_batches) start(a.r, a.k + 1);
+            if (a.k + 1 < s.sh.split.n) start(a.r, a.k + 1);
         }
     }
     for (hipStream_t q : {su, st}) {

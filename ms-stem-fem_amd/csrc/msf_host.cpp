@@ -430,4 +430,38 @@ SegmentTiles build_segments(const Groups& g, int seg)
     return t;
 }
 
+BatchSplit batches_of(int64_t P, int64_t depth)
+{
+    BatchSplit s;
+    s.P = P;
+    s.depth = std::max<int64_t>(1, std::min(depth, P));
+    s.n = (P + s.depth - 1) / s.depth;
+    return s;
+}
+
+BatchSplit batch_rule(int64_t P, int64_t plane, int64_t pixels, bool pairs, int unit)
+{
+    const int64_t per_pos = plane * 8;
+    int64_t bmax = std::max<int64_t>(1, (96ll << 20) / per_pos);
+    if (bmax >= 32) bmax -= bmax % 16; // whole groups of 16 positions per launch
+    const int64_t few = (P + bmax - 1) / bmax;
+    if (pairs && pixels >= 384 * 384 && few >= 3 && few % 2 &&
+        (P + few) / (few + 1) * plane >= kTwoChainPixels) {
+        BatchSplit s;
+        s.P = P;
+        s.n = few + 1;
+        // whole units may not fit the room, or leave a last batch of less
+        // than half the first: halve them
+        for (s.unit = unit; s.unit >= 1; s.unit /= 2) {
+            const int64_t units = (P + s.unit - 1) / s.unit;
+            s.depth = (units + s.n - 1) / s.n * s.unit;
+            if (s.depth <= bmax && units >= s.n && 2 * (P - s.begin(s.n - 1)) >= s.depth) break;
+        }
+        return s;
+    }
+    int64_t B = (P + few - 1) / few;
+    if (B > 16 && B % 16) B = std::min<int64_t>(bmax, B + 16 - B % 16);
+    return batches_of(P, B);
+}
+
 } // namespace msf

@@ -166,4 +166,28 @@ struct SegmentTiles {
 };
 SegmentTiles build_segments(const Groups& g, int seg);
 
+// A run's positions in n batches of at most `depth`, in raster order: batch k
+// holds positions [begin(k), begin(k + 1)).  unit 0: batches of `depth`, what
+// is left in the last; else whole units of that many positions, shared so
+// that batches differ by one unit (the last unit may be a partial one).
+struct BatchSplit {
+    int64_t P = 0, depth = 1, n = 1, unit = 0;
+    int64_t begin(int64_t k) const
+    {
+        if (unit == 0) return k * depth < P ? k * depth : P;
+        const int64_t units = (P + unit - 1) / unit, q = units / n, r = units % n;
+        const int64_t b = unit * (k * q + (k < r ? k : r));
+        return b < P ? b : P;
+    }
+};
+// batches of `depth` positions
+BatchSplit batches_of(int64_t P, int64_t depth);
+// The rule, for waves of `plane` stored values on a grid of `pixels`: the
+// fewest batches whose waves stay within 96 MiB, spread evenly; with pairs
+// (two chains of batches) an even number of three or more, in units of the
+// positions that a row-pass workgroup holds.
+BatchSplit batch_rule(int64_t P, int64_t plane, int64_t pixels, bool pairs, int unit);
+// Pixels of a launch from which two chains of batches are the rule.
+constexpr int64_t kTwoChainPixels = 4ll << 20;
+
 } // namespace msf

@@ -411,7 +411,7 @@ struct RunFlags {
 
 // Launch shape of one run.
 struct Shape {
-    int64_t B = 1, n_batches = 1;
+    msf::BatchSplit split;   // its depth sizes the batch buffers
     int col_tile = 0;        // configured tile, 0: the plan's default
     int chains = 1;
     int plan_v = 0;          // radix plans, vx + 2 vy
@@ -494,10 +494,8 @@ int prepare_groups(msf_ctx* c, Mem& m, RunPlan& pl, const msf_specimen* sp, cons
                    const msf_detector* det, const msf_fem* fem, RunFlags& f);
 int prepare_vacuum(msf_ctx* c, Mem& m, RunPlan& pl, const msf_specimen* sp, const msf_optics* o,
                    const RunFlags& f);
-// positions per batch by the rule: the fewest batches whose wave buffer stays
-// within 96 MiB, an even number of three or more where two chains of batches
-// share them (pairs)
-int64_t batch_rule(const RunFlags& f, bool pairs);
+// the run's batches by the rule (msf::batch_rule), with pairs for two chains of them
+msf::BatchSplit batch_rule(const RunFlags& f, bool pairs, int plan_v);
 // the context's second stream and the events that order two batch chains
 // (created on first use)
 int ensure_stream2(msf_ctx* c);

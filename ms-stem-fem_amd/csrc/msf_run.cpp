@@ -572,31 +572,20 @@ int tune_shape(msf_ctx* c, RunPlan& pl, const msf_specimen* sp, const std::vecto
                const RunFlags& f, const Twiddles& twx, const Twiddles& twy, int64_t B,
                int plan_rule, int all_alt, TunedShape& pick, int& state);
 
-// Pixels of a launch from which two chains of batches are the rule.
-constexpr int64_t kTwoChainPixels = 4ll << 20;
-
-// Positions per batch: the fewest batches whose waves stay within 96 MiB,
-// spread evenly.  On grids from 384^2 two chains (pairs) share an even number
-// of three or more, or the last one's passes run alone.  20 slices of 512^2:
-// 192 positions 4.65 -> 4.42 ms (four batches of 48 for three of 64), 150
-// 3.78 -> 3.58, 300 7.15 -> 6.99; 1024^2, 40 positions 4.83 -> 4.52; 384^2,
-// 300 positions, 15 slices 3.46 -> 3.29.  At 256^2 the smaller launches cost
-// more (600 positions, 10 slices 1.69 -> 1.75).
-int64_t batch_rule(const RunFlags& f, bool pairs)
+// Two chains (pairs) share an even number of three or more batches on grids
+// from 384^2, or the last one's passes run alone.  The batches are whole
+// row-pass workgroups and differ by one and a partial one at most: batches of
+// one rounded size end in an odd number again or in a remainder that fills no
+// CU.  12 slices, the fewest batches / one more of one rounded size / this
+// split, ms: 768^2 65 positions 2.94 / 2.82 (24, 24, 17) / 2.60 (20, 16, 16,
+// 13), 73 positions 3.07 / 3.03 (24, 24, 24, 1) / 2.82, 157 6.17 / 6.13 / 5.93;
+// 512^2 150 2.24 / 2.18 / 2.17, 385 5.34 / 5.36 (seven of 56) / 5.30; 384^2 300
+// 2.79 / 2.65 / 2.68, 769 6.73 / 6.73 / 6.54; 1024^2 (10 slices) 40 2.41 / 2.35 /
+// 2.33.  At 256^2 the smaller launches cost more (600 positions, 10 slices
+// 1.69 -> 1.75).
+msf::BatchSplit batch_rule(const RunFlags& f, bool pairs, int plan_v)
 {
-    const int64_t P = f.P;
-    const int64_t per_pos = f.plane * (int64_t)sizeof(float2);
-    int64_t bmax = std::max<int64_t>(1, (96ll << 20) / per_pos);
-    if (bmax >= 32) bmax -= bmax % 16; // whole groups of 16 positions per launch
-    int64_t nbat = (P + bmax - 1) / bmax, step = 16;
-    const int64_t even = (P + nbat) / (nbat + 1); // positions per batch with one batch more
-    if (pairs && f.M >= 384 * 384 && nbat >= 3 && nbat % 2 && even * f.plane >= kTwoChainPixels) {
-        ++nbat;
-        if (even < 96) step = 8;
-    }
-    int64_t B = (P + nbat - 1) / nbat;
-    if (B > 16 && B % step) B = std::min<int64_t>(bmax, B + step - B % step);
-    return std::max<int64_t>(1, std::min<int64_t>(B, P));
+    return msf::batch_rule(f.P, f.plane, f.M, pairs, msf::row_positions(f.ny, (plan_v >> 1) & 1));
 }
 
 // Batch depth, column tile, chains and radix plans: configured, by the rules
@@ -616,9 +605,10 @@ int launch_shape(msf_ctx* c, Mem& m, RunPlan& pl, const msf_specimen* sp,
     // partial sums then stay resident in the 256 MB Infinity Cache across the
     // two passes of a slice (512^2: 64 positions per batch, measured best of
     // 64..256).
-    int64_t B = c->cfg.batch ? (int64_t)c->cfg.batch
-                             : batch_rule(f, c->cfg.chains != 1 && !c->cfg.profile_kernels && !m.scratch());
-    B = std::max<int64_t>(1, std::min<int64_t>(B, P));
+    const msf::BatchSplit rule =
+        c->cfg.batch ? msf::batches_of(P, (int64_t)c->cfg.batch)
+                     : batch_rule(f, c->cfg.chains != 1 && !c->cfg.profile_kernels && !m.scratch(), plan_rule);
+    int64_t B = rule.depth;
     sh.col_tile = c->cfg.col_tile;
     int chains_cfg = c->cfg.chains;
     sh.plan_v = plan_rule;
@@ -669,16 +659,17 @@ int launch_shape(msf_ctx* c, Mem& m, RunPlan& pl, const msf_specimen* sp,
                             "msf_run_stem, or fewer positions, slices or a smaller grid");
         if (B > bfit) B = bfit;
     }
-    sh.B = B;
-    sh.n_batches = (P + B - 1) / B;
-    const bool big_launch = B * f.plane >= kTwoChainPixels;
+    // a depth from the tuning table or the scratch region has its own count
+    sh.split = B == rule.depth ? rule : msf::batches_of(P, B);
+    const bool big_launch = B * f.plane >= msf::kTwoChainPixels;
     const int chains_req = out.exit ? (chains_cfg == 1 ? 1 : 2)
                                     : (chains_cfg ? chains_cfg : (big_launch ? 2 : 1));
     // chains 3: batches in pairs on one stream, row and column passes of the
     // pair's two batches fused into one launch per step
-    sh.chains = (chains_req >= 2 && sh.n_batches >= 2 && !prof && !m.scratch())
+    sh.chains = (chains_req >= 2 && sh.split.n >= 2 && !prof && !m.scratch())
                     ? chains_req
                     : 1;
+    if (sh.chains == 1) sh.split = msf::batches_of(P, B);
     sh.auto_eager = c->cfg.chains == 0 && sh.chains == 2;
     return MSF_OK;
 }
@@ -696,7 +687,7 @@ int ensure_stream2(msf_ctx* c)
 int prepare_buffers(msf_ctx* c, Mem& m, RunPlan& pl, const RunFlags& f, const Shape& sh,
                     const std::vector<int2>& shifts, const RunOut& out, RunViews& v)
 {
-    const int64_t B = sh.B, P = f.P;
+    const int64_t B = sh.split.depth, P = f.P;
     const int nbins = pl.nbins;
     if (B > pl.cap_b) { // sizes depend on G, which changes with the groups
         for (int k = 0; k < 2; ++k)
@@ -881,7 +872,8 @@ int enqueue_job(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, const Run
                 const Shape& sh, const RunViews& v, const RunOut& out, Prof& prof)
 {
     const int nx = f.nx, ny = f.ny, S = f.S;
-    const int64_t P = f.P, B = sh.B;
+    const int64_t P = f.P;
+    const msf::BatchSplit& split = sh.split;
     const int chains = sh.chains;
     const PassArgs pa = pass_args(pl, sp, f, sh, v);
     hipStream_t streams[2] = {c->stream, c->stream2};
@@ -931,10 +923,9 @@ int enqueue_job(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, const Run
             }
             return MSF_OK;
         };
-        int64_t k = 0;
-        for (int64_t b0 = 0; b0 < P;) {
-            const int nbA = (int)std::min<int64_t>(B, P - b0);
-            const int64_t b1 = b0 + nbA;
+        for (int64_t k = 0; k < split.n; k += 2) {
+            const int64_t b0 = split.begin(k), b1 = split.begin(k + 1);
+            const int nbA = (int)(b1 - b0);
             msf::RowPassArgs rA, rB;
             msf::ColPassArgs cA, cB;
             bind(b0, nbA, 0, rA, cA);
@@ -943,7 +934,7 @@ int enqueue_job(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, const Run
                 if (int r = finish_batch(k, b0, nbA, 0, s)) return r;
                 break;
             }
-            const int nbB = (int)std::min<int64_t>(B, P - b1);
+            const int nbB = (int)(split.begin(k + 2) - b1);
             bind(b1, nbB, 1, rB, cB);
             row_at(rA, 0);
             HIPCHK(c, msf::launch_row_pass(ny, true, f.tmode, rA, s));
@@ -961,8 +952,6 @@ int enqueue_job(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, const Run
             }
             if (int r = finish_batch(k, b0, nbA, 0, s)) return r;
             if (int r = finish_batch(k + 1, b1, nbB, 1, s)) return r;
-            k += 2;
-            b0 = b1 + nbB;
         }
         return MSF_OK;
     }
@@ -983,9 +972,9 @@ int enqueue_job(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, const Run
         return copy_exit_waves(c, v.psi[b.ch], nx, ny, f.ncp, f.ka, f.kb, b.nb, streams[b.ch],
                                out.exit + (size_t)b.b0 * nx * ny * 2);
     };
-    int64_t k = 0;
-    for (int64_t b0 = 0; b0 < P; b0 += B, ++k) {
-        const int nb = (int)std::min<int64_t>(B, P - b0);
+    for (int64_t k = 0; k < split.n; ++k) {
+        const int64_t b0 = split.begin(k);
+        const int nb = (int)(split.begin(k + 1) - b0);
         const int ch = (int)(k % chains);
         hipStream_t s = streams[ch];
         msf::RowPassArgs r;
@@ -1013,7 +1002,7 @@ std::vector<uint64_t> graph_signature(const RunPlan& pl, const msf_specimen* sp,
                                       const Shape& sh, const RunViews& v, const RunOut& out)
 {
     auto u = [](const void* p) { return (uint64_t)(uintptr_t)p; };
-    return {sp->id, (uint64_t)f.P, (uint64_t)sh.B, (uint64_t)f.tmode, (uint64_t)f.want_adf,
+    return {sp->id, (uint64_t)f.P, (uint64_t)sh.split.depth, (uint64_t)sh.split.n, (uint64_t)sh.split.unit, (uint64_t)f.tmode, (uint64_t)f.want_adf,
             (uint64_t)f.want_d1 | (uint64_t)f.want_d2 << 1 | (uint64_t)f.want_pix << 2 |
                 (uint64_t)f.want_corr << 3,
             u(v.csum), u(v.csqr), (uint64_t)f.nphi, (uint64_t)pl.hg.corr, (uint64_t)f.want_mtf,
@@ -1093,14 +1082,13 @@ int tune_shape(msf_ctx* c, RunPlan& pl, const msf_specimen* sp, const std::vecto
     HIPCHK(c, hipEventCreate(&e1.e));
     const TrialFn trial = [&](const TunedShape& cand, double& cost) -> int {
         Shape ts;
-        ts.B = cand[0];
         ts.col_tile = cand[1];
         ts.chains = cand[2];
         ts.plan_v = cand[3];
         RunFlags ft = f;
-        ft.P = std::min<int64_t>(P, 4 * ts.B);
+        ft.P = std::min<int64_t>(P, 4 * (int64_t)cand[0]);
         ft.want_each = false;
-        ts.n_batches = (ft.P + ts.B - 1) / ts.B;
+        ts.split = msf::batches_of(ft.P, cand[0]);
         const std::vector<int2> sub(shifts.begin(), shifts.begin() + ft.P);
         RunViews tv;
         tv.twx = twx;
@@ -1237,16 +1225,16 @@ int run_internal(msf_ctx* c, Mem& m, const msf_specimen* sp, const msf_optics* o
     st.slice_loop_ms = t_end - t_loop;
     st.total_ms = now_ms() - t_start;
     st.probe_slices = (uint64_t)f.P * (uint64_t)f.S;
-    st.batch = (uint32_t)sh.B;
-    st.n_batches = (uint32_t)sh.n_batches;
+    st.batch = (uint32_t)sh.split.depth;
+    st.n_batches = (uint32_t)sh.split.n;
     // compulsory traffic of a full-batch pass: read + write of the compact wave
-    st.row_pass_bytes = 2.0 * (double)sh.B * f.nx * (f.ka + f.kb) * sizeof(float2);
+    st.row_pass_bytes = 2.0 * (double)sh.split.depth * f.nx * (f.ka + f.kb) * sizeof(float2);
     st.col_pass_bytes = st.row_pass_bytes;
     st.graph = graph_state;
     st.chains = sh.chains;
     st.fused_launches = prof.fused;
     st.col_tile = sh.col_tile ? sh.col_tile
-                              : msf::col_tile_auto(f.nx, sh.plan_v & 1, (int)sh.B, f.ncp,
+                              : msf::col_tile_auto(f.nx, sh.plan_v & 1, (int)sh.split.depth, f.ncp,
                                                    sh.chains == 2);
     st.autotuned = sh.tuned_state;
     st.row_fft_plan = 1 + ((sh.plan_v >> 1) & 1);
