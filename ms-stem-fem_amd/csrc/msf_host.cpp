@@ -70,12 +70,22 @@ std::vector<double> pow2_all(const std::vector<double>& k)
     return out;
 }
 
+// squares of frequencies in FFT order: rising over the low half, falling over
+// the high one (false for NaN)
+static bool fft_ordered(const std::vector<double>& k2)
+{
+    const size_t n = k2.size(), h = n / 2;
+    for (size_t j = 1; j < n; ++j)
+        if (j != h && !(j < h ? k2[j] >= k2[j - 1] : k2[j] <= k2[j - 1])) return false;
+    return true;
+}
+
 RowRanges slice_keep_ranges(const Domain& d)
 {
     const double c_bw = ref_pow2(d.bw_t);   // bw_limit.cpp:36
     const double c_pr = d.bw_t * d.bw_t;     // slice.cpp:1375
     const std::vector<double> kx2 = pow2_all(d.kx), ky2 = pow2_all(d.ky);
-    return row_ranges(d.nx, d.ny, [&](int i, int j) {
+    return row_ranges(d.nx, d.ny, fft_ordered(ky2), [&](int i, int j) {
         const double k2 = kx2[i] + ky2[j];
         return !(k2 >= c_bw) && (k2 < c_pr);
     });
@@ -85,7 +95,17 @@ RowRanges column_keep_ranges(const RowRanges& rows, int nx, int ny, int ncp)
 {
     const int ka = rows.amax, kb = rows.bmax, nc = ka + kb;
     auto kept = [&](int i, int j) { return j < rows.ab[2 * i] || j >= ny - rows.ab[2 * i + 1]; };
-    return row_ranges(ncp, nx, [&](int jc, int i) {
+    // a whole row is (ny, 0): all of both halves
+    const int h = ny / 2;
+    auto low = [&](int i) { return std::min(rows.ab[2 * i], h); };
+    auto high = [&](int i) { return rows.ab[2 * i] == ny ? h : rows.ab[2 * i + 1]; };
+    bool ordered = true;
+    for (int i = 1; i < nx; ++i) {
+        const int da = low(i) - low(i - 1), db = high(i) - high(i - 1);
+        if (i < nx / 2) ordered = ordered && da <= 0 && db <= 0;
+        else if (i > nx / 2) ordered = ordered && da >= 0 && db >= 0;
+    }
+    return row_ranges(ncp, nx, ordered, [&](int jc, int i) {
         return jc < nc && kept(i, jc < ka ? jc : jc - nc + ny);
     });
 }
@@ -94,22 +114,26 @@ RowRanges bwlimit_keep_ranges(const Domain& d)
 {
     const double c_bw = ref_pow2(d.bw_t);
     const std::vector<double> kx2 = pow2_all(d.kx), ky2 = pow2_all(d.ky);
-    return row_ranges(d.nx, d.ny, [&](int i, int j) { return !(kx2[i] + ky2[j] >= c_bw); });
+    return row_ranges(d.nx, d.ny, fft_ordered(ky2),
+                      [&](int i, int j) { return !(kx2[i] + ky2[j] >= c_bw); });
 }
 
 RowRanges template_keep_ranges(const Domain& d)
 {
     const double c2 = d.bw_pap * d.bw_pap; // scatterer_pap.hpp:82
     const std::vector<double> kx2 = pow2_all(d.kx), ky2 = pow2_all(d.ky);
-    return row_ranges(d.nx, d.ny, [&](int i, int j) { return kx2[i] + ky2[j] < c2; });
+    return row_ranges(d.nx, d.ny, fft_ordered(ky2),
+                      [&](int i, int j) { return kx2[i] + ky2[j] < c2; });
 }
 
 RowRanges aperture_keep_ranges(const Domain& d, double alpha_max)
 {
     const double l2 = d.lambda * d.lambda;      // adfstem.cpp:95
     const double a2 = alpha_max * alpha_max;    // adfstem.cpp:96
-    return row_ranges(d.nx, d.ny, [&](int i, int j) {
-        const double ksqr = d.kx[i] * d.kx[i] + d.ky[j] * d.ky[j];
+    std::vector<double> ky2(d.ky);
+    for (double& k : ky2) k *= k;
+    return row_ranges(d.nx, d.ny, fft_ordered(ky2), [&](int i, int j) {
+        const double ksqr = d.kx[i] * d.kx[i] + ky2[j];
         return l2 * ksqr < a2;
     });
 }

@@ -38,8 +38,8 @@ Domain make_domain(int nx, int ny, double xperiod, double yperiod, double xmin, 
                    double voltage);
 
 // Row-wise membership of a disk-like pixel set in FFT order: for row i the
-// kept columns are [0, a_i) U [ny - b_i, ny); ok == false if a set is not of
-// that form.
+// kept columns are [0, a_i) U [ny - b_i, ny); ok == false if a set is not
+// known to be of that form (the ranges then are not used).
 struct RowRanges {
     std::vector<int32_t> ab; // 2*nx: a_i, b_i
     int amax = 0, bmax = 0;  // union over rows
@@ -48,10 +48,12 @@ struct RowRanges {
 // keep(i, j) holds from j = 0 up to some j and from some j on to ny - 1 when
 // it tests a rounded sum that grows with |k_y|: k_y rises over [0, ny/2) and
 // -k_y falls over [ny/2, ny), and IEEE rounding is monotone.  A bisection of
-// each half then finds the same ranges as a test of every pixel.
-template <typename Pred> RowRanges row_ranges(int nx, int ny, Pred keep)
+// each half then finds the same ranges as a test of every pixel.  `ordered`
+// says that this holds (a bisection cannot tell).
+template <typename Pred> RowRanges row_ranges(int nx, int ny, bool ordered, Pred keep)
 {
     RowRanges r;
+    r.ok = ordered;
     r.ab.assign(2 * (size_t)nx, 0);
     const int h = ny / 2;
     for (int i = 0; i < nx; ++i) {
@@ -86,8 +88,9 @@ RowRanges slice_keep_ranges(const Domain& d);
 // The same kept set by column of the compact plane [nx][ncp] (compact
 // column jc holds full column j = jc < ka ? jc : jc - (ka + kb) + ny): the
 // kept rows of column jc are [0, c) U [nx - d, nx), returned as (c, d) pairs
-// (2*ncp entries; padding columns keep nothing).  ok == false if a column is
-// not of that form; the pairs then are not used.
+// (2*ncp entries; padding columns keep nothing).  ok == false unless the rows'
+// ranges shrink over i < nx/2 and grow from there on, which makes every column
+// of that form.
 RowRanges column_keep_ranges(const RowRanges& rows, int nx, int ny, int ncp);
 
 // bw_limit.cpp:30-47 alone (transmission band limit, slice.cpp:1731-1737)
