@@ -488,4 +488,30 @@ BatchSplit batch_rule(int64_t P, int64_t plane, int64_t pixels, bool pairs, int 
     return batches_of(P, B);
 }
 
+TunedShape tune_rule(const TuneSpace& t)
+{
+    const bool two = t.B * t.plane >= kTwoChainPixels && t.B < t.P;
+    return {(int)t.B, t.tile(t.B, t.plans[0], two), two ? 2 : 1, t.plans[0]};
+}
+
+std::vector<TunedShape> tune_candidates(const TuneSpace& t)
+{
+    std::vector<int64_t> bs = {t.B};
+    for (int64_t b : {t.B / 2, 2 * t.B}) {
+        if (t.B >= 32) b -= b % 16;
+        if (b >= 1 && b <= t.P && std::find(bs.begin(), bs.end(), b) == bs.end()) bs.push_back(b);
+    }
+    std::vector<TunedShape> c;
+    for (int pv : t.plans)
+        for (int64_t b : bs)
+            for (int ch : {1, 2, 3}) {
+                if (ch > 1 && b >= t.P) continue; // one batch
+                for (int w : {4, 8, 16})
+                    if (ch < 3 || t.fused(w, pv)) c.push_back({(int)b, w, ch, pv});
+            }
+    const TunedShape rule = tune_rule(t);
+    if (std::find(c.begin(), c.end(), rule) == c.end()) c.push_back(rule);
+    return c;
+}
+
 } // namespace msf

@@ -8,7 +8,9 @@
 // kernels only ever consume integer index data and never decide membership
 // in FP32.
 #pragma once
+#include <array>
 #include <cstdint>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -192,5 +194,22 @@ BatchSplit batches_of(int64_t P, int64_t depth);
 BatchSplit batch_rule(int64_t P, int64_t plane, int64_t pixels, bool pairs, int unit);
 // Pixels of a launch from which two chains of batches are the rule.
 constexpr int64_t kTwoChainPixels = 4ll << 20;
+
+// Launch shapes of the autotuner: batch, column tile, chains, radix plans
+// (vx + 2 vy).
+using TunedShape = std::array<int, 4>;
+struct TuneSpace {
+    int64_t P = 0, B = 0;       // positions; batch depth by the rule
+    int64_t plane = 0;          // stored values of a wave
+    std::vector<int> plans;     // the rule's first
+    std::function<int(int64_t b, int plans, bool beside)> tile; // the automatic tile of a batch
+    std::function<bool(int tile, int plans)> fused;  // chains 3 fuse their passes
+};
+// the shape a run of the rules takes
+TunedShape tune_rule(const TuneSpace& t);
+// The shapes to time: the rule's batch depth, half and twice it; column tiles
+// 4, 8 and 16; one chain, two chains, or fused batch pairs; and the rule's own
+// shape.
+std::vector<TunedShape> tune_candidates(const TuneSpace& t);
 
 } // namespace msf

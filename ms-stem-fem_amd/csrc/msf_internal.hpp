@@ -239,7 +239,7 @@ struct ServeState {
 // Launch shape of a run: positions per batch, column-pass tile, batch
 // chains in flight and the radix plans (vx + 2 vy, per axis 0 primary,
 // 1 alternate).
-using TunedShape = std::array<int, 4>;       // batch, col_tile, chains, plan
+using TunedShape = msf::TunedShape;
 // msf_config.autotune of served jobs: the tuning table's choices, no trials
 constexpr int32_t kAutotuneLookup = 2;
 

@@ -568,6 +568,28 @@ int64_t chain_bytes_per_position(const RunPlan& pl, const RunFlags& f)
 // batch steps.
 constexpr int64_t kTuneMinWork = 16384;
 
+// square grids whose slice passes can run as fused pass pairs (chains 3)
+static bool fused_shape(const RunFlags& f, int tile, int plan_v)
+{
+    return f.nx == f.ny && msf::fused_shape_ok(f.nx, (plan_v >> 1) & 1, plan_v & 1, tile) &&
+           msf::row_prunable(f.ny, f.ka, f.kb);
+}
+
+// what the tuner chooses among, for batches of B by the rule
+static msf::TuneSpace tune_space(const RunFlags& f, int64_t B, const std::vector<int>& plans)
+{
+    msf::TuneSpace t;
+    t.P = f.P;
+    t.B = B;
+    t.plane = f.plane;
+    t.plans = plans;
+    t.tile = [&f](int64_t b, int pv, bool beside) {
+        return msf::col_tile_auto(f.nx, pv & 1, (int)b, f.ncp, beside);
+    };
+    t.fused = [&f](int tile, int pv) { return fused_shape(f, tile, pv); };
+    return t;
+}
+
 int tune_shape(msf_ctx* c, RunPlan& pl, const msf_specimen* sp, const std::vector<int2>& shifts,
                const RunFlags& f, const Twiddles& twx, const Twiddles& twy, int64_t B,
                int plan_rule, int all_alt, TunedShape& pick, int& state);
@@ -630,9 +652,13 @@ int launch_shape(msf_ctx* c, Mem& m, RunPlan& pl, const msf_specimen* sp,
                                sh.tuned_state))
             return r;
         B = std::min<int64_t>(pick[0], P);
-        sh.col_tile = pick[1];
         chains_cfg = pick[2];
         sh.plan_v = pick[3];
+        // a tile that is the automatic one stays automatic, so that a smaller
+        // last batch has its own
+        const msf::TuneSpace t = tune_space(f, B, {sh.plan_v});
+        const bool own = chains_cfg < 3 && t.tile(B, sh.plan_v, chains_cfg == 2) == pick[1];
+        sh.col_tile = own ? 0 : pick[1];
     }
     // Two chains of batches in flight on two streams: the row passes (VALU
     // bound) of one chain overlap the column passes (memory bound) of the
@@ -1018,23 +1044,13 @@ std::vector<uint64_t> graph_signature(const RunPlan& pl, const msf_specimen* sp,
             (uint64_t)pl.nbins, (uint64_t)pl.n_tiles, (uint64_t)sh.col_tile, (uint64_t)sh.plan_v};
 }
 
-// square grids whose slice passes can run as fused pass pairs (chains 3)
-static bool fused_shape(const RunFlags& f, int tile, int plan_v)
-{
-    return f.nx == f.ny && msf::fused_shape_ok(f.nx, (plan_v >> 1) & 1, plan_v & 1, tile) &&
-           msf::row_prunable(f.ny, f.ka, f.kb);
-}
-
-// The autotuner's candidates and trials.  A trial runs the job's own launch
-// sequence (enqueue_job: both slice passes of every slice, the reductions and
-// FEM statistics, with the candidate's chains) over the first four batches
-// of the job's positions on trial buffers, once untimed and once timed; its
-// cost is seconds per position-slice.  Candidates: the rule's batch depth,
-// half and twice it; column tiles 4, 8 and 16; one chain, two chains, or
-// batch pairs with fused pass launches where the grid has them; with
-// autotune = 1 and fft_plan = 0 also the all-primary and all-alternate radix
-// plans.  Every candidate of one radix plan gives bit-identical results.
-
+// The autotuner's trials of its candidates (msf::tune_candidates).  A trial
+// runs the job's own launch sequence (enqueue_job: both slice passes of every
+// slice, the reductions and FEM statistics, with the candidate's chains) over
+// the first four batches of the job's positions on trial buffers, once untimed
+// and once timed; its cost is seconds per position-slice.  With autotune = 1
+// and fft_plan = 0 the candidates include the all-primary and all-alternate
+// radix plans; every candidate of one radix plan gives bit-identical results.
 int tune_shape(msf_ctx* c, RunPlan& pl, const msf_specimen* sp, const std::vector<int2>& shifts,
                const RunFlags& f, const Twiddles& twx, const Twiddles& twy, int64_t B,
                int plan_rule, int all_alt, TunedShape& pick, int& state)
@@ -1048,25 +1064,13 @@ int tune_shape(msf_ctx* c, RunPlan& pl, const msf_specimen* sp, const std::vecto
         << " " << (f.want_adf ? "a" : "") << (f.want_d1 ? "v" : "") << (f.want_d2 ? "b" : "")
         << (f.want_pix ? "p" : "") << (f.want_corr ? "c" : "") << (f.want_mtf ? "m" : "") << "-"
         << " " << (plans ? "plans" : "plan" + std::to_string(plan_rule));
-    const int ch0 = (B * f.plane >= (4ll << 20) && (P + B - 1) / B >= 2) ? 2 : 1;
-    const int tile0 = msf::col_tile_default(f.nx, plan_rule & 1, ch0 == 2);
-    const TunedShape rule = {(int)B, tile0, ch0, plan_rule};
-    std::vector<int64_t> bs = {B};
-    for (int64_t b : {B / 2, 2 * B}) {
-        if (B >= 32) b -= b % 16;
-        if (b >= 1 && b <= P && std::find(bs.begin(), bs.end(), b) == bs.end()) bs.push_back(b);
-    }
     std::vector<int> pvs = {plan_rule};
     if (plans)
         for (int pv : {0, all_alt})
             if (std::find(pvs.begin(), pvs.end(), pv) == pvs.end()) pvs.push_back(pv);
-    std::vector<TunedShape> cands;
-    for (int pv : pvs)
-        for (int64_t b : bs)
-            for (int w : {4, 8, 16})
-                for (int ch : {1, 2, 3})
-                    if (ch == 1 || ((P + b - 1) / b >= 2 && (ch == 2 || fused_shape(f, w, pv))))
-                        cands.push_back({(int)b, w, ch, pv});
+    const msf::TuneSpace space = tune_space(f, B, pvs);
+    const TunedShape rule = msf::tune_rule(space);
+    const std::vector<TunedShape> cands = msf::tune_candidates(space);
     RunPlan tb; // trial buffers, released on return
     tb.G = pl.G;
     tb.nbins = pl.nbins;
