@@ -506,7 +506,9 @@ std::vector<TunedShape> tune_candidates(const TuneSpace& t)
         for (int64_t b : bs)
             for (int ch : {1, 2, 3}) {
                 if (ch > 1 && b >= t.P) continue; // one batch
-                for (int w : {4, 8, 16})
+                std::vector<int> tiles = {4, 8, 16};
+                if (t.loop && t.loop(b, pv)) tiles = {t.tile(b, pv, ch == 2)};
+                for (int w : tiles)
                     if (ch < 3 || t.fused(w, pv)) c.push_back({(int)b, w, ch, pv});
             }
     const TunedShape rule = tune_rule(t);

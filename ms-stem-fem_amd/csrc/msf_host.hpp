@@ -203,13 +203,15 @@ struct TuneSpace {
     int64_t plane = 0;          // stored values of a wave
     std::vector<int> plans;     // the rule's first
     std::function<int(int64_t b, int plans, bool beside)> tile; // the automatic tile of a batch
+    std::function<bool(int64_t b, int plans)> loop;  // a batch takes the one-launch slice loop (null: none does)
     std::function<bool(int tile, int plans)> fused;  // chains 3 fuse their passes
 };
 // the shape a run of the rules takes
 TunedShape tune_rule(const TuneSpace& t);
 // The shapes to time: the rule's batch depth, half and twice it; column tiles
-// 4, 8 and 16; one chain, two chains, or fused batch pairs; and the rule's own
-// shape.
+// 4, 8 and 16, or where the slice loop runs in one launch, which has no tiles,
+// the automatic one; one chain, two chains, or fused batch pairs; and the
+// rule's own shape.
 std::vector<TunedShape> tune_candidates(const TuneSpace& t);
 
 } // namespace msf

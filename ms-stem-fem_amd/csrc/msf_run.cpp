@@ -576,7 +576,8 @@ static bool fused_shape(const RunFlags& f, int tile, int plan_v)
 }
 
 // what the tuner chooses among, for batches of B by the rule
-static msf::TuneSpace tune_space(const RunFlags& f, int64_t B, const std::vector<int>& plans)
+static msf::TuneSpace tune_space(const msf_specimen* sp, const RunFlags& f, int64_t B,
+                                 const std::vector<int>& plans)
 {
     msf::TuneSpace t;
     t.P = f.P;
@@ -585,6 +586,16 @@ static msf::TuneSpace tune_space(const RunFlags& f, int64_t B, const std::vector
     t.plans = plans;
     t.tile = [&f](int64_t b, int pv, bool beside) {
         return msf::col_tile_auto(f.nx, pv & 1, (int)b, f.ncp, beside);
+    };
+    t.loop = [&f, sp](int64_t b, int pv) {
+        msf::RowPassArgs r{};
+        msf::ColPassArgs cc{};
+        r.batch = (int)b;
+        r.plan = (pv >> 1) & 1;
+        r.prune = msf::row_prunable(f.ny, f.ka, f.kb);
+        cc.plan = pv & 1;
+        cc.prune = msf::col_prunable(f.nx, sp->keep.ab.data());
+        return msf::loop_supported(f.nx, f.ny, r, cc);
     };
     t.fused = [&f](int tile, int pv) { return fused_shape(f, tile, pv); };
     return t;
@@ -654,10 +665,11 @@ int launch_shape(msf_ctx* c, Mem& m, RunPlan& pl, const msf_specimen* sp,
         B = std::min<int64_t>(pick[0], P);
         chains_cfg = pick[2];
         sh.plan_v = pick[3];
-        // a tile that is the automatic one stays automatic, so that a smaller
-        // last batch has its own
-        const msf::TuneSpace t = tune_space(f, B, {sh.plan_v});
-        const bool own = chains_cfg < 3 && t.tile(B, sh.plan_v, chains_cfg == 2) == pick[1];
+        // a tile that is the automatic one, or that no pass uses, stays
+        // automatic, so that a smaller last batch has its own
+        const msf::TuneSpace t = tune_space(sp, f, B, {sh.plan_v});
+        const bool own = t.loop(B, sh.plan_v) ||
+                         (chains_cfg < 3 && t.tile(B, sh.plan_v, chains_cfg == 2) == pick[1]);
         sh.col_tile = own ? 0 : pick[1];
     }
     // Two chains of batches in flight on two streams: the row passes (VALU
@@ -1068,7 +1080,7 @@ int tune_shape(msf_ctx* c, RunPlan& pl, const msf_specimen* sp, const std::vecto
     if (plans)
         for (int pv : {0, all_alt})
             if (std::find(pvs.begin(), pvs.end(), pv) == pvs.end()) pvs.push_back(pv);
-    const msf::TuneSpace space = tune_space(f, B, pvs);
+    const msf::TuneSpace space = tune_space(sp, f, B, pvs);
     const TunedShape rule = msf::tune_rule(space);
     const std::vector<TunedShape> cands = msf::tune_candidates(space);
     RunPlan tb; // trial buffers, released on return
