@@ -146,7 +146,8 @@ typedef struct msf_stats {
     double row_pass_bytes, col_pass_bytes; /* compulsory HBM bytes of one launch */
     int32_t graph;                     /* 0: stream launches; 1: graph captured; 2: graph replayed */
     int32_t chains;                    /* batch chains in flight (msf_config.chains) */
-    int32_t col_tile;                  /* columns per column-pass workgroup used */
+    int32_t col_tile;                  /* columns per column-pass workgroup used; 0: every batch
+                                          ran its slices in one launch, without column passes */
     int32_t autotuned;                 /* 0: fixed rules; 1: tuned in this call; 2: tuned earlier */
     int32_t row_fft_plan;              /* radix plan of the row passes (length ny) and */
     int32_t col_fft_plan;              /* of the column passes (nx): 1 primary, 2 alternate */

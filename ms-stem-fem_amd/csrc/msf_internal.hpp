@@ -130,6 +130,7 @@ struct RunPlan {
     hipGraphExec_t graph = nullptr;
     std::vector<uint64_t> graph_sig;
     uint64_t graph_fused = 0; // fused pass launches in the captured graph
+    uint64_t graph_loops = 0; // one-launch slice loops in it
     RunPlan() = default;
     RunPlan(const RunPlan&) = delete;
     RunPlan& operator=(const RunPlan&) = delete;
@@ -441,6 +442,7 @@ struct Prof {
     std::vector<int> kind;
     hipEvent_t ka0 = nullptr, ka1 = nullptr; // pair stamped by a slice pass's own dispatch
     uint64_t fused = 0;                      // fused pass launches enqueued
+    uint64_t loops = 0;                      // batches enqueued as one-launch slice loops
     ~Prof()
     {
         for (hipEvent_t e : ev) (void)hipEventDestroy(e);

@@ -929,6 +929,7 @@ int enqueue_job(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, const Run
             row_at(r, 0);
             col_at(cc, 0);
             HIPCHK(c, msf::launch_slice_loop(nx, ny, f.tmode, msf::LoopArgs{r, cc, S}, s));
+            prof.loops += 1;
             return MSF_OK;
         }
         for (int n = 0; n < S; ++n) {
@@ -1219,14 +1220,17 @@ int run_internal(msf_ctx* c, Mem& m, const msf_specimen* sp, const msf_optics* o
                 HIPCHK(c, ei);
                 pl.graph_sig = sig;
                 pl.graph_fused = prof.fused;
+                pl.graph_loops = prof.loops;
                 graph_state = 1;
             }
         }
         if (captured) {
             HIPCHK(c, hipGraphLaunch(pl.graph, c->stream));
             prof.fused = pl.graph_fused;
+            prof.loops = pl.graph_loops;
         } else {
             graph_state = 0;
+            prof.loops = 0; // the attempt's
             if (int r = enqueue_job(c, pl, sp, f, sh, v, out, prof)) return r;
         }
     } else {
@@ -1249,9 +1253,11 @@ int run_internal(msf_ctx* c, Mem& m, const msf_specimen* sp, const msf_optics* o
     st.graph = graph_state;
     st.chains = sh.chains;
     st.fused_launches = prof.fused;
-    st.col_tile = sh.col_tile ? sh.col_tile
-                              : msf::col_tile_auto(f.nx, sh.plan_v & 1, (int)sh.split.depth, f.ncp,
-                                                   sh.chains == 2);
+    if (prof.loops == (uint64_t)sh.split.n) st.col_tile = 0; // no column pass ran
+    else if (sh.col_tile) st.col_tile = sh.col_tile;
+    else
+        st.col_tile = msf::col_tile_auto(f.nx, sh.plan_v & 1, (int)sh.split.depth, f.ncp,
+                                         sh.chains == 2);
     st.autotuned = sh.tuned_state;
     st.row_fft_plan = 1 + ((sh.plan_v >> 1) & 1);
     st.col_fft_plan = 1 + (sh.plan_v & 1);
