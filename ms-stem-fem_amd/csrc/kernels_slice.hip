@@ -175,19 +175,24 @@ static int col_places16(int nx, int v)
 // Launches of so few positions that the default tiles would leave CUs idle
 // (one position at 512^2: 44 workgroups of 8 columns for 256 CUs) take one
 // column per workgroup instead.
-// Launches of less than two rounds of 16-column tiles take tiles of 8, whose
-// last round leaves fewer CUs idle: column pass of 99 positions of 256^2
+// Launches of less than two rounds of 16-column tiles, with the GPU to
+// themselves, take tiles of 8, whose last round leaves fewer CUs idle: column pass of 99 positions of 256^2
 // (1,089 tiles of 16 for 1,024 places) 16.8 -> 16.0 us, of 192 26.8 -> 26.3,
 // of 91 positions of 192 x 96 10.2 -> 9.5; 256 positions (2.75 rounds) 32.5
-// against 33.0 with tiles of 8.  Row workgroups halved by the same rule: 3 %
-// faster at 192 x 96, 1 to 2 % slower at 256^2, not kept.
+// against 33.0 with tiles of 8.  Beside a second chain its passes fill those
+// CUs, and tiles of 16 stay: two batches on two chains, 12 slices, tiles of 8
+// against 16: 256^2 96 positions a batch (1.03 rounds) 775 -> 732 us, 144 983 ->
+// 947, 176 1155 -> 1120; 256 x 512 48 809 -> 770, 88 1270 -> 1211; 192^2 176 814 ->
+// 750, 272 1063 -> 1056, 296 (1.85 rounds) 1153 -> 1171; 256 x 384 and 256 x 128
+// within 2 % either way.  Row workgroups halved by the same rule: 3 % faster at
+// 192 x 96, 1 to 2 % slower at 256^2, not kept.
 int col_tile_auto(int nx, int v, int batch, int ncp, bool beside)
 {
     const int w = col_tile_default(nx, v, beside);
     constexpr int64_t kCUs = 256;
     const int64_t tiles = (int64_t)batch * (ncp / std::max(w, 1));
     if (tiles < kCUs) return 1;
-    return w == 16 && tiles < 2 * kCUs * col_places16(nx, v) ? 8 : w;
+    return w == 16 && !beside && tiles < 2 * kCUs * col_places16(nx, v) ? 8 : w;
 }
 
 // The difference of two of a 3-point step's inputs carries a third of the
