@@ -4,6 +4,7 @@
 #include "msf_internal.hpp"
 
 #include <algorithm>
+#include <set>
 
 using namespace msf_impl;
 
@@ -14,17 +15,13 @@ double ms_since(double t0) { return now_ms() - t0; }
 // Device bytes of a resident specimen's stacks and tables.
 uint64_t specimen_bytes(const msf_specimen* sp)
 {
-    uint64_t b = 0;
-    for (const DevBuf* d : {&sp->t32, &sp->t64, &sp->px, &sp->py, &sp->px64, &sp->py64, &sp->dkeep,
-                            &sp->dcolkeep})
-        b += d->bytes;
-    return b;
+    return sp->t32.bytes + sp->t64.bytes + sp->tables.bytes;
 }
 
 // Device bytes a job claims while it runs, over-estimated by 10 %: vacuum
-// waves, batch buffers of both chains and set-up temporaries, and for a job
-// that builds its own specimen that specimen's stacks and the species maps
-// of its build.  A job on a resident specimen claims no stacks: they are
+// waves and the work array of their set-up, batch buffers of both chains and
+// other set-up temporaries, and for a job that builds its own specimen that
+// specimen's stacks and the work arrays of its build.  A job on a resident specimen claims no stacks: they are
 // counted once, as resident bytes, while jobs refer to them.
 uint64_t job_footprint(const ServeJob& j)
 {
@@ -41,11 +38,18 @@ uint64_t job_footprint(const ServeJob& j)
     uint64_t wave = j.cfg.batch ? (uint64_t)j.cfg.batch * M * 8 : (112ull << 20);
     wave = std::min<uint64_t>(wave, P * M * 8 + (16ull << 20));
     uint64_t b = 16 * M * S                     // u0 stack (rows doubled, FP32)
-                 + 64 * M                       // probe, vacuum wave, per-pixel sums
+                 + std::min(16 * M * S, std::max<uint64_t>(32ull << 20, 16 * M)) // its work array
+                 + 64 * M                       // vacuum exit wave, per-pixel sums
                  + 2 * wave;                    // two chains of wave buffers
-    if (!j.spec)
+    if (!j.spec) {
+        // per slice and species a spectrum and a count map, per slice the
+        // band-limited plane, 96 MiB of slices or one; a template per species
+        const uint64_t nsp = std::set<uint32_t>(j.Z.begin(), j.Z.end()).size();
+        const uint64_t one = 20 * M * nsp + 16 * M;
+        const uint64_t build = std::min(S * one, std::max<uint64_t>(96ull << 20, one)) + 8 * M * nsp;
         b += 24 * M * S                         // t (FP32 + FP64) stacks
-             + (256ull << 20);                  // species maps of the set-up
+             + std::max<uint64_t>(256ull << 20, build); // the build's, later the group sums
+    }
     if (j.mtf.size() && j.fem.mtf_sampling_rate != 0.0)
         b += 2 * std::min<uint64_t>(P, (wave / 8 / std::max<uint64_t>(M, 1)) + 16) * M * 16;
     return b + b / 10 + (16ull << 20);
