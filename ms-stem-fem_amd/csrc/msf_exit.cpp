@@ -10,6 +10,7 @@
 #include "msf_internal.hpp"
 
 #include <algorithm>
+#include <cstdlib>
 #include <cstring>
 #include <system_error>
 
@@ -35,6 +36,7 @@ PinnedPool& pool()
 struct PinnedBlock {
     int kind;
     char* p = nullptr;
+    bool pinned = true;
     explicit PinnedBlock(int k) : kind(k) {}
     PinnedBlock(const PinnedBlock&) = delete;
     PinnedBlock& operator=(const PinnedBlock&) = delete;
@@ -50,13 +52,21 @@ struct PinnedBlock {
             }
         }
         void* q = nullptr;
-        const hipError_t e = hipHostMalloc(&q, kPinnedBytes[kind], hipHostMallocPortable);
-        if (e == hipSuccess) p = static_cast<char*>(q);
-        return e;
+        pinned = hipHostMalloc(&q, kPinnedBytes[kind], hipHostMallocPortable) == hipSuccess;
+        if (!pinned) { // the copy still works from ordinary memory
+            (void)hipGetLastError();
+            q = std::malloc(kPinnedBytes[kind]);
+        }
+        p = static_cast<char*>(q);
+        return p ? hipSuccess : hipErrorOutOfMemory;
     }
     ~PinnedBlock()
     {
         if (!p) return;
+        if (!pinned) {
+            std::free(p);
+            return;
+        }
         {
             std::lock_guard<std::mutex> lk(pool().m);
             std::vector<void*>& v = pool().idle[kind];
