@@ -180,10 +180,19 @@ __global__ void __launch_bounds__((LoopShape<NX, NY, VX, VY>::NT)) slice_loop_ke
     }
 }
 
-// Grids compiled in: sides of 64 to 256 whose plane fits.
+// Grids compiled in: sides of 64 to 256 whose plane fits, with the lines
+// between the loop and the passes (loop_faster): MIN, MIN2, A, B, A2, B2.
 #define MSF_LOOP_GRIDS(G)                                                                          \
-    G(64, 64) G(64, 96) G(96, 64) G(64, 128) G(128, 64) G(96, 96) G(64, 192) G(192, 64)            \
-    G(96, 128) G(128, 96) G(64, 256) G(256, 64) G(128, 128)
+    G(64, 64, 1, 257, 3.98f, 1.19f, 3.98f, 1.19f) G(64, 96, 4, 257, 2.80f, 0.87f, 0.0f, 1.10f)     \
+    G(96, 64, 4, 257, 2.75f, 0.66f, 0.0f, 0.0f) G(64, 128, 4, 257, 1.70f, 1.07f, -0.09f, 1.20f)    \
+    G(128, 64, 4, 257, 1.32f, 1.06f, 0.02f, 1.11f) G(96, 96, 16, 257, 1.22f, 0.79f, 0.05f, 0.91f)  \
+    G(64, 192, 64, 257, 0.90f, 0.82f, -0.17f, 0.92f)                                               \
+    G(192, 64, 64, 257, 1.15f, 0.94f, -0.25f, 1.12f)                                               \
+    G(96, 128, 64, 257, 0.77f, 0.93f, -0.34f, 0.99f)                                               \
+    G(128, 96, 64, 257, 0.83f, 0.77f, -0.76f, 0.83f)                                               \
+    G(64, 256, 128, 257, 1.09f, 0.95f, 0.14f, 1.10f)                                               \
+    G(256, 64, 128, 257, 1.10f, 1.02f, 0.14f, 1.21f)                                               \
+    G(128, 128, 128, 352, 0.70f, 0.95f, 0.10f, 1.08f)
 
 // the automatic radix plan of a side (256: the alternate)
 template <int N> static constexpr int loop_plan() { return N == 256 ? 1 : 0; }
@@ -196,22 +205,40 @@ static bool loop_ok(const RowPassArgs& r, const ColPassArgs& c)
 }
 
 // The loop runs a position on one CU, the passes spread it over all: up to
-// 64^2 the loop is always the faster, then from as many positions as fill
-// the chip well enough.  Loop against passes for 10 slices, with the sums:
-// 64^2 58 / 91 us at 1 position, 64 / 153 at 256; 96^2 131 / 125 at 4, 133 /
-// 158 at 16; 96x128 152 / 157 at 64; 128^2 179 / 163 at 64, 183 / 249 at 128,
-// 186 / 291 at 256, 614 / 741 at 1024.
-static int loop_min_batch(int nx, int ny)
+// 64^2 the loop is always the faster, then from as many positions as fill the
+// chip well enough (MIN).  256 positions are a round of the CUs, and a round
+// takes the same time however few of them it has, while the passes grow with
+// the positions: a second round pays from MIN2 positions on, and of more than
+// two rounds the loop is the faster while rounds <= A + B positions / 256 (the
+// passes' fixed and per-position time over a round's, fitted to 30 batches of
+// 513 to 2600 positions per grid; wrong by 4 % of the time at most).  On two
+// chains one batch's last round and the next one's first run together, and
+// the passes fill each other's gaps: there rounds and positions are those of
+// all batches together, with A2 and B2 (512 to 7000 positions).  Passes / loop
+// in us, sums included, 24 slices: 128^2 257 positions 650 / 772, 384 799 / 767,
+// 513 988 / 1117, 640 1162 / 1111, 769 1342 / 1466; 128 x 96 640 994 / 1074, 768
+// 1114 / 1077; 64 x 192 513 828 / 954, 704 1004 / 946; 96 x 128 513 882 / 978, 640
+// 1019 / 990; 96^2 257 709 / 581, 769 995 / 1087; 256 x 64 513 1048 / 991.  Two
+// chains, 12 slices: 128^2 1300 positions 1082 / 1149, 2300 1873 / 1689; 128 x 96
+// 2300 1325 / 1611; 96 x 64 4200 1352 / 1538; 64 x 128 1657 / 1421.
+struct LoopLine {
+    int min, min2;
+    float a, b, a2, b2;
+};
+static bool loop_faster(const LoopLine& l, int batch, int64_t together)
 {
-    const int n = nx * ny;
-    return n <= 64 * 64 ? 1 : n <= 128 * 64 ? 4 : (n - 128 * 64) / 64;
+    if (batch < l.min) return false;
+    const int64_t n = together ? together : batch, rounds = (n + 255) / 256;
+    if (together) return (float)rounds <= l.a2 + l.b2 * (float)n / 256.f;
+    if (rounds <= 2) return rounds < 2 || batch >= l.min2;
+    return (float)rounds <= l.a + l.b * (float)n / 256.f;
 }
 
-bool loop_supported(int nx, int ny, const RowPassArgs& r, const ColPassArgs& c)
+bool loop_supported(int nx, int ny, const RowPassArgs& r, const ColPassArgs& c, int64_t together)
 {
-    if (r.batch < loop_min_batch(nx, ny)) return false;
-#define MSF_GRID(NX, NY)                                                                           \
-    if (nx == NX && ny == NY) return loop_ok<NX, NY>(r, c);
+#define MSF_GRID(NX, NY, ...)                                                                      \
+    if (nx == NX && ny == NY)                                                                      \
+        return loop_ok<NX, NY>(r, c) && loop_faster(LoopLine{__VA_ARGS__}, r.batch, together);
     MSF_LOOP_GRIDS(MSF_GRID)
 #undef MSF_GRID
     return false;
@@ -221,7 +248,7 @@ hipError_t launch_slice_loop(int nx, int ny, int tmode, const LoopArgs& a, hipSt
 {
     if (a.row.batch <= 0 || a.slices <= 0) return hipErrorInvalidValue;
     const dim3 grid((unsigned)a.row.batch);
-#define MSF_GRID(NX, NY)                                                                           \
+#define MSF_GRID(NX, NY, ...)                                                                      \
     if (nx == NX && ny == NY) {                                                                    \
         if (!loop_ok<NX, NY>(a.row, a.col)) return hipErrorNotSupported;                           \
         constexpr int VX = loop_plan<NX>(), VY = loop_plan<NY>();                                  \

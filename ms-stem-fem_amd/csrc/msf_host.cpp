@@ -507,7 +507,8 @@ std::vector<TunedShape> tune_candidates(const TuneSpace& t)
             for (int ch : {1, 2, 3}) {
                 if (ch > 1 && b >= t.P) continue; // one batch
                 std::vector<int> tiles = {4, 8, 16};
-                if (t.loop && t.loop(b, pv)) tiles = {t.tile(b, pv, ch == 2)};
+                const auto& loop = ch == 2 && t.loop_beside ? t.loop_beside : t.loop;
+                if (loop && loop(b, pv)) tiles = {t.tile(b, pv, ch == 2)};
                 for (int w : tiles)
                     if (ch < 3 || t.fused(w, pv)) c.push_back({(int)b, w, ch, pv});
             }

@@ -203,7 +203,9 @@ struct TuneSpace {
     int64_t plane = 0;          // stored values of a wave
     std::vector<int> plans;     // the rule's first
     std::function<int(int64_t b, int plans, bool beside)> tile; // the automatic tile of a batch
-    std::function<bool(int64_t b, int plans)> loop;  // a batch takes the one-launch slice loop (null: none does)
+    // a batch takes the one-launch slice loop (null: none does), alone or
+    // beside a second chain (null: as alone)
+    std::function<bool(int64_t b, int plans)> loop, loop_beside;
     std::function<bool(int tile, int plans)> fused;  // chains 3 fuse their passes
 };
 // the shape a run of the rules takes

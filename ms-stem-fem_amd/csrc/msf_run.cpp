@@ -587,7 +587,7 @@ static msf::TuneSpace tune_space(const msf_specimen* sp, const RunFlags& f, int6
     t.tile = [&f](int64_t b, int pv, bool beside) {
         return msf::col_tile_auto(f.nx, pv & 1, (int)b, f.ncp, beside);
     };
-    t.loop = [&f, sp](int64_t b, int pv) {
+    const auto loop = [&f, sp](int64_t b, int pv, bool beside) {
         msf::RowPassArgs r{};
         msf::ColPassArgs cc{};
         r.batch = (int)b;
@@ -595,8 +595,10 @@ static msf::TuneSpace tune_space(const msf_specimen* sp, const RunFlags& f, int6
         r.prune = msf::row_prunable(f.ny, f.ka, f.kb);
         cc.plan = pv & 1;
         cc.prune = msf::col_prunable(f.nx, sp->keep.ab.data());
-        return msf::loop_supported(f.nx, f.ny, r, cc);
+        return msf::loop_supported(f.nx, f.ny, r, cc, beside ? f.P : 0);
     };
+    t.loop = [loop](int64_t b, int pv) { return loop(b, pv, false); };
+    t.loop_beside = [loop](int64_t b, int pv) { return loop(b, pv, true); };
     t.fused = [&f](int tile, int pv) { return fused_shape(f, tile, pv); };
     return t;
 }
@@ -668,7 +670,7 @@ int launch_shape(msf_ctx* c, Mem& m, RunPlan& pl, const msf_specimen* sp,
         // a tile that is the automatic one, or that no pass uses, stays
         // automatic, so that a smaller last batch has its own
         const msf::TuneSpace t = tune_space(sp, f, B, {sh.plan_v});
-        const bool own = t.loop(B, sh.plan_v) ||
+        const bool own = (chains_cfg == 2 ? t.loop_beside : t.loop)(B, sh.plan_v) ||
                          (chains_cfg < 3 && t.tile(B, sh.plan_v, chains_cfg == 2) == pick[1]);
         sh.col_tile = own ? 0 : pick[1];
     }
@@ -925,7 +927,7 @@ int enqueue_job(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, const Run
     };
     // the slice loop of one batch alone
     auto slices_alone = [&](msf::RowPassArgs& r, msf::ColPassArgs& cc, hipStream_t s) -> int {
-        if (!prof.on && msf::loop_supported(nx, ny, r, cc)) { // one launch, waves in LDS
+        if (!prof.on && msf::loop_supported(nx, ny, r, cc, chains == 2 ? P : 0)) { // one launch, waves in LDS
             row_at(r, 0);
             col_at(cc, 0);
             HIPCHK(c, msf::launch_slice_loop(nx, ny, f.tmode, msf::LoopArgs{r, cc, S}, s));
