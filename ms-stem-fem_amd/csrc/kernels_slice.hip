@@ -160,12 +160,16 @@ int col_tile(int nx)
     }
 }
 
-// 16-column tiles of a length that a CU holds at once
+// 16-column tiles of a length that a CU holds at once; 0 for lengths of which
+// 8 columns do not fill a wavefront (16 and 32): their tiles of 8 leave half
+// or more of its lanes idle (12 slices, per column pass: 400 positions of 16 x 64
+// 4.4 us with tiles of 16, 5.6 with 8; 900 of 16 x 256 14.0 and 20.2; 900 of
+// 32 x 256 15.0 and 20.0; 900 of 64 x 32 10.3 and 9.3)
 static int col_places16(int nx, int v)
 {
     switch (nx) {
 #define MSF_CASE(N) case N: return v ? col_per_cu<N, AltPlan<N>::exists ? 1 : 0, 16>(true) : col_per_cu<N, 0, 16>(true);
-        MSF_CASE(16) MSF_CASE(32) MSF_CASE(64) MSF_CASE(96) MSF_CASE(128) MSF_CASE(192) MSF_CASE(256)
+        MSF_CASE(64) MSF_CASE(96) MSF_CASE(128) MSF_CASE(192) MSF_CASE(256)
 #undef MSF_CASE
     default:
         return 0;
