@@ -90,7 +90,8 @@ struct LoopArgs {
 // true when the grid has such a launch for these arguments and it is the
 // faster way for their batch; together: the positions of all batches where
 // two chains of them run, else 0
-bool loop_supported(int nx, int ny, const RowPassArgs& r, const ColPassArgs& c, int64_t together);
+bool loop_supported(int nx, int ny, const RowPassArgs& r, const ColPassArgs& c, int slices,
+                    int64_t together);
 hipError_t launch_slice_loop(int nx, int ny, int tmode, const LoopArgs& a, hipStream_t s);
 
 // Grouped launches: one launch runs the same pass over the batches of up to

@@ -181,18 +181,21 @@ __global__ void __launch_bounds__((LoopShape<NX, NY, VX, VY>::NT)) slice_loop_ke
 }
 
 // Grids compiled in: sides of 64 to 256 whose plane fits, with the lines
-// between the loop and the passes (loop_faster): MIN, MIN2, A, B, A2, B2.
+// between the loop and the passes (loop_faster): MIN, MINS, MIN2, A, B, A2, B2.
 #define MSF_LOOP_GRIDS(G)                                                                          \
-    G(64, 64, 1, 257, 3.98f, 1.19f, 3.98f, 1.19f) G(64, 96, 4, 257, 2.80f, 0.87f, 0.0f, 1.10f)     \
-    G(96, 64, 4, 257, 2.75f, 0.66f, 0.0f, 0.0f) G(64, 128, 4, 257, 1.70f, 1.07f, -0.09f, 1.20f)    \
-    G(128, 64, 4, 257, 1.32f, 1.06f, 0.02f, 1.11f) G(96, 96, 16, 257, 1.22f, 0.79f, 0.05f, 0.91f)  \
-    G(64, 192, 64, 257, 0.90f, 0.82f, -0.17f, 0.92f)                                               \
-    G(192, 64, 64, 257, 1.15f, 0.94f, -0.25f, 1.12f)                                               \
-    G(96, 128, 64, 257, 0.77f, 0.93f, -0.34f, 0.99f)                                               \
-    G(128, 96, 64, 257, 0.83f, 0.77f, -0.76f, 0.83f)                                               \
-    G(64, 256, 128, 257, 1.09f, 0.95f, 0.14f, 1.10f)                                               \
-    G(256, 64, 128, 257, 1.10f, 1.02f, 0.14f, 1.21f)                                               \
-    G(128, 128, 128, 352, 0.70f, 0.95f, 0.10f, 1.08f)
+    G(64, 64, 1, 1, 257, 3.98f, 1.19f, 3.98f, 1.19f)                                               \
+    G(64, 96, 4, 4, 257, 2.80f, 0.87f, 0.0f, 1.10f)                                                \
+    G(96, 64, 4, 4, 257, 2.75f, 0.66f, 0.0f, 0.0f)                                                 \
+    G(64, 128, 4, 4, 257, 1.70f, 1.07f, -0.09f, 1.20f)                                             \
+    G(128, 64, 4, 4, 257, 1.32f, 1.06f, 0.02f, 1.11f)                                              \
+    G(96, 96, 16, 16, 257, 1.22f, 0.79f, 0.05f, 0.91f)                                             \
+    G(64, 192, 64, 100, 257, 0.90f, 0.82f, -0.17f, 0.92f)                                          \
+    G(192, 64, 64, 64, 257, 1.15f, 0.94f, -0.25f, 1.12f)                                           \
+    G(96, 128, 64, 100, 257, 0.77f, 0.93f, -0.34f, 0.99f)                                          \
+    G(128, 96, 80, 100, 257, 0.83f, 0.77f, -0.76f, 0.83f)                                          \
+    G(64, 256, 128, 128, 257, 1.09f, 0.95f, 0.14f, 1.10f)                                          \
+    G(256, 64, 128, 128, 257, 1.10f, 1.02f, 0.14f, 1.21f)                                          \
+    G(128, 128, 128, 128, 352, 0.70f, 0.95f, 0.10f, 1.08f)
 
 // the automatic radix plan of a side (256: the alternate)
 template <int N> static constexpr int loop_plan() { return N == 256 ? 1 : 0; }
@@ -206,7 +209,8 @@ static bool loop_ok(const RowPassArgs& r, const ColPassArgs& c)
 
 // The loop runs a position on one CU, the passes spread it over all: up to
 // 64^2 the loop is always the faster, then from as many positions as fill the
-// chip well enough (MIN).  256 positions are a round of the CUs, and a round
+// chip well enough (MIN; MINS of fewer than 4 slices, which leave the loop's
+// start and end a larger part).  256 positions are a round of the CUs, and a round
 // takes the same time however few of them it has, while the passes grow with
 // the positions: a second round pays from MIN2 positions on, and of more than
 // two rounds the loop is the faster while rounds <= A + B positions / 256 (the
@@ -220,25 +224,28 @@ static bool loop_ok(const RowPassArgs& r, const ColPassArgs& c)
 // 1114 / 1077; 64 x 192 513 828 / 954, 704 1004 / 946; 96 x 128 513 882 / 978, 640
 // 1019 / 990; 96^2 257 709 / 581, 769 995 / 1087; 256 x 64 513 1048 / 991.  Two
 // chains, 12 slices: 128^2 1300 positions 1082 / 1149, 2300 1873 / 1689; 128 x 96
-// 2300 1325 / 1611; 96 x 64 4200 1352 / 1538; 64 x 128 1657 / 1421.
+// 2300 1325 / 1611; 96 x 64 4200 1352 / 1538; 64 x 128 1657 / 1421.  40 slices,
+// 64 and 80 positions: 64 x 192 568 / 555 and 639 / 553, 96 x 128 594 / 578 and
+// 653 / 579, 128 x 96 577 / 627 and 655 / 624; one slice of 64: 39 / 45 each.
 struct LoopLine {
-    int min, min2;
+    int min, min_short, min2;
     float a, b, a2, b2;
 };
-static bool loop_faster(const LoopLine& l, int batch, int64_t together)
+static bool loop_faster(const LoopLine& l, int batch, int slices, int64_t together)
 {
-    if (batch < l.min) return false;
+    if (batch < (slices < 4 ? l.min_short : l.min)) return false;
     const int64_t n = together ? together : batch, rounds = (n + 255) / 256;
     if (together) return (float)rounds <= l.a2 + l.b2 * (float)n / 256.f;
     if (rounds <= 2) return rounds < 2 || batch >= l.min2;
     return (float)rounds <= l.a + l.b * (float)n / 256.f;
 }
 
-bool loop_supported(int nx, int ny, const RowPassArgs& r, const ColPassArgs& c, int64_t together)
+bool loop_supported(int nx, int ny, const RowPassArgs& r, const ColPassArgs& c, int slices,
+                    int64_t together)
 {
 #define MSF_GRID(NX, NY, ...)                                                                      \
     if (nx == NX && ny == NY)                                                                      \
-        return loop_ok<NX, NY>(r, c) && loop_faster(LoopLine{__VA_ARGS__}, r.batch, together);
+        return loop_ok<NX, NY>(r, c) && loop_faster(LoopLine{__VA_ARGS__}, r.batch, slices, together);
     MSF_LOOP_GRIDS(MSF_GRID)
 #undef MSF_GRID
     return false;

@@ -595,7 +595,7 @@ static msf::TuneSpace tune_space(const msf_specimen* sp, const RunFlags& f, int6
         r.prune = msf::row_prunable(f.ny, f.ka, f.kb);
         cc.plan = pv & 1;
         cc.prune = msf::col_prunable(f.nx, sp->keep.ab.data());
-        return msf::loop_supported(f.nx, f.ny, r, cc, beside ? f.P : 0);
+        return msf::loop_supported(f.nx, f.ny, r, cc, f.S, beside ? f.P : 0);
     };
     t.loop = [loop](int64_t b, int pv) { return loop(b, pv, false); };
     t.loop_beside = [loop](int64_t b, int pv) { return loop(b, pv, true); };
@@ -927,7 +927,7 @@ int enqueue_job(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, const Run
     };
     // the slice loop of one batch alone
     auto slices_alone = [&](msf::RowPassArgs& r, msf::ColPassArgs& cc, hipStream_t s) -> int {
-        if (!prof.on && msf::loop_supported(nx, ny, r, cc, chains == 2 ? P : 0)) { // one launch, waves in LDS
+        if (!prof.on && msf::loop_supported(nx, ny, r, cc, S, chains == 2 ? P : 0)) { // one launch, waves in LDS
             row_at(r, 0);
             col_at(cc, 0);
             HIPCHK(c, msf::launch_slice_loop(nx, ny, f.tmode, msf::LoopArgs{r, cc, S}, s));
