@@ -16,7 +16,7 @@ namespace msf {
 
 // ------------------------------------------------------- fused pass pair
 // One launch runs a row pass of one batch and a column pass of another
-// (independent buffers), so that the VALU-bound row workgroups and the
+// (independent buffers), so that the row workgroups, which compute more, and the
 // memory-bound column workgroups share the CUs instead of following each
 // other.  Both passes need workgroups of the same size (RT = W * T).  Launch
 // blocks alternate in groups of eight, eight of each pass per sixteen, so

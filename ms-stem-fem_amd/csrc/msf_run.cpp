@@ -674,9 +674,9 @@ int launch_shape(msf_ctx* c, Mem& m, RunPlan& pl, const msf_specimen* sp,
                          (chains_cfg < 3 && t.tile(B, sh.plan_v, chains_cfg == 2) == pick[1]);
         sh.col_tile = own ? 0 : pick[1];
     }
-    // Two chains of batches in flight on two streams: the row passes (VALU
-    // bound) of one chain overlap the column passes (memory bound) of the
-    // other.  Automatic: two chains, launched on the streams, once a launch
+    // Two chains of batches in flight on two streams: the row passes (which
+    // compute and wait) of one chain overlap the column passes (memory bound)
+    // of the other.  Automatic: two chains, launched on the streams, once a launch
     // covers >= 4M pixels (512^2: +4 % over one chain, graph or not; the
     // runtime replays a two-branch graph's branches one after the other);
     // below that one chain replayed as a graph, where launch cost matters.
@@ -947,7 +947,7 @@ int enqueue_job(msf_ctx* c, const RunPlan& pl, const msf_specimen* sp, const Run
     if (chains == 3) {
         // Paired batches on one stream: the row pass of one batch and the
         // column pass of the other share a launch (fused_pass_kernel), so the
-        // VALU-bound row workgroups and the memory-bound column workgroups of
+        // row workgroups, which compute more, and the memory-bound column workgroups of
         // the two batches run side by side on every CU.  Per pair (A, B):
         // A.row0, then (A.col n + B.row n), (A.row n+1 + B.col n), ...,
         // B.col S-1; each batch still sees its passes in slice order, and the

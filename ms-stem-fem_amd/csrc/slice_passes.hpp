@@ -56,8 +56,8 @@ template <typename T> __device__ __forceinline__ const T& elem_at(const T* base,
 //   B = tau U_im + u_im + ti (A + u0_re) / s     (TMODE 0)
 // since the reference's in-place update forms Im from the updated Re, whose
 // value is (A + u0_re) / s; TMODE 1 (exact product) has B = tau U_im + u_im +
-// ti U_re.  Eight operations a value: the row pass is bound by them, and the
-// products with u and u0 taken apart were twelve.
+// ti U_re.  Eight operations a value; with the products of u and u0 taken apart
+// they were twelve (32 more instructions of 551 a wave at 512).
 template <bool FIRST, int TMODE>
 __device__ __forceinline__ float2 transmit_point(float2 u, float2 t, float2 u0, float is)
 {
@@ -167,8 +167,9 @@ template <int NY, int V> __host__ __device__ constexpr int row_len()
     return P::T >= 16 ? P::kExchangeLen : (P::kExchangeLen + 7) / 16 * 16 + 8;
 }
 //
-// The row pass keeps the vector unit busy for 70 to 80 % of its time and
-// waits for the rest between load, transforms and store, so what is uniform or
+// The row pass waits between load, transforms and store as much as it computes
+// (512^2: 551 vector instructions a wave keep the vector unit busy for 63 % of
+// the pass, the LDS for 40 %, without bank conflicts), so what is uniform or
 // known at compile time stays out of the vector unit: the workgroup's
 // division, the row and u0 addresses (a base per wavefront, the element in the
 // instruction), the table staging in 16-byte words, the wrap of the shifted
@@ -509,7 +510,8 @@ __device__ __forceinline__ void col_body(const ColPassArgs& a, int blk, int nblk
     P::template run<false, float2, WAVE, PS>(x, lds, tw, t);
 
     // band limit (bw_limit + propagate's k^2 test, decided on the host) and
-    // propagator P_x[i] * P_y[j]; P_y carries the 1/sqrtNxNy of the FFT and of the transmission
+    // propagator P_x[i] * P_y[j]; P_y carries the 1/(nx ny) of the transforms and
+    // of the transmission, over the FP32 transforms' gain (fp32_gain)
     const float2 pyj = active ? a.py[j] : float2{0.f, 0.f};
     // kept rows of this column, decided on the host (one pair per column
     // instead of a range table per row)
