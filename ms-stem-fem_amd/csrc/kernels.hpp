@@ -62,7 +62,7 @@ struct ColPassArgs {
     int tile;               // columns per workgroup (4, 8 or 16; 0 = default)
     int prune;              // 1: rows [3nx/8, 5nx/8) are masked for every column
     int plan;               // radix plan of length nx: 0 primary, 1 alternate (has_alt_plan)
-    int beside;             // 1: another chain of batches runs beside this one (col_tile_default)
+    int beside;             // 1: another chain of batches runs beside this one (col_tile_auto)
     uint32_t div;           // set by the launch: div_mul of the tiles per position
 };
 // multiplier for a kernel's division by d (1 <= d < 2^31)

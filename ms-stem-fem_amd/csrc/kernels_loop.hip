@@ -13,8 +13,8 @@
 // propagate_point), so results equal theirs bit for bit.
 //
 // Bound by the latency of one CU working through a position: 64^2 3.3 us a
-// slice (4 positions per CU fit the LDS, 2 the registers), 128^2 15.7 us for
-// up to 256 positions at once, against 14 and 29 us for a slice's two passes
+// slice (4 positions per CU fit the LDS, 2 the registers), 128^2 14.6 us for
+// up to 256 positions at once, against 13 and 23 us for a slice's two passes
 // over 256 positions.  Tried without gain: 512 instead of 1024 lanes at 128^2
 // (17 us), a 16 x 8 plan at 128 (spills, 18 us), the transmission and vacuum
 // pairs read ahead of the inverse transform (spills at 128^2, 17 us), 64^2
